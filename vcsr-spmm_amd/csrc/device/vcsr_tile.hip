@@ -645,8 +645,9 @@ __global__ __launch_bounds__(256) void vcsr_tile_reduce(int32_t O, int32_t ld, i
     int32_t cl = 1;
     while (cl < nvec && cl < 64) cl <<= 1;
     auto part = [&](const int4& s, int32_t j, int32_t cv) {
-        return *reinterpret_cast<const V*>(partials + (int64_t)s.y * O +
-                                           (int64_t)j * ((int64_t)s.z * O) + (int64_t)cv * VEC);
+        return load_mem(partials + (int64_t)s.y * O + (int64_t)j * ((int64_t)s.z * O) +
+                            vec_col<VEC>(cv * VEC, O),
+                        V());
     };
     // acc += partials g, g + groups, ... of column vector cv of row s.
     auto sum_group = [&](const int4& s, int32_t g, int32_t groups, int32_t cv, V acc) {
@@ -670,8 +671,7 @@ __global__ __launch_bounds__(256) void vcsr_tile_reduce(int32_t O, int32_t ld, i
         return acc;
     };
     auto store = [&](const int4& s, int32_t cv, const V& x) {
-        V* dst = reinterpret_cast<V*>(C + (int64_t)s.x * ld + (int64_t)cv * VEC);
-        *dst = accumulate ? add_vec(*dst, x) : x;
+        store_cols<VEC, false>(C + (int64_t)s.x * ld, cv * VEC, O, x, accumulate);
     };
     if ((int32_t)blockIdx.x < n_heavy) {
         const int4 s = split[blockIdx.x];
@@ -716,6 +716,13 @@ __global__ __launch_bounds__(256) void vcsr_tile_reduce(int32_t O, int32_t ld, i
 // component c, so D_c[i][j] is C[row i][c0 + VEC*j + c].  A group of 16
 // entries is four k-steps; the view stores its values in operand order, so
 // lane l reads the A operands of all four as one 16-byte load.
+//
+// Rows of B and C need not be aligned to VEC floats: a lane whose columns
+// would reach past O takes the last VEC of the row and stores its own ones
+// (vec_col, store_cols), so every O over 32 reads 16 bytes per lane.
+// Block-sparse 16K matrix, O = 65 / 127 / 333: 51.8 / 84.1 / 229 us with the
+// 4-byte lanes an odd O used to take, 39.8 / 41.8 / 101 now; O = 64, 100,
+// 512 unchanged.
 //
 // One wave per (piece, column tile of 16*VEC columns).  The grid runs
 // column-tile-major with the XCD-aware block order, so each XCD works on one
@@ -774,7 +781,7 @@ __global__ __launch_bounds__(256) void vcsr_tile_mma_kernel(
     const int kq = lane >> 4, jl = lane & 15;  // MFMA k index, column lane
     const int32_t col = ct * 16 * VEC + VEC * jl;
     const bool kok = col < O;
-    const uint32_t koff = (uint32_t)(kok ? col : 0) * 4u;
+    const uint32_t koff = (uint32_t)vec_col<VEC>(col, O) * 4u;
     // Entry t's B slice for this lane; zeros for "no row" and columns past O.
     auto load_b = [&](int32_t t) -> V {
         if constexpr (BUF) {
@@ -782,7 +789,7 @@ __global__ __launch_bounds__(256) void vcsr_tile_mma_kernel(
         } else {
             const uint32_t br = lb[t];
             if (br == kNoRow || !kok) return zero_vec(V());
-            return *reinterpret_cast<const V*>(B + (int64_t)br * ld + col);
+            return load_mem(B + (int64_t)br * ld + koff / 4, V());
         }
     };
     const float* vp = ent_val + (int64_t)e0 * kTileMmaRows + 4 * lane;
@@ -876,12 +883,10 @@ __global__ __launch_bounds__(256) void vcsr_tile_mma_kernel(
         V x;
 #pragma unroll
         for (int c = 0; c < VEC; ++c) reinterpret_cast<float*>(&x)[c] = d[c][v];
-        if (part < 0) {
-            V* dst = reinterpret_cast<V*>(C + (int64_t)(row0 + r) * ld + col);
-            store_nt(dst, accumulate ? add_vec(*dst, x) : x);
-        } else {
-            *reinterpret_cast<V*>(partials + (int64_t)(part + r) * O + col) = x;
-        }
+        if (part < 0)
+            store_cols<VEC, true>(C + (int64_t)(row0 + r) * ld, col, O, x, accumulate);
+        else
+            store_cols<VEC, false>(partials + (int64_t)(part + r) * O, col, O, x, false);
     }
 }
 
@@ -1025,12 +1030,25 @@ hipError_t launch_vec(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t
 
 }  // namespace
 
-// Floats per lane and B slice: 4 when O allows 8 lanes (16 for 16-row MFMA
-// tiles, whose column tiles are 16 lanes wide) of 16-byte vectors and B and
-// C are 16-byte aligned, else 2 or 1.  At O = 32, 4 floats per lane measured
-// 3% / 8% faster than 2 on the banded / power-law matrices.
-static int tile_vec(int32_t O, bool a16, bool a8, bool mma) {
-    if (O % 4 == 0 && a16 && O >= (mma ? 64 : 32)) return 4;
+// Floats per lane of a 16-row tile's column tile (16 lanes) for w columns of
+// any alignment: the narrowest whose one column tile covers w, else 4.  Idle
+// lanes are cheaper than a second column tile, which reads every B row and
+// all values again: block-sparse 16K matrix, O = 24 16.7 us as one tile of
+// 2 floats per lane against 24.6 as two of 1, O = 50 22.7 as one of 4
+// against 30.4 as two of 2.
+static int tile_mma_vec(const DeviceFmt& d, int32_t w) {
+    int vec = w > 32 ? 4 : w > 16 ? 2 : 1;
+    const int64_t n_ct = vec > 1 ? (w + 8 * vec - 1) / (8 * vec) : 0;
+    if (vec > 1 && (int64_t)d.tv_n_chunks * n_ct <= 4 * (int64_t)device_cus(d.device)) vec /= 2;
+    return vec;
+}
+
+// Floats per lane and B slice of the other tiles: 4 when O allows 8 lanes of
+// 16-byte vectors and B and C are 16-byte aligned, else 2 or 1.  At O = 32,
+// 4 floats per lane measured 3% / 8% faster than 2 on the banded /
+// power-law matrices.
+static int tile_vec(int32_t O, bool a16, bool a8) {
+    if (O % 4 == 0 && a16 && O >= 32) return 4;
     if (O % 2 == 0 && a8 && O >= 32) return 2;
     return 1;
 }
@@ -1054,8 +1072,10 @@ static TileSlicing tile_slicing(const Vcsr& v, const DeviceFmt& d, const float* 
     // Narrow B: narrower per-lane vectors give streams of at least 8-16
     // lanes, so fewer streams share a tile's entries (measured at O = 8:
     // 4-byte loads with 8 streams 1.3x faster than 16-byte loads with 32).
-    TileSlicing ts{tile_vec(O, a16, a8, d.tv_R == kTileMmaRows), O};
-    if (ts.vec == 4 && d.tv_R != kTileMmaRows) {
+    TileSlicing ts{tile_vec(O, a16, a8), O};
+    if (d.tv_R == kTileMmaRows) {
+        ts.vec = tile_mma_vec(d, d.tv_partial_rows > 0 ? std::min(O, kTileWideCols) : O);
+    } else if (ts.vec == 4) {
         if ((uint64_t)v.N * (uint64_t)O * 4u > kTileSliceBytes) ts.width = std::min(O, kTileSliceCols);
         else ts.width = std::min(O, kTileWideCols);
     }
@@ -1097,7 +1117,7 @@ hipError_t launch_vcsr_tile(const Vcsr& v, const DeviceFmt& d, const float* B, i
     for (int32_t c0 = 0; c0 < O; c0 += ts.width) {
         const int32_t w = std::min(ts.width, O - c0);
         hipError_t e;
-        switch (ts.vec) {
+        switch (d.tv_R == kTileMmaRows ? tile_mma_vec(d, w) : ts.vec) {
             case 4: e = launch_vec<4>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;
             case 2: e = launch_vec<2>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;
             default: e = launch_vec<1>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;
@@ -1111,9 +1131,11 @@ MfmaWork tile_mfma_work(const DeviceFmt& d, int32_t O) {
     MfmaWork w;
     w.flops_per_op = 2 * 16 * 16 * 4;
     if (d.tv_R != kTileMmaRows || O <= 0) return w;
-    const int vec = tile_vec(O, true, true, true);
-    const int64_t n_ct = (O + 16 * vec - 1) / (16 * vec);
-    w.ops = d.tv_n_entries / 4 * n_ct * vec;
+    const int32_t width = d.tv_partial_rows > 0 ? std::min(O, kTileWideCols) : O;
+    for (int32_t c0 = 0; c0 < O; c0 += width) {
+        const int32_t n = std::min(width, O - c0), vec = tile_mma_vec(d, n);
+        w.ops += d.tv_n_entries / 4 * ((n + 16 * vec - 1) / (16 * vec)) * vec;
+    }
     return w;
 }
 

@@ -64,6 +64,71 @@ __device__ __forceinline__ void store_nt(float4* p, float4 x) {
     __builtin_nontemporal_store(__builtin_bit_cast(nt_float4, x), reinterpret_cast<nt_float4*>(p));
 }
 
+// The same vectors in memory at any 4-byte boundary (rows of B and C whose
+// length is not a multiple of the vector): gfx950's wide loads and stores
+// need dword alignment only.
+typedef float mem_float2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float mem_float4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float load_mem(const float* p, float) { return *p; }
+__device__ __forceinline__ float2 load_mem(const float* p, float2) {
+    return __builtin_bit_cast(float2, *reinterpret_cast<const mem_float2*>(p));
+}
+__device__ __forceinline__ float4 load_mem(const float* p, float4) {
+    return __builtin_bit_cast(float4, *reinterpret_cast<const mem_float4*>(p));
+}
+template <bool NT>
+__device__ __forceinline__ void store_mem(float* p, float x) {
+    if constexpr (NT) __builtin_nontemporal_store(x, p);
+    else *p = x;
+}
+template <bool NT>
+__device__ __forceinline__ void store_mem(float* p, float2 x) {
+    const mem_float2 y = __builtin_bit_cast(mem_float2, x);
+    if constexpr (NT) __builtin_nontemporal_store(y, reinterpret_cast<mem_float2*>(p));
+    else *reinterpret_cast<mem_float2*>(p) = y;
+}
+template <bool NT>
+__device__ __forceinline__ void store_mem(float* p, float4 x) {
+    const mem_float4 y = __builtin_bit_cast(mem_float4, x);
+    if constexpr (NT) __builtin_nontemporal_store(y, reinterpret_cast<mem_float4*>(p));
+    else *reinterpret_cast<mem_float4*>(p) = y;
+}
+
+// Columns of a row of `width` (>= VEC) floats held by a lane whose first
+// column is k, a multiple of VEC.  A vector that would reach past the row's
+// end is moved back to end with it (vec_col), so that every access stays
+// inside the row; it then holds some of the previous lane's columns again,
+// and store_cols writes only the lane's own.
+template <int VEC>
+__device__ __forceinline__ int32_t vec_col(int32_t k, int32_t width) {
+    return VEC == 1 ? min(k, width - 1) : min(k, width - VEC);
+}
+// row[k ..] = x (or += x), row being the row's first column.  The test for
+// rows of whole vectors is the same for every lane (a scalar branch).
+template <int VEC, bool NT>
+__device__ __forceinline__ void store_cols(float* row, int32_t k, int32_t width,
+                                           typename VecT<VEC>::T x, bool accumulate) {
+    using V = typename VecT<VEC>::T;
+    if (width % VEC == 0) {
+        if (accumulate) x = add_vec(load_mem(row + k, V()), x);
+        store_mem<NT>(row + k, x);
+        return;
+    }
+    if (k + VEC <= width) {
+        if (accumulate) x = add_vec(load_mem(row + k, V()), x);
+        store_mem<NT>(row + k, x);
+        return;
+    }
+#pragma unroll
+    for (int c = 1; c < VEC; ++c) {
+        const int32_t col = width - VEC + c;
+        if (col < k) continue;
+        float y = reinterpret_cast<const float*>(&x)[c];
+        if (accumulate) y += row[col];
+        store_mem<NT>(row + col, y);
+    }
+}
+
 // gfx9 raw buffer resource flags: 32-bit data, no swizzle.  Loads past the
 // record count return zeros instead of faulting.
 constexpr int32_t kRawBufferFlags = 0x00020000;
