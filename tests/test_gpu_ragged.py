@@ -4,7 +4,7 @@ boundary, the last vector of a row moved back to end with it."""
 import numpy as np
 import pytest
 
-from test_gpu_parity import _block_csr, _Shifted
+from test_gpu_parity import _block_csr, _Shifted, assert_within_tolerance
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +41,69 @@ def test_mfma_tiles_any_width_are_bit_exact(gpu, orc, st, O, off):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
     got = _spmm(vs, fmt, B, C0, off, st, True)
     assert np.array_equal(got, C0 + ref)
+
+
+def _mixed_blocks(vs, rng, h):
+    """Block rows of h equal-pattern rows: short and long ones, one cut into
+    several pieces (600 columns), empty rows, a last block row cut short."""
+    N = 1500
+    rows, cols, r = [], [], 0
+    for n in [1, 5, 33, 64, 65, 97, 129, 600, 0, 7, 40, 63, 2, 90, 20, 20, 11]:
+        c = np.sort(rng.choice(N, size=n, replace=False))
+        for i in range(h):
+            keep = c if i == 0 else c[rng.random(n) < 0.9]
+            rows.append(np.full(keep.size, r + i))
+            cols.append(keep)
+        r += h
+    rows, cols = np.concatenate(rows).astype(np.int32), np.concatenate(cols).astype(np.int32)
+    vals = rng.standard_normal(rows.size).astype(np.float32)
+    live = rows < r - 1 if h > 1 else rows < r
+    return vs.coo_to_csr(vs.Coo.from_arrays(r - (h > 1), N, rows[live], cols[live], vals[live]))
+
+
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("O", [1, 3, 4, 7, 8, 9, 15, 16, 17, 31, 32, 33, 50, 64, 65, 127, 129, 255,
+                               257])
+@pytest.mark.parametrize("R", [2, 3, 4, 8])
+def test_tall_tiles_any_width(gpu, orc, st, R, O, off):
+    """Tiles of 2 to 8 rows at every width class and its edges, split tiles
+    and their reduce among them: C = A*B and C += A*B against the oracle."""
+    vs = gpu
+    rng = np.random.default_rng(1000 * R + O)
+    csr = _mixed_blocks(vs, rng, R)
+    fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
+    fmt.set_tile_rows(R)
+    fmt.upload(st)
+    assert fmt.launch_info(O)["split_rows"] >= R - 1
+    B = vs.gen_dense(O, 0, csr.N, O)
+    C0 = rng.integers(-2, 3, size=(csr.M, O)).astype(np.float32)
+    ref = orc.spmm_f64(csr.M, csr.row_ptr, csr.col, csr.val, B)
+    assert_within_tolerance(_spmm(vs, fmt, B, C0, off, st, False), ref, csr.row_ptr, csr.val, B,
+                            f"R{R} O{O}")
+    got = _spmm(vs, fmt, B, C0, off, st, True)
+    # One more rounding of values up to |C0| + |ref|.
+    err = np.abs(got - (C0 + ref)) - 2.0 ** -23 * (np.abs(C0) + np.abs(ref))
+    l1 = np.array([np.abs(csr.val[a:b]).sum() for a, b in zip(csr.row_ptr, csr.row_ptr[1:])])
+    assert (err <= 1e-4 * l1[:, None] * np.abs(B).max()).all()
+
+
+@pytest.mark.parametrize("O", [5, 12, 30, 47, 100])
+@pytest.mark.parametrize("R", [2, 3, 4, 8])
+def test_tall_tiles_nonfinite_b(gpu, orc, st, R, O):
+    """inf and NaN in B reach exactly the rows the oracle's loop reaches,
+    also in the last, moved-back vector of a row and its neighbours."""
+    vs = gpu
+    rng = np.random.default_rng(R + O)
+    csr = _mixed_blocks(vs, rng, R)
+    fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
+    fmt.set_tile_rows(R)
+    fmt.upload(st)
+    B = vs.gen_dense(O, 0, csr.N, O)
+    for r, c, x in [(3, O - 1, np.inf), (700, O - 2, np.nan), (701, 0, -np.inf), (1499, O - 1, np.nan)]:
+        B[r, c] = x
+    ref = orc.spmm_f32(csr.M, csr.row_ptr, csr.col, csr.val, B)
+    got = _spmm(vs, fmt, B, np.zeros((csr.M, O), np.float32), 0, st, False)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isinf(got), np.isinf(ref))
+    fin = np.isfinite(ref)
+    assert np.allclose(got[fin], ref[fin], rtol=1e-4, atol=1e-4)

@@ -58,6 +58,11 @@ hipError_t launch_vcsr_tile(const Vcsr& v, const DeviceFmt& d, const float* B, i
                             float* C, int32_t accumulate, float* partials, hipStream_t st);
 int64_t tile_partials_floats(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t O,
                              const float* C);
+// The launch over its tiles of 2, 3, 4 or 8 rows (vcsr_tile_tall.hip) for
+// columns [0, O) of B and C, at most 256, whose rows are ld floats apart;
+// b_bytes from B to the end of its last row.
+hipError_t launch_vcsr_tall(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
+                            int32_t accumulate, uint64_t b_bytes, float* partials, hipStream_t st);
 // Partial-row floats that cover tile_partials_floats for every O, B and C:
 // a view with split tiles is launched in column slices of at most 256
 // columns, and its partial rows are one slice wide.

@@ -225,6 +225,8 @@ int vcsr_fmt_upload(vcsr_fmt* fmt, void* stream) {
                 std::memcpy(&tv_val[q * ds + ds - 1], &tv_brow[q], sizeof(float));
             }
         }
+        std::vector<int32_t> tv_pieces(tv.pieces);
+        tv_pieces.insert(tv_pieces.end(), {0, 0, (int32_t)tv.n_entries(), -1});
         DeviceFmt d;
         hip_check(hipGetDevice(&d.device), "hipGetDevice");
         try {
@@ -249,7 +251,8 @@ int vcsr_fmt_upload(vcsr_fmt* fmt, void* stream) {
             d.tv_R = tv.R;
             d.tv_chunks = upload_array(tv.chunks, st, "upload tile chunks");
             d.tv_n_chunks = (int32_t)(tv.chunks.size() / 4);
-            d.tv_pieces = upload_array(tv.pieces, st, "upload tile pieces");
+            d.tv_pieces = upload_array(tv_pieces, st, "upload tile pieces");
+            d.tv_n_pieces = (int32_t)(tv.pieces.size() / 4);
             // 1- and 3-row tiles carry the B rows in their value records.
             if (!vcsr::tile_dev_folds_brow(tv.R))
                 d.tv_brow = upload_array(tv_brow, st, "upload tile entries");

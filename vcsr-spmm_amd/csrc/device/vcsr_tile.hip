@@ -11,41 +11,36 @@
 // the B-row traffic through the vector memory pipe, the limiting resource of
 // a row-stationary SpMM, by the block height.
 //
-// Work item (one wave): MERGE consecutive work items of the view, each a run
-// of tile pieces with at most tile_piece_entries(R) entries
+// This file holds the single-row kernel, the matrix-core kernel of 16-row
+// tiles, the reduce of split tiles and the launcher; tiles of 2 to 8 rows are
+// in vcsr_tile_tall.hip.
+//
+// Single-row work item (one wave): MERGE consecutive work items of the view,
+// each a run of tile pieces with at most tile_piece_entries(1) entries
 // (host/tile_view.hpp).
-// Phase 1 (lane per entry): read the entry's B row and R values (the view
-// stores the values of its slots next to each other, for 1- and 3-row tiles
-// in one record with the B row, so these are coalesced loads, not gathers
-// from the VCSR value array) and stage (B-row byte offset, values) in the
-// wave's LDS list.
+// Phase 1 (lane per entry): read the entry's record (value and B row, stored
+// together, so these are coalesced loads, not gathers from the VCSR value
+// array) and stage (B-row byte offset, value) in the wave's LDS list.
 // Phase 2, per column tile of LPE*VEC columns: the wave is S = 64/LPE
 // streams of LPE lanes; one load instruction serves one entry of every
 // stream.
 //  - Several pieces: each stream takes a contiguous run of whole pieces
-//    (balanced by entry count), accumulates the piece's R rows and stores
-//    them when its last entry has been applied.  No cross-lane reduction.
-//    Single-row tiles with several work items per wave instead give every
-//    stream an equal run of entries; a piece cut between runs is finished
-//    by the stream that began it, from the later streams' partial sums in
-//    LDS.
-//  - One piece (a long tile): the streams interleave over its entries, whose
+//    (balanced by entry count), accumulates the piece's row and stores it
+//    when its last entry has been applied.  No cross-lane reduction.  With
+//    several work items per wave every stream gets an equal run of entries
+//    instead; a piece cut between runs is finished by the stream that began
+//    it, from the later streams' partial sums in LDS.
+//  - One piece (a long row): the streams interleave over its entries, whose
 //    list is padded to whole blocks, and their sums are added with
 //    cross-lane shuffles before the store.
 // Loads are issued in blocks of U back to back before the block's FMAs; B is
 // read with raw buffer loads whose range check turns out-of-range offsets
 // into zeros, so inactive lanes and placeholder entries need no branch.
-// Rows absent from an entry are updated with a zero value (no per-row
-// select); this is exact for finite B.  A piece of a taller tile (or of any
-// tile off the buffer path) whose sum comes out non-finite is recomputed
-// with the presence bits (read from global memory on that rare path) before
-// it is stored, so inf / NaN in B reach exactly the rows the reference's
-// loop reaches; single-row tiles on the buffer path need no such check.
 //
 // The host launcher runs one launch per column slice of at most 256
-// columns (128 when B is over 512 MB) for 16-byte vectors, and for any
-// vector width when tiles are split (their partial rows are one slice
-// wide); tiles of 16 rows go to the MFMA kernel further down.
+// columns (128 when B is over 512 MB) for taller tiles and for single-row
+// tiles with 16-byte vectors, and for any vector width when tiles are split
+// (their partial rows are one slice wide).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -61,9 +56,6 @@ namespace {
 // Waves per block of the VALU tile kernel: 2 (1.5% faster than 4 on the
 // banded matrix — a freed wave slot waits less for a whole block to fit).
 constexpr int kWaves = 2;
-// Buffer offset of "no B row": at least 2^31, above any buffer-path B size,
-// and still below 2^32 after adding a column offset (< 2^31).
-constexpr uint32_t kNoRow = 0x80000000u;
 // Compute units of a device (256 on MI355X), read once per device.
 int device_cus(int device) {
     static std::atomic<int> cus[64];
@@ -84,88 +76,39 @@ constexpr int32_t kTileWideCols = 256;
 constexpr int32_t kTileSliceCols = 128;
 constexpr uint64_t kTileSliceBytes = 512ull << 20;
 
-template <int R>
-__device__ __forceinline__ void store_vals(float* p, const float (&a)[R]) {
-    if constexpr (R == 1) {
-        p[0] = a[0];
-    } else if constexpr (R == 2) {
-        *reinterpret_cast<float2*>(p) = make_float2(a[0], a[1]);
-    } else {
-#pragma unroll
-        for (int q = 0; q < R; q += 4)
-            *reinterpret_cast<float4*>(p + q) = make_float4(a[q], a[q + 1], a[q + 2], a[q + 3]);
-    }
-}
-
-template <int R>
-__device__ __forceinline__ void load_vals(const float* p, float (&a)[R]) {
-    if constexpr (R == 1) {
-        a[0] = p[0];
-    } else if constexpr (R == 2) {
-        const float2 x = *reinterpret_cast<const float2*>(p);
-        a[0] = x.x;
-        a[1] = x.y;
-    } else {
-#pragma unroll
-        for (int q = 0; q < R; q += 4) {
-            const float4 x = *reinterpret_cast<const float4*>(p + q);
-            a[q] = x.x;
-            a[q + 1] = x.y;
-            a[q + 2] = x.z;
-            a[q + 3] = x.w;
-        }
-    }
-}
-
-// z + x * 0 for every component of x, as fused multiply-adds (no rounding:
-// x * 0 is a signed zero for finite x, NaN otherwise).
-__device__ __forceinline__ float fma_zero_acc(float x, float z) { return __builtin_fmaf(x, 0.f, z); }
-__device__ __forceinline__ float fma_zero_acc(float2 x, float z) {
-    return __builtin_fmaf(x.y, 0.f, __builtin_fmaf(x.x, 0.f, z));
-}
-__device__ __forceinline__ float fma_zero_acc(float4 x, float z) {
-    return __builtin_fmaf(x.w, 0.f, __builtin_fmaf(x.z, 0.f, __builtin_fmaf(x.y, 0.f,
-                          __builtin_fmaf(x.x, 0.f, z))));
-}
-
-// Compile-time shape of the per-wave LDS of the VALU tile kernel.
-template <int VEC, int LPE, int R, int MERGE>
+// Compile-time shape of the per-wave LDS of the single-row kernel.
+template <int VEC, int LPE, int MERGE>
 struct TileShape {
     static constexpr int S = 64 / LPE;                          // streams per wave
-    static constexpr int RS = tile_slot_stride(R);              // slots stored per entry
-    static constexpr int EMAX = tile_piece_entries(R) * MERGE;  // entries per wave
+    static constexpr int EMAX = tile_piece_entries(1) * MERGE;  // entries per wave
     static constexpr int PMAX = kTileChunkPieces * MERGE;       // pieces per wave
-    // Loads per block: 8, or 4 when 8+ streams split a tall tile's entries
-    // (fewer padded entries per block: banded 62K matrix, O = 8 / 32, 3%
-    // faster; single-row tiles, which merge four items, measured slower).
-    static constexpr int U = (S >= 8 && R > 1) ? 4 : 8;
+    static constexpr int U = 8;                                 // loads per block
     // A one-piece item's list is padded with "no row" entries of value 0 up
     // to a multiple of S*UT, so that its blocks are full blocks of U loads
-    // per stream and at most one each of U/2, U/4, ... UT (UT = 2).
-    static constexpr int UT = U >= 2 ? 2 : U;
+    // per stream and at most one each of U/2, U/4.
+    static constexpr int UT = 2;
     static constexpr int EPAD = (EMAX + S * U - 1) / (S * U) * (S * U);
-    // Single-row tiles with several work items per wave: each stream takes
-    // an equal run of the wave's entries, cutting pieces where the runs
-    // meet (the piece's owner adds the other streams' partial sums after the
-    // loop).  Whole pieces per stream leave most streams idle behind a long
-    // row's piece: power-law 322K matrix, O = 8 / 32, 41% of the B-load
-    // slots busy against 84%, 37.1 / 46.1 against 30.0 / 40.1 us.  A stream
-    // that ends a piece begun in an earlier run writes its partial sum to
-    // LDS at once (held in registers, the 16-byte-vector build kept it on
-    // the stack and ran 1.7x slower).
-    static constexpr bool EQ = R == 1 && MERGE > 1;
+    // Several work items per wave: each stream takes an equal run of the
+    // wave's entries, cutting pieces where the runs meet (the piece's owner
+    // adds the other streams' partial sums after the loop).  Whole pieces per
+    // stream leave most streams idle behind a long row's piece: power-law
+    // 322K matrix, O = 8 / 32, 41% of the B-load slots busy against 84%, 37.1
+    // / 46.1 against 30.0 / 40.1 us.  A stream that ends a piece begun in an
+    // earlier run writes its partial sum to LDS at once (held in registers,
+    // the 16-byte-vector build kept it on the stack and ran 1.7x slower).
+    static constexpr bool EQ = MERGE > 1;
 };
 
 // One wave's LDS: staged entries (B-row byte offsets and values), the piece
 // table with its end sentinels, per-piece "not finite" flags and the streams'
 // first pieces.
-template <int VEC, int LPE, int R, int MERGE>
+template <int VEC, int LPE, int MERGE>
 struct TileLds {
-    using Sh = TileShape<VEC, LPE, R, MERGE>;
-    __align__(16) float val[Sh::EPAD * Sh::RS];
+    using Sh = TileShape<VEC, LPE, MERGE>;
+    __align__(16) float val[Sh::EPAD];
     // Equal-run streams: per lane, the partial sum of the piece open at its
     // stream's first entry, and per stream that piece (-1: none).
-    typename VecT<VEC>::T xs[Sh::EQ ? 64 * R : 1];
+    typename VecT<VEC>::T xs[Sh::EQ ? 64 : 1];
     int32_t headp[Sh::EQ ? Sh::S : 1];
     uint32_t brow[Sh::EPAD];
     int4 piece[Sh::PMAX + 2];
@@ -177,29 +120,24 @@ struct TileLds {
 // on one wave.  BUF: B smaller than 2 GB, read with raw buffer loads at
 // 32-bit byte offsets; otherwise 64-bit addresses from B row indices
 // (LPE = 64 only).
-template <int VEC, int LPE, int R, int MERGE, bool BUF>
+template <int VEC, int LPE, int MERGE, bool BUF>
 __device__ __forceinline__ void tile_item(
-    int32_t c0, int32_t c1, int lane, TileLds<VEC, LPE, R, MERGE>& L, int32_t O, int32_t ld,
+    int32_t c0, int32_t c1, int lane, TileLds<VEC, LPE, MERGE>& L, int32_t O, int32_t ld,
     int32_t accumulate, uint32_t b_bytes, const int4* __restrict__ chunks,
-    const int4* __restrict__ pieces, const int32_t* __restrict__ ent_brow,
-    const uint16_t* __restrict__ ent_mask, const float* __restrict__ ent_val,
-    const float* __restrict__ B, float* __restrict__ C, float* __restrict__ partials) {
+    const int4* __restrict__ pieces, const uint16_t* __restrict__ ent_mask,
+    const float* __restrict__ ent_val, const float* __restrict__ B, float* __restrict__ C,
+    float* __restrict__ partials) {
     using V = typename VecT<VEC>::T;
-    using Sh = TileShape<VEC, LPE, R, MERGE>;
+    using Sh = TileShape<VEC, LPE, MERGE>;
     constexpr int S = Sh::S;
-    constexpr int RS = Sh::RS;
-    constexpr bool FOLD = tile_dev_folds_brow(R);            // B row inside the values
-    constexpr int DS = tile_dev_stride(R);                   // floats per entry in ent_val
     constexpr int U = Sh::U;
     constexpr int UT = Sh::UT;
-    // Pieces are checked for non-finite sums (and recomputed with the
-    // presence bits) because a tile row absent from an entry gets 0 * b,
-    // NaN for an infinite b, and because placeholders read B row 0 off the
-    // buffer path.  Single-row tiles on the buffer path have neither: every
-    // entry is present in its row and placeholders load zeros, so their sums
-    // are already the reference's (power-law 322K matrix, O = 8 / 32: 7% /
-    // 5% faster without the check at each piece end).
-    constexpr bool CHECK = !(R == 1 && BUF);
+    // Off the buffer path placeholders read B row 0 times 0, which is NaN for
+    // an infinite b, so a piece's sum is checked and recomputed without them
+    // (the presence bits tell).  On the buffer path placeholders load zeros,
+    // so the sums are already the reference's (power-law 322K matrix, O = 8 /
+    // 32: 7% / 5% faster without the check at each piece end).
+    constexpr bool CHECK = !BUF;
     uint32_t* lb = L.brow;
     uint8_t* lbad = L.bad;
     float* lv = L.val;
@@ -215,34 +153,18 @@ __device__ __forceinline__ void tile_item(
     const int32_t ne_pad = pad ? (ne + S * UT - 1) / (S * UT) * (S * UT) : ne;  // <= EPAD
     for (int32_t i = lane; i < ne_pad; i += 64) {
         uint32_t br = (uint32_t)kTileNoEntry;
-        float a[RS];
+        float a = 0.f;
         if (i < ne) {
-            const int64_t e = (int64_t)e0 + i;
-            if constexpr (FOLD) {
-                // One load: the values, then the B row's bits (for 3 rows in
-                // the padding slot, which the FMAs never read).
-                float rec[DS];
-                load_vals<DS>(ent_val + e * DS, rec);
-                br = __builtin_bit_cast(uint32_t, rec[DS - 1]);
-#pragma unroll
-                for (int q = 0; q < RS; ++q) a[q] = rec[q];
-            } else {
-                br = (uint32_t)ent_brow[e];
-                load_vals<RS>(ent_val + e * RS, a);
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < RS; ++q) a[q] = 0.f;
+            // One load: the value, then the B row's bits.
+            const float2 rec = *reinterpret_cast<const float2*>(ent_val + 2 * ((int64_t)e0 + i));
+            a = rec.x;
+            br = __builtin_bit_cast(uint32_t, rec.y);
         }
         // Placeholders: "no row" on the buffer path, else row 0 times 0.
         const bool real = br != (uint32_t)kTileNoEntry;
         const uint32_t off = BUF ? (real ? br * row_bytes : kNoRow) : (real ? br : 0u);
         lb[i] = off;
-        // 3-row tiles: the offset also goes into the padding slot of the
-        // entry's 4-float value record (the FMAs never read that slot), so
-        // the one-piece loop reads each entry with one 16-byte LDS read.
-        if constexpr (RS > R) a[RS - 1] = __builtin_bit_cast(float, off);
-        store_vals<RS>(lv + i * RS, a);
+        lv[i] = a;
     }
     if (np > 1) {
         for (int32_t j = lane; j < np; j += 64) {
@@ -274,60 +196,37 @@ __device__ __forceinline__ void tile_item(
             return ok ? b : zero_vec(V());
         }
     };
-    // acc[r] += a[r] * b for every tile row; absent rows have a[r] = 0, which
-    // is exact while b is finite.  A non-finite b reaching an absent row
-    // (0 * inf = NaN) shows up as a non-finite row sum at the store, and the
-    // piece is then recomputed with the presence bits (redo_piece).
-    auto apply = [&](V (&acc)[R], int32_t tc, bool ok, const V& b) {
-        float a[RS];
-        load_vals<RS>(lv + tc * RS, a);
-#pragma unroll
-        for (int r = 0; r < R; ++r) fma_vec(acc[r], ok ? a[r] : 0.f, b);
+    auto apply = [&](V& acc, int32_t tc, bool ok, const V& b) {
+        const float a = lv[tc];
+        fma_vec(acc, ok ? a : 0.f, b);
     };
-    // Whether every accumulator of this lane is finite (lanes past O hold
-    // nothing to store).  z = fma(x, 0, z) over all of them stays finite
-    // exactly when every x is (x * 0 is NaN for inf and NaN).  Rows absent
-    // from the piece are included: their sums are zero for finite B, so this
-    // can only send a piece to the exact recomputation more often.
-    auto piece_finite = [&](const V (&acc)[R], bool kok) -> bool {
-        float z = 0.f;
-#pragma unroll
-        for (int r = 0; r < R; ++r) z = fma_zero_acc(acc[r], z);
-        return __builtin_isfinite(z) || !kok;
+    // Whether this lane's sums are finite (lanes past O hold nothing to
+    // store): fma(x, 0, z) over them stays finite exactly when every x is.
+    auto piece_finite = [&](const V& acc, bool kok) -> bool {
+        return __builtin_isfinite(fma_zero_acc(acc, 0.f)) || !kok;
     };
-    // Writes the accumulated rows of piece pc (its first pc.y rows exist) to
-    // C or to its partial rows.
-    auto store_piece = [&](const int4 pc, const V (&acc)[R], int32_t k, bool kok) {
+    // Writes the sums of row `row` to C, or to partial row `part` if that is
+    // not negative.
+    auto store_row = [&](int32_t row, int32_t part, const V& acc, int32_t k, bool kok) {
         if (!kok) return;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (r >= pc.y) break;
-            if (pc.w < 0) {
-                V* dst = reinterpret_cast<V*>(C + (int64_t)(pc.x + r) * ld + k);
-                store_nt(dst, accumulate ? add_vec(*dst, acc[r]) : acc[r]);
-            } else {
-                *reinterpret_cast<V*>(partials + (int64_t)(pc.w + r) * O + k) = acc[r];
-            }
+        if (part < 0) {
+            V* dst = reinterpret_cast<V*>(C + (int64_t)row * ld + k);
+            store_nt(dst, accumulate ? add_vec(*dst, acc) : acc);
+        } else {
+            *reinterpret_cast<V*>(partials + (int64_t)part * O + k) = acc;
         }
     };
-    // Exact recomputation of piece pc (entries tb .. te-1) in entry order,
-    // skipping absent rows (taken only for pieces whose sum is not finite,
-    // which were not stored).
+    // Recomputation of piece pc (entries tb .. te-1) in entry order without
+    // its placeholders (taken only for pieces whose sum is not finite, which
+    // were not stored).
     auto redo_piece = [&](const int4 pc, int32_t tb, int32_t te, int32_t k, uint32_t koff,
                           bool kok) {
-        V acc[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] = zero_vec(V());
+        V acc = zero_vec(V());
         for (int32_t t = tb; t < te; ++t) {
             const V b = load_b(t, true, koff);
-            float a[RS];
-            load_vals<RS>(lv + t * RS, a);
-            const uint32_t m = ent_mask[(int64_t)e0 + t];
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                if ((m >> r) & 1u) fma_vec(acc[r], a[r], b);
+            if (ent_mask[(int64_t)e0 + t] & 1u) fma_vec(acc, lv[t], b);
         }
-        store_piece(pc, acc, k, kok);
+        if (pc.y > 0) store_row(pc.x, pc.w, acc, k, kok);
     };
 
     if (np > 1) {
@@ -382,9 +281,7 @@ __device__ __forceinline__ void tile_item(
             const int32_t k = k0 + kl * VEC;
             const bool kok = k < O;
             const uint32_t koff = (uint32_t)((kok || BUF) ? k : 0) * 4u;
-            V acc[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) acc[r] = zero_vec(V());
+            V acc = zero_vec(V());
             int32_t p = pa, pend = lp[pa + 1].z;
             // Without the finiteness check, the row and partial row of piece
             // p are read when the piece starts, so its store waits on no LDS
@@ -409,8 +306,7 @@ __device__ __forceinline__ void tile_item(
                         if (carry && p == pa) {
                             // The end of a piece begun in an earlier run: its
                             // owner adds this partial sum after the loop.
-#pragma unroll
-                            for (int r = 0; r < R; ++r) L.xs[lane * R + r] = acc[r];
+                            L.xs[lane] = acc;
                         } else if constexpr (CHECK) {
                             // A stream stores a piece only if all its lanes'
                             // sums are finite; otherwise redo_piece computes
@@ -420,13 +316,12 @@ __device__ __forceinline__ void tile_item(
                                 bad = true;
                                 lbad[p] = 1;
                             } else {
-                                store_piece(lp[p], acc, k, kok);
+                                store_row(lp[p].x, lp[p].w, acc, k, kok);
                             }
                         } else {
-                            store_piece(make_int4(cur_x, 1, 0, cur_w), acc, k, kok);
+                            store_row(cur_x, cur_w, acc, k, kok);
                         }
-#pragma unroll
-                        for (int r = 0; r < R; ++r) acc[r] = zero_vec(V());
+                        acc = zero_vec(V());
                         ++p;
                         pend = lp[p + 1].z;
                         if constexpr (!CHECK) {
@@ -450,23 +345,18 @@ __device__ __forceinline__ void tile_item(
                 pb = p;
                 const bool open = lp[p].z < te || (te == tb && carry);
                 const bool middle = open && carry && p == pa;
-                if (middle) {
-#pragma unroll
-                    for (int r = 0; r < R; ++r) L.xs[lane * R + r] = acc[r];
-                }
+                if (middle) L.xs[lane] = acc;
                 if (kl == 0) L.headp[sub] = carry ? pa : -1;
                 wave_sync();
                 if (open && !middle) {
                     for (int32_t s2 = sub + 1; s2 < S && L.headp[s2] == p; ++s2)
-#pragma unroll
-                        for (int r = 0; r < R; ++r)
-                            acc[r] = add_vec(acc[r], L.xs[(s2 * LPE + kl) * R + r]);
+                        acc = add_vec(acc, L.xs[s2 * LPE + kl]);
                     if constexpr (CHECK) {
                         const uint64_t bm = __ballot(!piece_finite(acc, kok));
                         if ((bm & smask) != 0) redo_piece(lp[p], lp[p].z, lp[p + 1].z, k, koff, kok);
-                        else store_piece(lp[p], acc, k, kok);
+                        else store_row(lp[p].x, lp[p].w, acc, k, kok);
                     } else {
-                        store_piece(lp[p], acc, k, kok);
+                        store_row(lp[p].x, lp[p].w, acc, k, kok);
                     }
                 }
                 wave_sync();
@@ -490,9 +380,7 @@ __device__ __forceinline__ void tile_item(
             const int32_t k = k0 + kl * VEC;
             const bool kok = k < O;
             const uint32_t koff = (uint32_t)((kok || BUF) ? k : 0) * 4u;
-            V acc[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) acc[r] = zero_vec(V());
+            V acc = zero_vec(V());
             auto block = [&](auto full_c, int32_t i0) {
                 constexpr bool FULL = decltype(full_c)::value;
                 V b[U];
@@ -515,42 +403,19 @@ __device__ __forceinline__ void tile_item(
                 auto block_n = [&](auto nu_c, int32_t i0) {
                     constexpr int NU = decltype(nu_c)::value;
                     V b[NU];
-                    if constexpr (RS > R) {
-                        // One LDS record per entry: values and B-row offset
-                        // (banded 62K matrix: O = 8 / 32 5% / 7% faster than
-                        // separate offset and value reads, O = 128 2%).
-                        static_assert(RS == 4, "padding slot of a 4-float record");
-                        float4 rec[NU];
 #pragma unroll
-                        for (int u = 0; u < NU; ++u)
-                            rec[u] = *reinterpret_cast<const float4*>(lv + (sub + S * (i0 + u)) * RS);
+                    for (int u = 0; u < NU; ++u) b[u] = load_b(sub + S * (i0 + u), true, koff);
 #pragma unroll
-                        for (int u = 0; u < NU; ++u)
-                            b[u] = load_b_buf<VEC>(rsrc, __builtin_bit_cast(uint32_t, rec[u].w) + koff);
-#pragma unroll
-                        for (int u = 0; u < NU; ++u)
-#pragma unroll
-                            for (int r = 0; r < R; ++r)
-                                fma_vec(acc[r], reinterpret_cast<const float*>(&rec[u])[r], b[u]);
-                    } else {
-#pragma unroll
-                        for (int u = 0; u < NU; ++u) b[u] = load_b(sub + S * (i0 + u), true, koff);
-#pragma unroll
-                        for (int u = 0; u < NU; ++u) apply(acc, sub + S * (i0 + u), true, b[u]);
-                    }
+                    for (int u = 0; u < NU; ++u) apply(acc, sub + S * (i0 + u), true, b[u]);
                 };
                 const int32_t nper_pad = ne_pad / S;
                 int32_t i0 = 0;
                 for (; i0 + U <= nper_pad; i0 += U) block_n(std::integral_constant<int, U>(), i0);
-                if constexpr (U / 2 >= UT) {
-                    if (i0 + U / 2 <= nper_pad) {
-                        block_n(std::integral_constant<int, U / 2>(), i0);
-                        i0 += U / 2;
-                    }
+                if (i0 + U / 2 <= nper_pad) {
+                    block_n(std::integral_constant<int, U / 2>(), i0);
+                    i0 += U / 2;
                 }
-                if constexpr (U / 4 >= UT) {
-                    if (i0 + U / 4 <= nper_pad) block_n(std::integral_constant<int, U / 4>(), i0);
-                }
+                if (i0 + U / 4 <= nper_pad) block_n(std::integral_constant<int, U / 4>(), i0);
             } else {
                 for (int32_t i0 = 0; i0 < nper; i0 += U) {
                     if (i0 + U <= nfull) block(std::true_type(), i0);
@@ -558,63 +423,34 @@ __device__ __forceinline__ void tile_item(
                 }
             }
 #pragma unroll
-            for (int sh = LPE; sh < 64; sh <<= 1) {
-#pragma unroll
-                for (int r = 0; r < R; ++r) acc[r] = add_vec(acc[r], shfl_xor_vec(acc[r], sh));
-            }
-            // The butterfly leaves every stream the same sums (each step adds
-            // the same two values in either order), so stream s stores rows
-            // s, s + S, ...: one store instruction per S rows instead of one
-            // per row (banded 62K matrix, O = 8: 9.9 -> 9.45 us).  A sum that
-            // is not finite is recomputed exactly by stream 0.
-            const bool bad = CHECK && !piece_finite(acc, kok);
-            if (__any(bad)) {
+            for (int sh = LPE; sh < 64; sh <<= 1) acc = add_vec(acc, shfl_xor_vec(acc, sh));
+            if (CHECK && __any(!piece_finite(acc, kok))) {
                 if (sub == 0) redo_piece(pc1, pc1.z, ne, k, koff, kok);
-            } else if (kok) {
-#pragma unroll
-                for (int i = 0; i < (R + S - 1) / S; ++i) {
-                    const int r = i * S + sub;
-                    if (r < R && r < pc1.y) {
-                        V x = acc[0];
-#pragma unroll
-                        for (int q = 1; q < R; ++q)
-                            if (q == r) x = acc[q];
-                        if (pc1.w < 0) {
-                            V* dst = reinterpret_cast<V*>(C + (int64_t)(pc1.x + r) * ld + k);
-                            store_nt(dst, accumulate ? add_vec(*dst, x) : x);
-                        } else {
-                            *reinterpret_cast<V*>(partials + (int64_t)(pc1.w + r) * O + k) = x;
-                        }
-                    }
-                }
+            } else if (sub == 0 && pc1.y > 0) {
+                store_row(pc1.x, pc1.w, acc, k, kok);
             }
         }
     }
 }
 
-
-// One wave per MERGE consecutive work items of the view.  Up to 3 tile rows
-// (one work item per wave) the register budget is held to 5 waves per SIMD:
-// measured faster than 4 on the banded workload; 6 spills, and so does 5
-// with 4 rows.
-template <int VEC, int LPE, int R, int MERGE, bool BUF>
+// One wave per MERGE consecutive work items of the view.
+template <int VEC, int LPE, int MERGE, bool BUF>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu((R <= 3 && MERGE == 1) ? 5 : 1, 8)))
+__attribute__((amdgpu_waves_per_eu(MERGE == 1 ? 5 : 1, 8)))
 void vcsr_tile_kernel(
     int32_t n_chunks, int32_t O, int32_t ld, int32_t accumulate, uint32_t b_bytes,
     const int4* __restrict__ chunks, const int4* __restrict__ pieces,
-    const int32_t* __restrict__ ent_brow, const uint16_t* __restrict__ ent_mask,
-    const float* __restrict__ ent_val, const float* __restrict__ B, float* __restrict__ C,
-    float* __restrict__ partials) {
-    __shared__ TileLds<VEC, LPE, R, MERGE> s_lds[kWaves];
+    const uint16_t* __restrict__ ent_mask, const float* __restrict__ ent_val,
+    const float* __restrict__ B, float* __restrict__ C, float* __restrict__ partials) {
+    __shared__ TileLds<VEC, LPE, MERGE> s_lds[kWaves];
     // Wave-uniform indices, so the work-item records are scalar loads.
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = (int)(threadIdx.x & 63);
     const int32_t w = (int32_t)(xcd_remap(blockIdx.x, gridDim.x) * kWaves) + wave;
     const int32_t c0 = w * MERGE;
     if (c0 >= n_chunks) return;
-    tile_item<VEC, LPE, R, MERGE, BUF>(c0, min(n_chunks, c0 + MERGE) - 1, lane, s_lds[wave], O, ld,
-                                       accumulate, b_bytes, chunks, pieces, ent_brow, ent_mask,
+    tile_item<VEC, LPE, MERGE, BUF>(c0, min(n_chunks, c0 + MERGE) - 1, lane, s_lds[wave], O, ld,
+                                       accumulate, b_bytes, chunks, pieces, ent_mask,
                                        ent_val, B, C, partials);
 }
 
@@ -944,28 +780,26 @@ hipError_t launch_mma(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t
     return hipGetLastError();
 }
 
-template <int VEC, int LPE, int R, bool BUF>
+template <int VEC, int LPE, bool BUF>
 hipError_t launch_one(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
                       int32_t accumulate, uint32_t b_bytes, float* partials, hipStream_t st) {
-    // Eight streams per wave (B slices of at most 8 columns) and single-row
-    // tiles: four work items per wave, so each stream still gets several
-    // rows.  Taller tiles stay one per wave (their streams split the tile's
-    // entries): measured 1.7x faster than four per wave at O = 8, R = 3.
-    constexpr int MERGE = (64 / LPE >= 8 && R == 1) ? 4 : 1;
+    // Eight streams per wave: four work items per wave, so that each stream
+    // still gets several rows.
+    constexpr int MERGE = 64 / LPE >= 8 ? 4 : 1;
     const int64_t waves = ((int64_t)d.tv_n_chunks + MERGE - 1) / MERGE;
     const dim3 grid((unsigned)((waves + kWaves - 1) / kWaves)), block(64 * kWaves);
-    hipLaunchKernelGGL((vcsr_tile_kernel<VEC, LPE, R, MERGE, BUF>), grid, block, 0, st, d.tv_n_chunks, O,
+    hipLaunchKernelGGL((vcsr_tile_kernel<VEC, LPE, MERGE, BUF>), grid, block, 0, st, d.tv_n_chunks, O,
                        ld, accumulate, b_bytes, reinterpret_cast<const int4*>(d.tv_chunks),
-                       reinterpret_cast<const int4*>(d.tv_pieces), d.tv_brow, d.tv_mask, d.tv_val, B,
-                       C, partials);
+                       reinterpret_cast<const int4*>(d.tv_pieces), d.tv_mask, d.tv_val, B, C,
+                       partials);
     return hipGetLastError();
 }
 
-template <int VEC, int R>
+template <int VEC>
 hipError_t launch_r(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
                     int32_t accumulate, uint64_t b_bytes, float* partials, hipStream_t st) {
     if (b_bytes + 64u * 4u * (uint64_t)VEC >= kBufferLimit)
-        return launch_one<VEC, 64, R, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
+        return launch_one<VEC, 64, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
     const uint32_t bb = (uint32_t)b_bytes;
     // Lanes per entry: the smallest power of two covering O, at least 8 (at
     // most 8 streams per wave, so every stream gets several tiles); 8 lanes
@@ -973,11 +807,11 @@ hipError_t launch_r(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, f
     const int32_t need = (O + VEC - 1) / VEC;
     if constexpr (VEC == 1 || VEC == 4) {
         if (need <= 8)
-            return launch_one<VEC, 8, R, true>(d, B, O, ld, C, accumulate, bb, partials, st);
+            return launch_one<VEC, 8, true>(d, B, O, ld, C, accumulate, bb, partials, st);
     }
-    if (need <= 16) return launch_one<VEC, 16, R, true>(d, B, O, ld, C, accumulate, bb, partials, st);
-    if (need <= 32) return launch_one<VEC, 32, R, true>(d, B, O, ld, C, accumulate, bb, partials, st);
-    return launch_one<VEC, 64, R, true>(d, B, O, ld, C, accumulate, bb, partials, st);
+    if (need <= 16) return launch_one<VEC, 16, true>(d, B, O, ld, C, accumulate, bb, partials, st);
+    if (need <= 32) return launch_one<VEC, 32, true>(d, B, O, ld, C, accumulate, bb, partials, st);
+    return launch_one<VEC, 64, true>(d, B, O, ld, C, accumulate, bb, partials, st);
 }
 
 // Columns [0, O) of B and C, whose rows are ld floats apart (B and C point
@@ -990,11 +824,11 @@ hipError_t launch_vec(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t
         const uint64_t b_bytes = v.N > 0 ? ((uint64_t)(v.N - 1) * (uint64_t)ld + (uint64_t)O) * 4u : 0u;
         hipError_t e;
         switch (d.tv_R) {
-            case 1: e = launch_r<VEC, 1>(d, B, O, ld, C, accumulate, b_bytes, partials, st); break;
-            case 2: e = launch_r<VEC, 2>(d, B, O, ld, C, accumulate, b_bytes, partials, st); break;
-            case 3: e = launch_r<VEC, 3>(d, B, O, ld, C, accumulate, b_bytes, partials, st); break;
-            case 4: e = launch_r<VEC, 4>(d, B, O, ld, C, accumulate, b_bytes, partials, st); break;
-            case 8: e = launch_r<VEC, 8>(d, B, O, ld, C, accumulate, b_bytes, partials, st); break;
+            case 1: e = launch_r<VEC>(d, B, O, ld, C, accumulate, b_bytes, partials, st); break;
+            case 2:
+            case 3:
+            case 4:
+            case 8: e = launch_vcsr_tall(d, B, O, ld, C, accumulate, b_bytes, partials, st); break;
             case kTileMmaRows:
                 e = launch_mma<VEC>(v, d, B, O, ld, C, accumulate, partials, st);
                 break;
@@ -1043,7 +877,12 @@ static int tile_mma_vec(const DeviceFmt& d, int32_t w) {
     return vec;
 }
 
-// Floats per lane and B slice of the other tiles: 4 when O allows 8 lanes of
+// Floats per lane of tiles of 2 to 8 rows for w columns of any alignment
+// (the shapes of vcsr_tile_tall.hip); the reduce of their partial rows takes
+// the same.
+static int tile_tall_vec(int32_t R, int32_t w) { return w > 32 || (w > 16 && R < 4) ? 4 : 1; }
+
+// Floats per lane and B slice of single-row tiles: 4 when O allows 8 lanes of
 // 16-byte vectors and B and C are 16-byte aligned, else 2 or 1.  At O = 32,
 // 4 floats per lane measured 3% / 8% faster than 2 on the banded /
 // power-law matrices.
@@ -1075,7 +914,8 @@ static TileSlicing tile_slicing(const Vcsr& v, const DeviceFmt& d, const float* 
     TileSlicing ts{tile_vec(O, a16, a8), O};
     if (d.tv_R == kTileMmaRows) {
         ts.vec = tile_mma_vec(d, d.tv_partial_rows > 0 ? std::min(O, kTileWideCols) : O);
-    } else if (ts.vec == 4) {
+    } else if (ts.vec == 4 || d.tv_R > 1) {
+        if (d.tv_R > 1) ts.vec = tile_tall_vec(d.tv_R, O);
         if ((uint64_t)v.N * (uint64_t)O * 4u > kTileSliceBytes) ts.width = std::min(O, kTileSliceCols);
         else ts.width = std::min(O, kTileWideCols);
     }
@@ -1117,7 +957,7 @@ hipError_t launch_vcsr_tile(const Vcsr& v, const DeviceFmt& d, const float* B, i
     for (int32_t c0 = 0; c0 < O; c0 += ts.width) {
         const int32_t w = std::min(ts.width, O - c0);
         hipError_t e;
-        switch (d.tv_R == kTileMmaRows ? tile_mma_vec(d, w) : ts.vec) {
+        switch (d.tv_R == kTileMmaRows ? tile_mma_vec(d, w) : d.tv_R > 1 ? tile_tall_vec(d.tv_R, w) : ts.vec) {
             case 4: e = launch_vec<4>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;
             case 2: e = launch_vec<2>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;
             default: e = launch_vec<1>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;

@@ -14,9 +14,20 @@
 //     into the piece's R accumulator rows.
 //  3. The streams' sums are added by an xor butterfly inside the piece's
 //     lanes, and stream s stores rows s, s + S, ... .
+// Bound by the L2-to-CU path (one B slice per entry) at wide B, by the view's
+// arrival and the loads' latency at narrow B.  Against one kernel for all
+// tile heights that packed several tiles per wave in stream mode: only this
+// path's registers are held (66 instead of 94 at 3 rows and O = 128: 7 waves
+// per SIMD instead of 5), a wave waits for one record and one round of entry
+// loads instead of up to four loads in sequence, and short tiles share a wave
+// without a per-entry test for the piece's end.  Banded 62K matrix, three
+// formats in turn, O = 8 / 32 / 128 / 512: 17.3 / 23.1 / 33.2 / 151 -> 8.4 /
+// 12.2 / 30.3 / 145 us; 30K rows of 6-row blocks, O = 50: 27.5 -> 12.2.
 // Rows absent from an entry are updated with a zero value, which is exact for
 // finite B; a piece with a non-finite sum is recomputed with the presence
 // bits before it is stored.
+#include <type_traits>
+
 #include "../host/tile_view.hpp"
 #include "common.hpp"
 #include "launch.hpp"
@@ -26,15 +37,12 @@ namespace vcsr {
 namespace {
 
 constexpr int kWaves = 2;
-// Buffer offset of "no B row": at least 2^31, above any buffer-path B size,
-// and still below 2^32 after adding a column offset (< 2^31).
-constexpr uint32_t kNoRow = 0x80000000u;
 
-template <int LPE, int S, int R>
+// U loads per block.
+template <int LPE, int S, int R, int U>
 struct TallShape {
     static constexpr int TL = LPE * S;      // lanes per piece
     static constexpr int G = 64 / TL;       // pieces per wave
-    static constexpr int U = S >= 8 ? 4 : 8;  // loads per block
     static constexpr int UT = 2;            // the list is padded to S*UT entries
     // Entries staged at a time; longer pieces (8-row tiles) take several
     // rounds, which keeps the LDS list small.
@@ -47,15 +55,15 @@ struct TallShape {
     static_assert(SEG % (S * UT) == 0, "padded list fits");
 };
 
-template <int LPE, int S, int R>
+template <int LPE, int S, int R, int U>
 struct TallLds {
-    using Sh = TallShape<LPE, S, R>;
+    using Sh = TallShape<LPE, S, R, U>;
     // The lists of a wave's pieces start S entries further on in the banks.
     __align__(16) float val[Sh::G][(Sh::SEG + (Sh::G > 1 ? S : 0)) * Sh::VF];
     uint32_t off[Sh::REC ? 1 : Sh::G][Sh::REC ? 1 : Sh::SEG + (Sh::G > 1 ? S : 0)];
 };
 
-template <int VEC, int LPE, int S, int R, bool BUF>
+template <int VEC, int LPE, int S, int R, int U, bool BUF>
 __global__ __launch_bounds__(64 * kWaves)
 __attribute__((amdgpu_waves_per_eu(R <= 3 ? 5 : 1, 8)))
 void vcsr_tall_kernel(
@@ -64,11 +72,11 @@ void vcsr_tall_kernel(
     const uint16_t* __restrict__ ent_mask, const float* __restrict__ ent_val,
     const float* __restrict__ B, float* __restrict__ C, float* __restrict__ partials) {
     using V = typename VecT<VEC>::T;
-    using Sh = TallShape<LPE, S, R>;
-    constexpr int TL = Sh::TL, G = Sh::G, U = Sh::U, UT = Sh::UT, SEG = Sh::SEG, VF = Sh::VF;
+    using Sh = TallShape<LPE, S, R, U>;
+    constexpr int TL = Sh::TL, G = Sh::G, UT = Sh::UT, SEG = Sh::SEG, VF = Sh::VF;
     constexpr int RS = tile_slot_stride(R);      // value floats per entry of the view
     constexpr bool FOLD = tile_dev_folds_brow(R);
-    __shared__ TallLds<LPE, S, R> s_lds[kWaves];
+    __shared__ TallLds<LPE, S, R, U> s_lds[kWaves];
 
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = (int)(threadIdx.x & 63);
@@ -199,7 +207,13 @@ void vcsr_tall_kernel(
             }
         }
         if constexpr (U / 4 >= UT) {
-            if (i0 + U / 4 <= steps) block(std::integral_constant<int, U / 4>(), i0);
+            if (i0 + U / 4 <= steps) {
+                block(std::integral_constant<int, U / 4>(), i0);
+                i0 += U / 4;
+            }
+        }
+        if constexpr (U / 8 >= UT) {
+            if (i0 + U / 8 <= steps) block(std::integral_constant<int, U / 8>(), i0);
         }
     }
 
@@ -247,60 +261,60 @@ void vcsr_tall_kernel(
     }
 }
 
-template <int VEC, int LPE, int S, int R, bool BUF>
+template <int VEC, int LPE, int S, int R, int U, bool BUF>
 hipError_t launch_shape(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
                         int32_t accumulate, uint32_t b_bytes, float* partials, hipStream_t st) {
-    constexpr int per = TallShape<LPE, S, R>::G * kWaves;
+    constexpr int per = TallShape<LPE, S, R, U>::G * kWaves;
     const dim3 grid((unsigned)(((int64_t)d.tv_n_pieces + per - 1) / per)), block(64 * kWaves);
-    hipLaunchKernelGGL((vcsr_tall_kernel<VEC, LPE, S, R, BUF>), grid, block, 0, st, d.tv_n_pieces, O,
+    hipLaunchKernelGGL((vcsr_tall_kernel<VEC, LPE, S, R, U, BUF>), grid, block, 0, st, d.tv_n_pieces, O,
                        ld, accumulate, b_bytes, reinterpret_cast<const int4*>(d.tv_pieces),
                        d.tv_brow, d.tv_mask, d.tv_val, B, C, partials);
     return hipGetLastError();
 }
+
+template <int X>
+using I = std::integral_constant<int, X>;
 
 template <int R>
 hipError_t launch_rows(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
                        int32_t accumulate, uint64_t b_bytes, float* partials, hipStream_t st) {
     if (b_bytes >= kBufferLimit) {
         if (O < 4)
-            return launch_shape<1, 64, 1, R, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
-        return launch_shape<4, 64, 1, R, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
+            return launch_shape<1, 64, 1, R, 8, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
+        return launch_shape<4, 64, 1, R, 8, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
     }
     const uint32_t bb = (uint32_t)b_bytes;
-#define GO(V, L, S) return launch_shape<V, L, S, R, true>(d, B, O, ld, C, accumulate, bb, partials, st)
-    static const int cfg = getenv("TALL") ? atoi(getenv("TALL")) : 0;
-    if (O <= 8) {
-        if (cfg == 1) GO(1, 8, 4);
-        if (cfg == 2) GO(1, 8, 2);
-        if (cfg == 3) GO(1, 8, 1);
-        GO(1, 8, 8);
-    }
-    if (O <= 16) {
-        if (cfg == 1) GO(2, 8, 4);
-        if (cfg == 2) GO(2, 8, 2);
-        if (cfg == 3) GO(1, 16, 4);
-        if (cfg == 4) GO(1, 16, 2);
-        GO(2, 8, 8);
-    }
+    // The shape <floats per lane, lanes per entry, streams per piece, loads
+    // per block> by width, and by the pieces' mean entry count where that
+    // decides how many lanes a piece can feed.  us per SpMM on banded
+    // matrices of 62K rows, three formats in turn (so that the view comes
+    // from beyond L2), blocks of 3 / 6 / 4 / 2 rows with 64 / 60 / 40 / 40
+    // entries a row and 120K rows of 3-row blocks with 24:
+    //  O = 8   <1,8,4,8> 8.4 / 9.7 / 7.1 / 7.8 / 8.8;   <1,8,8,4> 9.4 (3 rows)
+    //  O = 16  <1,16,4,8> 10.3 / 10.5 / 7.7 / 10.9 / 12.7
+    //          <1,16,2,8> 10.4 / 11.5 / 8.2 / 8.8 / 10.4
+    //  O = 32  <4,8,4,4> 12.2 / 15.0 / 10.1 / 12.4 / 12.9
+    //          <1,32,2,16> 13.1 / 13.2 / 9.3 / 11.9 / 14.7
+    //  O = 64  <4,16,4,4> 18.1 / 18.1 / 13.2 / 17.3 / 20.0
+    //          <4,16,2,4> 18.9 / 19.7 / 13.6 / 17.4 / 17.8
+    //  O = 128 <4,32,2,4> 30.3 / 26.2 / 20.4 / 28.3 / 29.7
+    //          <4,32,1,8> 31.5 / 30.1 / 20.8 / 29.6 / 34.2
+    const int64_t mean = d.tv_n_entries / d.tv_n_pieces;
+    auto go = [&](auto vec, auto lpe, auto s, auto u) {
+        return launch_shape<decltype(vec)::value, decltype(lpe)::value, decltype(s)::value, R,
+                            decltype(u)::value, true>(d, B, O, ld, C, accumulate, bb, partials, st);
+    };
+    if (O <= 8) return go(I<1>(), I<8>(), I<4>(), I<8>());
+    if (O <= 16)
+        return mean > 48 ? go(I<1>(), I<16>(), I<4>(), I<8>()) : go(I<1>(), I<16>(), I<2>(), I<8>());
     if (O <= 32) {
-        if (cfg == 1) GO(4, 8, 4);
-        if (cfg == 2) GO(4, 8, 2);
-        if (cfg == 3) GO(2, 16, 4);
-        if (cfg == 4) GO(2, 16, 2);
-        if (cfg == 5) GO(1, 32, 2);
-        GO(4, 8, 8);
+        if constexpr (R >= 4) return go(I<1>(), I<32>(), I<2>(), I<16>());
+        else return go(I<4>(), I<8>(), I<4>(), I<4>());
     }
-    if (O <= 64) {
-        if (cfg == 1) GO(4, 16, 2);
-        if (cfg == 2) GO(4, 16, 1);
-        if (cfg == 3) GO(2, 32, 2);
-        GO(4, 16, 4);
-    }
-    if (O <= 128) {
-        if (cfg == 1) GO(4, 32, 1);
-        GO(4, 32, 2);
-    }
-    GO(4, 64, 1);
+    if (O <= 64)
+        return mean > 32 ? go(I<4>(), I<16>(), I<4>(), I<4>()) : go(I<4>(), I<16>(), I<2>(), I<4>());
+    if (O <= 128) return go(I<4>(), I<32>(), I<2>(), I<4>());
+    return go(I<4>(), I<64>(), I<1>(), I<8>());
 }
 
 }  // namespace

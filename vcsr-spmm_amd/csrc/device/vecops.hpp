@@ -149,6 +149,21 @@ __device__ __forceinline__ typename VecT<VEC>::T load_b_buf(__amdgpu_buffer_rsrc
         return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
 }
 
+// Buffer offset of "no B row": at least 2^31, above any buffer-path B size,
+// and still below 2^32 after adding a column offset (< 2^31).
+constexpr uint32_t kNoRow = 0x80000000u;
+
+// z + x * 0 for every component of x, as fused multiply-adds (no rounding:
+// x * 0 is a signed zero for finite x, NaN otherwise).
+__device__ __forceinline__ float fma_zero_acc(float x, float z) { return __builtin_fmaf(x, 0.f, z); }
+__device__ __forceinline__ float fma_zero_acc(float2 x, float z) {
+    return __builtin_fmaf(x.y, 0.f, __builtin_fmaf(x.x, 0.f, z));
+}
+__device__ __forceinline__ float fma_zero_acc(float4 x, float z) {
+    return __builtin_fmaf(x.w, 0.f, __builtin_fmaf(x.z, 0.f, __builtin_fmaf(x.y, 0.f,
+                          __builtin_fmaf(x.x, 0.f, z))));
+}
+
 // Orders this wave's LDS writes before its later LDS reads (the wave's
 // lanes run in lock step; the fences keep the compiler from reordering).
 __device__ __forceinline__ void wave_sync() {

@@ -41,7 +41,9 @@ struct DeviceFmt {
     int32_t tv_R = 1;                   // accumulator rows per tile
     int32_t* tv_chunks = nullptr;       // 4*tv_n_chunks: entry range, piece range
     int32_t tv_n_chunks = 0;
-    int32_t* tv_pieces = nullptr;       // 4 per piece: row, rows, first entry, partial row
+    int32_t* tv_pieces = nullptr;       // 4 per piece: row, rows, first entry, partial row;
+                                        // then one whose first entry is the entry count
+    int32_t tv_n_pieces = 0;
     int32_t* tv_brow = nullptr;         // per entry: B row, kTileNoEntry for placeholders
                                         // (not uploaded for 1- and 3-row tiles)
     float* tv_val = nullptr;            // tile_dev_stride per entry: values (0 where absent),
