@@ -107,3 +107,68 @@ def test_tall_tiles_nonfinite_b(gpu, orc, st, R, O):
     assert np.array_equal(np.isinf(got), np.isinf(ref))
     fin = np.isfinite(ref)
     assert np.allclose(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
+
+
+def _mixed_rows(vs, rng, long_row=True):
+    """Row lengths around the edges of work items (16, 32, 64 entries), empty
+    rows, runs of one-entry rows and a row cut into ten pieces."""
+    lens = [0, 1, 2, 15, 16, 17, 31, 32, 33, 0, 0, 63, 64, 65, 1, 1, 1, 129] + [1] * 70 + \
+        [3, 5, 7] * 30 + [40, 20] * 8 + ([600] if long_row else []) + [0] * 40 + [2]
+    N = 1500
+    rows = np.repeat(np.arange(len(lens)), lens).astype(np.int32)
+    cols = np.concatenate([np.sort(rng.choice(N, size=n, replace=False)) for n in lens])
+    return vs.coo_to_csr(vs.Coo.from_arrays(len(lens), N, rows, cols.astype(np.int32),
+                                            rng.standard_normal(rows.size).astype(np.float32)))
+
+
+_ROW_WIDTHS = [1, 3, 7, 8, 9, 16, 17, 30, 32, 33, 50, 64, 65, 127, 129, 255, 257]
+
+
+@pytest.mark.parametrize("copies,O,off", [(c, O, off) for c in (1, 40) for O in _ROW_WIDTHS
+                                          for off in (0, 4)] +
+                         [(600, O, 0) for O in _ROW_WIDTHS if O < 130])
+def test_row_tiles_any_width(gpu, orc, st, copies, O, off):
+    """Single-row tiles at every width class and its edges; 40 and 600
+    copies of the matrix below each other take 1, 2 and 4 work items per
+    wave.  C = A*B and C += A*B against the oracle, twice the same bits."""
+    vs = gpu
+    rng = np.random.default_rng(O)
+    one = _mixed_rows(vs, rng)
+    rp = np.concatenate([[0]] + [one.row_ptr[1:].astype(np.int64) + i * one.nnz
+                                 for i in range(copies)]).astype(np.int32)
+    csr = vs.Csr.from_arrays(one.M * copies, one.N, rp, np.tile(one.col, copies),
+                             np.tile(one.val, copies))
+    fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
+    fmt.set_tile_rows(1)
+    fmt.upload(st)
+    B = vs.gen_dense(O, 0, csr.N, O)
+    C0 = rng.integers(-2, 3, size=(csr.M, O)).astype(np.float32)
+    ref = np.tile(orc.spmm_f64(one.M, one.row_ptr, one.col, one.val, B), (copies, 1))
+    got = _spmm(vs, fmt, B, C0, off, st, False)
+    assert_within_tolerance(got, ref, csr.row_ptr, csr.val, B, f"O{O}")
+    assert np.array_equal(got, _spmm(vs, fmt, B, C0, off, st, False))
+    got = _spmm(vs, fmt, B, C0, off, st, True)
+    err = np.abs(got - (C0 + ref)) - 2.0 ** -23 * (np.abs(C0) + np.abs(ref))
+    l1 = np.add.reduceat(np.append(np.abs(csr.val), 0), csr.row_ptr[:-1])
+    l1[np.diff(csr.row_ptr) == 0] = 0
+    assert (err <= 1e-4 * l1[:, None] * np.abs(B).max()).all()
+
+
+@pytest.mark.parametrize("O", [5, 8, 12, 30, 47, 100])
+def test_row_tiles_nonfinite_b(gpu, orc, st, O):
+    """inf and NaN in B reach exactly the rows the oracle's loop reaches."""
+    vs = gpu
+    rng = np.random.default_rng(O)
+    csr = _mixed_rows(vs, rng)
+    fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
+    fmt.set_tile_rows(1)
+    fmt.upload(st)
+    B = vs.gen_dense(O, 0, csr.N, O)
+    for r, c, x in [(0, 0, np.nan), (3, O - 1, np.inf), (700, O - 2, np.nan), (701, 0, -np.inf)]:
+        B[r, c] = x
+    ref = orc.spmm_f32(csr.M, csr.row_ptr, csr.col, csr.val, B)
+    got = _spmm(vs, fmt, B, np.zeros((csr.M, O), np.float32), 0, st, False)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isinf(got), np.isinf(ref))
+    fin = np.isfinite(ref)
+    assert np.allclose(got[fin], ref[fin], rtol=1e-4, atol=1e-4)

@@ -10,6 +10,9 @@
 
 namespace vcsr {
 
+// Compute units of a device (256 on MI355X), read once per device.
+int device_cus(int device);
+
 // csr_naive.hip: C = A*B, one thread per row.
 hipError_t launch_csr_naive(int32_t M, const int32_t* rowptr, const int32_t* col,
                             const float* val, const float* B, int32_t O, float* C,
@@ -52,22 +55,25 @@ int64_t rowmajor_partials_floats(const DeviceFmt& d, int32_t O);
 // vcsr_tile.hip: tile-stationary traversal of the VCSR slots through the
 // row-tile view; C = A*B (accumulate = 0) or C += A*B (accumulate = 1).
 // `partials` holds the partial rows of split tiles: at least
-// tile_partials_floats(v, d, B, O, C) floats (none when the view has no
+// tile_partials_floats(v, d, O) floats (none when the view has no
 // split tile); every partial row the launch reads it writes first.
 hipError_t launch_vcsr_tile(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t O,
                             float* C, int32_t accumulate, float* partials, hipStream_t st);
-int64_t tile_partials_floats(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t O,
-                             const float* C);
-// The launch over its tiles of 2, 3, 4 or 8 rows (vcsr_tile_tall.hip) for
+int64_t tile_partials_floats(const Vcsr& v, const DeviceFmt& d, int32_t O);
+// The launches over single-row tiles (vcsr_tile_row.hip) and over tiles of
+// 2, 3, 4 or 8 rows (vcsr_tile_tall.hip) for
 // columns [0, O) of B and C, at most 256, whose rows are ld floats apart;
 // b_bytes from B to the end of its last row.
+hipError_t launch_vcsr_row_tiles(const DeviceFmt& d, const float* B, int32_t O, int32_t ld,
+                                 float* C, int32_t accumulate, uint64_t b_bytes, float* partials,
+                                 hipStream_t st);
 hipError_t launch_vcsr_tall(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
                             int32_t accumulate, uint64_t b_bytes, float* partials, hipStream_t st);
-// Partial-row floats that cover tile_partials_floats for every O, B and C:
+// Partial-row floats that cover tile_partials_floats for every O:
 // a view with split tiles is launched in column slices of at most 256
 // columns, and its partial rows are one slice wide.
 int64_t tile_partials_upload_floats(const DeviceFmt& d);
-// What launch_vcsr_tile launches for these B and C: floats per lane, column
+// What launch_vcsr_tile launches at width O: floats per lane, column
 // slices (one launch each), whether the tiles run on the matrix cores, the
 // reduce launches and the partial-row floats.
 struct TilePlan {
@@ -77,11 +83,9 @@ struct TilePlan {
     int32_t reduce_launches = 0;
     int64_t partial_floats = 0;
 };
-TilePlan tile_launch_plan(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t O,
-                          const float* C);
+TilePlan tile_launch_plan(const Vcsr& v, const DeviceFmt& d, int32_t O);
 // MFMA instructions launch_vcsr_tile issues for one SpMM of width O when
-// the view has 16-row tiles (none otherwise), as launched for the alignment
-// of 16-byte aligned B and C.
+// the view has 16-row tiles (none otherwise).
 MfmaWork tile_mfma_work(const DeviceFmt& d, int32_t O);
 
 // A row-stationary work item covers at most this many (group, lane) pair

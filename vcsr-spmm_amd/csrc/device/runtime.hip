@@ -174,7 +174,7 @@ void free_device_fmt(DeviceFmt& d) {
                     (void*)d.items, (void*)d.pair_rec, (void*)d.row_items, (void*)d.split_rows,
                     (void*)d.tv_chunks, (void*)d.tv_pieces, (void*)d.tv_brow, (void*)d.tv_val,
                     (void*)d.tv_mask,
-                    (void*)d.tv_split, (void*)d.partials})
+                    (void*)d.tv_items, (void*)d.tv_dest, (void*)d.tv_split, (void*)d.partials})
         if (p) (void)hipFree(p);
     if (d.device >= 0 && d.device != cur && cur >= 0) (void)hipSetDevice(cur);
     d = DeviceFmt();
@@ -225,8 +225,32 @@ int vcsr_fmt_upload(vcsr_fmt* fmt, void* stream) {
                 std::memcpy(&tv_val[q * ds + ds - 1], &tv_brow[q], sizeof(float));
             }
         }
-        std::vector<int32_t> tv_pieces(tv.pieces);
-        tv_pieces.insert(tv_pieces.end(), {0, 0, (int32_t)tv.n_entries(), -1});
+        const size_t n_pieces = tv.pieces.size() / 4, n_items = tv.chunks.size() / 4;
+        std::vector<int32_t> tv_pieces, tv_items, tv_dest;
+        if (tv.R == 1) {
+            // Each entry's record {value, B row | end of piece << 31}.
+            tv_dest.resize(n_pieces);
+            for (size_t q = 0; q < tv_brow.size(); ++q) {
+                const uint32_t br = tv_brow[q] == vcsr::kTileNoEntry ? (uint32_t)vcsr::kTileNoRow
+                                                                     : (uint32_t)tv_brow[q];
+                std::memcpy(&tv_val[2 * q + 1], &br, sizeof(float));
+            }
+            for (size_t p = 0; p < n_pieces; ++p) {
+                const int32_t* pc = &tv.pieces[4 * p];
+                const size_t end = p + 1 < n_pieces ? (size_t)pc[6] : tv_brow.size();
+                uint32_t br;
+                std::memcpy(&br, &tv_val[2 * end - 1], sizeof(float));
+                br |= 0x80000000u;
+                std::memcpy(&tv_val[2 * end - 1], &br, sizeof(float));
+                tv_dest[p] = pc[3] < 0 ? pc[0] : ~pc[3];
+            }
+            for (size_t c = 0; c < n_items; ++c)
+                tv_items.insert(tv_items.end(), {tv.chunks[4 * c], tv.chunks[4 * c + 2]});
+            tv_items.insert(tv_items.end(), {(int32_t)tv.n_entries(), (int32_t)n_pieces});
+        } else {
+            tv_pieces = tv.pieces;
+            tv_pieces.insert(tv_pieces.end(), {0, 0, (int32_t)tv.n_entries(), -1});
+        }
         DeviceFmt d;
         hip_check(hipGetDevice(&d.device), "hipGetDevice");
         try {
@@ -249,7 +273,9 @@ int vcsr_fmt_upload(vcsr_fmt* fmt, void* stream) {
             d.n_split = (int32_t)(rv.split_rows.size() / 3);
             d.n_partials = rv.n_partials;
             d.tv_R = tv.R;
-            d.tv_chunks = upload_array(tv.chunks, st, "upload tile chunks");
+            if (tv.R != 1) d.tv_chunks = upload_array(tv.chunks, st, "upload tile chunks");
+            d.tv_items = upload_array(tv_items, st, "upload tile items");
+            d.tv_dest = upload_array(tv_dest, st, "upload piece rows");
             d.tv_n_chunks = (int32_t)(tv.chunks.size() / 4);
             d.tv_pieces = upload_array(tv_pieces, st, "upload tile pieces");
             d.tv_n_pieces = (int32_t)(tv.pieces.size() / 4);
@@ -258,7 +284,7 @@ int vcsr_fmt_upload(vcsr_fmt* fmt, void* stream) {
                 d.tv_brow = upload_array(tv_brow, st, "upload tile entries");
             d.tv_val = upload_array(vcsr::tile_dev_folds_brow(tv.R) ? tv_val : tv.val, st,
                                     "upload tile values");
-            d.tv_mask = upload_array(tv.mask, st, "upload tile masks");
+            if (tv.R != 1) d.tv_mask = upload_array(tv.mask, st, "upload tile masks");
             d.tv_n_entries = tv.n_entries();
             d.tv_split = upload_array(tv.split, st, "upload split tiles");
             d.tv_n_split = (int32_t)(tv.split.size() / 4);
@@ -353,7 +379,7 @@ int spmm_vcsr_ex(const vcsr_fmt* fmt, const float* dB, int32_t O, int32_t tileK,
         // (out of device memory) is it allocated here, on the first call
         // that needs it, after waiting for the stream.
         const int64_t need = kernel == VCSR_KERNEL_TILE
-                                 ? vcsr::tile_partials_floats(fmt->v, d, dB, O, dC)
+                                 ? vcsr::tile_partials_floats(fmt->v, d, O)
                                  : kernel == VCSR_KERNEL_ROW ? vcsr::rowmajor_partials_floats(d, O)
                                                              : 0;
         if (need > d.partials_floats) {
@@ -399,7 +425,7 @@ int spmm_vcsr_noalloc(const vcsr_fmt* fmt, const float* dB, int32_t O, float* dC
         if (dev != d.device)
             throw vcsr::Error(VCSR_ESTATE, "format uploaded to another device than the current one");
         float* sp = scratch_on_current_device();
-        const int64_t need_floats = vcsr::tile_partials_floats(fmt->v, d, dB, O, dC);
+        const int64_t need_floats = vcsr::tile_partials_floats(fmt->v, d, O);
         if (need_floats > (int64_t)kScratchFloats)
             throw vcsr::Error(VCSR_ERANGE,
                               "split tiles need " + std::to_string(need_floats) +
@@ -431,9 +457,7 @@ int vcsr_launch_info_get(const vcsr_fmt* fmt, int32_t O, int32_t kernel, vcsr_la
         out->kernel = kernel == VCSR_KERNEL_AUTO ? VCSR_KERNEL_TILE : kernel;
         if (out->kernel != VCSR_KERNEL_TILE) return;
         const DeviceFmt& d = fmt->dev;
-        // As launched on 16-byte aligned B and C (device allocations are).
-        const float* aligned = reinterpret_cast<const float*>(uintptr_t(256));
-        const vcsr::TilePlan p = vcsr::tile_launch_plan(fmt->v, d, aligned, O, aligned);
+        const vcsr::TilePlan p = vcsr::tile_launch_plan(fmt->v, d, O);
         out->tile_rows = d.tv_R;
         out->tiles = fmt->tv_tiles;
         out->entries = d.tv_n_entries;

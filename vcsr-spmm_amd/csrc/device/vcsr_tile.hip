@@ -51,11 +51,7 @@
 #include "vecops.hpp"
 
 namespace vcsr {
-namespace {
 
-// Waves per block of the VALU tile kernel: 2 (1.5% faster than 4 on the
-// banded matrix — a freed wave slot waits less for a whole block to fit).
-constexpr int kWaves = 2;
 // Compute units of a device (256 on MI355X), read once per device.
 int device_cus(int device) {
     static std::atomic<int> cus[64];
@@ -70,389 +66,13 @@ int device_cus(int device) {
     return n;
 }
 
+namespace {
+
 // Column slices (launch_vcsr_tile): at most kTileWideCols columns per
 // launch, and kTileSliceCols when B is over twice the MALL's 256 MB.
 constexpr int32_t kTileWideCols = 256;
 constexpr int32_t kTileSliceCols = 128;
 constexpr uint64_t kTileSliceBytes = 512ull << 20;
-
-// Compile-time shape of the per-wave LDS of the single-row kernel.
-template <int VEC, int LPE, int MERGE>
-struct TileShape {
-    static constexpr int S = 64 / LPE;                          // streams per wave
-    static constexpr int EMAX = tile_piece_entries(1) * MERGE;  // entries per wave
-    static constexpr int PMAX = kTileChunkPieces * MERGE;       // pieces per wave
-    static constexpr int U = 8;                                 // loads per block
-    // A one-piece item's list is padded with "no row" entries of value 0 up
-    // to a multiple of S*UT, so that its blocks are full blocks of U loads
-    // per stream and at most one each of U/2, U/4.
-    static constexpr int UT = 2;
-    static constexpr int EPAD = (EMAX + S * U - 1) / (S * U) * (S * U);
-    // Several work items per wave: each stream takes an equal run of the
-    // wave's entries, cutting pieces where the runs meet (the piece's owner
-    // adds the other streams' partial sums after the loop).  Whole pieces per
-    // stream leave most streams idle behind a long row's piece: power-law
-    // 322K matrix, O = 8 / 32, 41% of the B-load slots busy against 84%, 37.1
-    // / 46.1 against 30.0 / 40.1 us.  A stream that ends a piece begun in an
-    // earlier run writes its partial sum to LDS at once (held in registers,
-    // the 16-byte-vector build kept it on the stack and ran 1.7x slower).
-    static constexpr bool EQ = MERGE > 1;
-};
-
-// One wave's LDS: staged entries (B-row byte offsets and values), the piece
-// table with its end sentinels, per-piece "not finite" flags and the streams'
-// first pieces.
-template <int VEC, int LPE, int MERGE>
-struct TileLds {
-    using Sh = TileShape<VEC, LPE, MERGE>;
-    __align__(16) float val[Sh::EPAD];
-    // Equal-run streams: per lane, the partial sum of the piece open at its
-    // stream's first entry, and per stream that piece (-1: none).
-    typename VecT<VEC>::T xs[Sh::EQ ? 64 : 1];
-    int32_t headp[Sh::EQ ? Sh::S : 1];
-    uint32_t brow[Sh::EPAD];
-    int4 piece[Sh::PMAX + 2];
-    int32_t first[Sh::S + 1];
-    uint8_t bad[Sh::PMAX];
-};
-
-// Work items c0 .. c1 (MERGE consecutive items of the view, fewer at the end)
-// on one wave.  BUF: B smaller than 2 GB, read with raw buffer loads at
-// 32-bit byte offsets; otherwise 64-bit addresses from B row indices
-// (LPE = 64 only).
-template <int VEC, int LPE, int MERGE, bool BUF>
-__device__ __forceinline__ void tile_item(
-    int32_t c0, int32_t c1, int lane, TileLds<VEC, LPE, MERGE>& L, int32_t O, int32_t ld,
-    int32_t accumulate, uint32_t b_bytes, const int4* __restrict__ chunks,
-    const int4* __restrict__ pieces, const uint16_t* __restrict__ ent_mask,
-    const float* __restrict__ ent_val, const float* __restrict__ B, float* __restrict__ C,
-    float* __restrict__ partials) {
-    using V = typename VecT<VEC>::T;
-    using Sh = TileShape<VEC, LPE, MERGE>;
-    constexpr int S = Sh::S;
-    constexpr int U = Sh::U;
-    constexpr int UT = Sh::UT;
-    // Off the buffer path placeholders read B row 0 times 0, which is NaN for
-    // an infinite b, so a piece's sum is checked and recomputed without them
-    // (the presence bits tell).  On the buffer path placeholders load zeros,
-    // so the sums are already the reference's (power-law 322K matrix, O = 8 /
-    // 32: 7% / 5% faster without the check at each piece end).
-    constexpr bool CHECK = !BUF;
-    uint32_t* lb = L.brow;
-    uint8_t* lbad = L.bad;
-    float* lv = L.val;
-    int4* lp = L.piece;
-    int32_t* lf = L.first;
-    const int32_t e0 = uniform(chunks[c0].x), ne = uniform(chunks[c1].y) - e0;  // <= EMAX
-    const int32_t p0 = uniform(chunks[c0].z), np = uniform(chunks[c1].w) - p0;  // <= PMAX
-
-    // Phase 1: stage the entries (and a one-piece item's padding, buffer
-    // path) and the piece table.
-    const uint32_t row_bytes = (uint32_t)ld * 4u;
-    const bool pad = BUF && np == 1;
-    const int32_t ne_pad = pad ? (ne + S * UT - 1) / (S * UT) * (S * UT) : ne;  // <= EPAD
-    for (int32_t i = lane; i < ne_pad; i += 64) {
-        uint32_t br = (uint32_t)kTileNoEntry;
-        float a = 0.f;
-        if (i < ne) {
-            // One load: the value, then the B row's bits.
-            const float2 rec = *reinterpret_cast<const float2*>(ent_val + 2 * ((int64_t)e0 + i));
-            a = rec.x;
-            br = __builtin_bit_cast(uint32_t, rec.y);
-        }
-        // Placeholders: "no row" on the buffer path, else row 0 times 0.
-        const bool real = br != (uint32_t)kTileNoEntry;
-        const uint32_t off = BUF ? (real ? br * row_bytes : kNoRow) : (real ? br : 0u);
-        lb[i] = off;
-        lv[i] = a;
-    }
-    if (np > 1) {
-        for (int32_t j = lane; j < np; j += 64) {
-            int4 pc = pieces[p0 + j];
-            pc.z -= e0;
-            lp[j] = pc;
-            lbad[j] = 0;
-        }
-        if (lane < 2) lp[np + lane] = make_int4(0, 0, ne, -1);  // end sentinels
-    }
-    wave_sync();
-
-    const __amdgpu_buffer_rsrc_t rsrc =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), (short)0, (int)b_bytes,
-                                          kRawBufferFlags);
-    const int sub = lane / LPE, kl = lane % LPE;
-
-    // One entry's B slice; zeros for "no row" (placeholders, lanes past the
-    // end) on the buffer path.  The offset is read for every lane (tc is a
-    // valid index) and lanes past the end get the "no row" bit ORed in, so
-    // the tail blocks issue their loads back to back like the full ones (a
-    // conditional read becomes a branch and an LDS wait per load).
-    auto load_b = [&](int32_t tc, bool ok, uint32_t koff) -> V {
-        if constexpr (BUF) {
-            const uint32_t off = (lb[tc] + koff) | (ok ? 0u : kNoRow);
-            return load_b_buf<VEC>(rsrc, off);
-        } else {
-            const V b = *reinterpret_cast<const V*>(B + (int64_t)lb[tc] * ld + koff / 4);
-            return ok ? b : zero_vec(V());
-        }
-    };
-    auto apply = [&](V& acc, int32_t tc, bool ok, const V& b) {
-        const float a = lv[tc];
-        fma_vec(acc, ok ? a : 0.f, b);
-    };
-    // Whether this lane's sums are finite (lanes past O hold nothing to
-    // store): fma(x, 0, z) over them stays finite exactly when every x is.
-    auto piece_finite = [&](const V& acc, bool kok) -> bool {
-        return __builtin_isfinite(fma_zero_acc(acc, 0.f)) || !kok;
-    };
-    // Writes the sums of row `row` to C, or to partial row `part` if that is
-    // not negative.
-    auto store_row = [&](int32_t row, int32_t part, const V& acc, int32_t k, bool kok) {
-        if (!kok) return;
-        if (part < 0) {
-            V* dst = reinterpret_cast<V*>(C + (int64_t)row * ld + k);
-            store_nt(dst, accumulate ? add_vec(*dst, acc) : acc);
-        } else {
-            *reinterpret_cast<V*>(partials + (int64_t)part * O + k) = acc;
-        }
-    };
-    // Recomputation of piece pc (entries tb .. te-1) in entry order without
-    // its placeholders (taken only for pieces whose sum is not finite, which
-    // were not stored).
-    auto redo_piece = [&](const int4 pc, int32_t tb, int32_t te, int32_t k, uint32_t koff,
-                          bool kok) {
-        V acc = zero_vec(V());
-        for (int32_t t = tb; t < te; ++t) {
-            const V b = load_b(t, true, koff);
-            if (ent_mask[(int64_t)e0 + t] & 1u) fma_vec(acc, lv[t], b);
-        }
-        if (pc.y > 0) store_row(pc.x, pc.w, acc, k, kok);
-    };
-
-    if (np > 1) {
-        int32_t pa, pb, tb, te;  // this stream's pieces and entries
-        if constexpr (Sh::EQ) {
-            // Entries tb .. te-1, and pa the piece holding entry tb (the
-            // last piece starting at or before it; pieces are not empty).
-            tb = (sub * ne) / S;
-            te = ((sub + 1) * ne) / S;
-            int32_t lo = 0, hi = np - 1;
-            while (lo < hi) {
-                const int32_t mid = (lo + hi + 1) >> 1;
-                if (lp[mid].z <= tb) lo = mid;
-                else hi = mid - 1;
-            }
-            pa = lo;
-            pb = pa;  // set after the loop: the first piece not completed
-        } else {
-            // Stream s takes the pieces whose entry midpoint falls in the s-th
-            // S-quantile of the item: first piece lf[s], end piece lf[s + 1].
-            if (lane <= S) {
-                int32_t lo = 0, hi = np;
-                while (lo < hi) {
-                    const int32_t mid = (lo + hi) >> 1;
-                    const int32_t sm = ((lp[mid].z + lp[mid + 1].z) * S) / (2 * ne);
-                    if (sm < lane) lo = mid + 1;
-                    else hi = mid;
-                }
-                lf[lane] = lo;
-            }
-            wave_sync();
-            pa = lf[sub];
-            pb = lf[sub + 1];
-            tb = lp[pa].z;
-            te = lp[pb].z;
-        }
-        // Equal runs: piece pa began in an earlier stream's run; this stream
-        // only contributes a partial sum to it.
-        const bool carry = Sh::EQ && lp[pa].z < tb;
-        // Lanes of this lane's stream, for ballots.
-        const uint64_t smask =
-            LPE == 64 ? ~0ull : (((1ull << (LPE & 63)) - 1ull) << ((sub * LPE) & 63));
-        int32_t nmax = te - tb, nmin = te - tb;
-#pragma unroll
-        for (int sh = LPE; sh < 64; sh <<= 1) {
-            nmax = max(nmax, __shfl_xor(nmax, sh));
-            nmin = min(nmin, __shfl_xor(nmin, sh));
-        }
-        nmax = uniform(nmax);
-        nmin = uniform(nmin);
-        for (int32_t k0 = 0; k0 < O; k0 += LPE * VEC) {
-            const int32_t k = k0 + kl * VEC;
-            const bool kok = k < O;
-            const uint32_t koff = (uint32_t)((kok || BUF) ? k : 0) * 4u;
-            V acc = zero_vec(V());
-            int32_t p = pa, pend = lp[pa + 1].z;
-            // Without the finiteness check, the row and partial row of piece
-            // p are read when the piece starts, so its store waits on no LDS
-            // read (power-law 322K matrix, O = 8 / 32 / 128: 2% / 3% / 0.6%).
-            int32_t cur_x = lp[pa].x, cur_w = lp[pa].w;
-            bool bad = false;
-            auto block = [&](auto full_c, int32_t i0) {
-                constexpr bool FULL = decltype(full_c)::value;
-                V b[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int32_t t = tb + i0 + u;
-                    const bool ok = FULL || t < te;
-                    b[u] = load_b(ok ? t : 0, ok, koff);
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int32_t t = tb + i0 + u;
-                    const bool ok = FULL || t < te;
-                    apply(acc, ok ? t : 0, ok, b[u]);
-                    if (ok && t + 1 == pend) {
-                        if (carry && p == pa) {
-                            // The end of a piece begun in an earlier run: its
-                            // owner adds this partial sum after the loop.
-                            L.xs[lane] = acc;
-                        } else if constexpr (CHECK) {
-                            // A stream stores a piece only if all its lanes'
-                            // sums are finite; otherwise redo_piece computes
-                            // and stores it after the loop.
-                            const uint64_t bm = __ballot(!piece_finite(acc, kok));
-                            if ((bm & smask) != 0) {
-                                bad = true;
-                                lbad[p] = 1;
-                            } else {
-                                store_row(lp[p].x, lp[p].w, acc, k, kok);
-                            }
-                        } else {
-                            store_row(cur_x, cur_w, acc, k, kok);
-                        }
-                        acc = zero_vec(V());
-                        ++p;
-                        pend = lp[p + 1].z;
-                        if constexpr (!CHECK) {
-                            cur_x = lp[p].x;
-                            cur_w = lp[p].w;
-                        }
-                    }
-                }
-            };
-            for (int32_t i0 = 0; i0 < nmax; i0 += U) {
-                if (i0 + U <= nmin) block(std::true_type(), i0);
-                else block(std::false_type(), i0);
-            }
-            if constexpr (Sh::EQ) {
-                // Piece p is still open at the end of the run when it began
-                // before te.  If it is piece pa begun in an earlier run, the
-                // whole run was a middle part of it; otherwise this stream
-                // owns it and adds the following runs' partial sums (each
-                // stream's first piece and its sum up to that piece's end or
-                // its run's) in stream order.
-                pb = p;
-                const bool open = lp[p].z < te || (te == tb && carry);
-                const bool middle = open && carry && p == pa;
-                if (middle) L.xs[lane] = acc;
-                if (kl == 0) L.headp[sub] = carry ? pa : -1;
-                wave_sync();
-                if (open && !middle) {
-                    for (int32_t s2 = sub + 1; s2 < S && L.headp[s2] == p; ++s2)
-                        acc = add_vec(acc, L.xs[s2 * LPE + kl]);
-                    if constexpr (CHECK) {
-                        const uint64_t bm = __ballot(!piece_finite(acc, kok));
-                        if ((bm & smask) != 0) redo_piece(lp[p], lp[p].z, lp[p + 1].z, k, koff, kok);
-                        else store_row(lp[p].x, lp[p].w, acc, k, kok);
-                    } else {
-                        store_row(lp[p].x, lp[p].w, acc, k, kok);
-                    }
-                }
-                wave_sync();
-            }
-            if (__any(bad)) {
-                wave_sync();
-                for (int32_t q = pa; q < pb; ++q)
-                    if (lbad[q]) redo_piece(lp[q], lp[q].z, lp[q + 1].z, k, koff, kok);
-                wave_sync();
-                for (int32_t q = pa; q < pb; ++q) lbad[q] = 0;
-                wave_sync();
-            }
-        }
-    } else {
-        // One piece: entries t = sub + S*i, summed across streams at the end.
-        // Its record is wave-uniform (scalar loads; no LDS table).
-        const int4 pc1 = make_int4(uniform(pieces[p0].x), uniform(pieces[p0].y),
-                                   uniform(pieces[p0].z) - e0, uniform(pieces[p0].w));
-        const int32_t nper = (ne + S - 1) / S, nfull = ne / S;
-        for (int32_t k0 = 0; k0 < O; k0 += LPE * VEC) {
-            const int32_t k = k0 + kl * VEC;
-            const bool kok = k < O;
-            const uint32_t koff = (uint32_t)((kok || BUF) ? k : 0) * 4u;
-            V acc = zero_vec(V());
-            auto block = [&](auto full_c, int32_t i0) {
-                constexpr bool FULL = decltype(full_c)::value;
-                V b[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int32_t t = sub + S * (i0 + u);
-                    const bool ok = FULL || t < ne;
-                    b[u] = load_b(ok ? t : 0, ok, koff);
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int32_t t = sub + S * (i0 + u);
-                    const bool ok = FULL || t < ne;
-                    apply(acc, ok ? t : 0, ok, b[u]);
-                }
-            };
-            if constexpr (BUF) {
-                // Full blocks of U loads per stream, then one of UT if the
-                // padded list has that many left.
-                auto block_n = [&](auto nu_c, int32_t i0) {
-                    constexpr int NU = decltype(nu_c)::value;
-                    V b[NU];
-#pragma unroll
-                    for (int u = 0; u < NU; ++u) b[u] = load_b(sub + S * (i0 + u), true, koff);
-#pragma unroll
-                    for (int u = 0; u < NU; ++u) apply(acc, sub + S * (i0 + u), true, b[u]);
-                };
-                const int32_t nper_pad = ne_pad / S;
-                int32_t i0 = 0;
-                for (; i0 + U <= nper_pad; i0 += U) block_n(std::integral_constant<int, U>(), i0);
-                if (i0 + U / 2 <= nper_pad) {
-                    block_n(std::integral_constant<int, U / 2>(), i0);
-                    i0 += U / 2;
-                }
-                if (i0 + U / 4 <= nper_pad) block_n(std::integral_constant<int, U / 4>(), i0);
-            } else {
-                for (int32_t i0 = 0; i0 < nper; i0 += U) {
-                    if (i0 + U <= nfull) block(std::true_type(), i0);
-                    else block(std::false_type(), i0);
-                }
-            }
-#pragma unroll
-            for (int sh = LPE; sh < 64; sh <<= 1) acc = add_vec(acc, shfl_xor_vec(acc, sh));
-            if (CHECK && __any(!piece_finite(acc, kok))) {
-                if (sub == 0) redo_piece(pc1, pc1.z, ne, k, koff, kok);
-            } else if (sub == 0 && pc1.y > 0) {
-                store_row(pc1.x, pc1.w, acc, k, kok);
-            }
-        }
-    }
-}
-
-// One wave per MERGE consecutive work items of the view.
-template <int VEC, int LPE, int MERGE, bool BUF>
-__global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(MERGE == 1 ? 5 : 1, 8)))
-void vcsr_tile_kernel(
-    int32_t n_chunks, int32_t O, int32_t ld, int32_t accumulate, uint32_t b_bytes,
-    const int4* __restrict__ chunks, const int4* __restrict__ pieces,
-    const uint16_t* __restrict__ ent_mask, const float* __restrict__ ent_val,
-    const float* __restrict__ B, float* __restrict__ C, float* __restrict__ partials) {
-    __shared__ TileLds<VEC, LPE, MERGE> s_lds[kWaves];
-    // Wave-uniform indices, so the work-item records are scalar loads.
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int lane = (int)(threadIdx.x & 63);
-    const int32_t w = (int32_t)(xcd_remap(blockIdx.x, gridDim.x) * kWaves) + wave;
-    const int32_t c0 = w * MERGE;
-    if (c0 >= n_chunks) return;
-    tile_item<VEC, LPE, MERGE, BUF>(c0, min(n_chunks, c0 + MERGE) - 1, lane, s_lds[wave], O, ld,
-                                       accumulate, b_bytes, chunks, pieces, ent_mask,
-                                       ent_val, B, C, partials);
-}
 
 // Adds the piece partials of the rows of split tiles into C.  split: {row,
 // first partial row, stride, pieces}, in decreasing piece count.  Lanes
@@ -780,40 +400,6 @@ hipError_t launch_mma(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t
     return hipGetLastError();
 }
 
-template <int VEC, int LPE, bool BUF>
-hipError_t launch_one(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
-                      int32_t accumulate, uint32_t b_bytes, float* partials, hipStream_t st) {
-    // Eight streams per wave: four work items per wave, so that each stream
-    // still gets several rows.
-    constexpr int MERGE = 64 / LPE >= 8 ? 4 : 1;
-    const int64_t waves = ((int64_t)d.tv_n_chunks + MERGE - 1) / MERGE;
-    const dim3 grid((unsigned)((waves + kWaves - 1) / kWaves)), block(64 * kWaves);
-    hipLaunchKernelGGL((vcsr_tile_kernel<VEC, LPE, MERGE, BUF>), grid, block, 0, st, d.tv_n_chunks, O,
-                       ld, accumulate, b_bytes, reinterpret_cast<const int4*>(d.tv_chunks),
-                       reinterpret_cast<const int4*>(d.tv_pieces), d.tv_mask, d.tv_val, B, C,
-                       partials);
-    return hipGetLastError();
-}
-
-template <int VEC>
-hipError_t launch_r(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
-                    int32_t accumulate, uint64_t b_bytes, float* partials, hipStream_t st) {
-    if (b_bytes + 64u * 4u * (uint64_t)VEC >= kBufferLimit)
-        return launch_one<VEC, 64, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
-    const uint32_t bb = (uint32_t)b_bytes;
-    // Lanes per entry: the smallest power of two covering O, at least 8 (at
-    // most 8 streams per wave, so every stream gets several tiles); 8 lanes
-    // occur for VEC = 4 (O = 32) and VEC = 1 (O <= 8).
-    const int32_t need = (O + VEC - 1) / VEC;
-    if constexpr (VEC == 1 || VEC == 4) {
-        if (need <= 8)
-            return launch_one<VEC, 8, true>(d, B, O, ld, C, accumulate, bb, partials, st);
-    }
-    if (need <= 16) return launch_one<VEC, 16, true>(d, B, O, ld, C, accumulate, bb, partials, st);
-    if (need <= 32) return launch_one<VEC, 32, true>(d, B, O, ld, C, accumulate, bb, partials, st);
-    return launch_one<VEC, 64, true>(d, B, O, ld, C, accumulate, bb, partials, st);
-}
-
 // Columns [0, O) of B and C, whose rows are ld floats apart (B and C point
 // at the first column; ld > O for one column slice of wider matrices).
 template <int VEC>
@@ -824,7 +410,9 @@ hipError_t launch_vec(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t
         const uint64_t b_bytes = v.N > 0 ? ((uint64_t)(v.N - 1) * (uint64_t)ld + (uint64_t)O) * 4u : 0u;
         hipError_t e;
         switch (d.tv_R) {
-            case 1: e = launch_r<VEC>(d, B, O, ld, C, accumulate, b_bytes, partials, st); break;
+            case 1:
+                e = launch_vcsr_row_tiles(d, B, O, ld, C, accumulate, b_bytes, partials, st);
+                break;
             case 2:
             case 3:
             case 4:
@@ -877,87 +465,64 @@ static int tile_mma_vec(const DeviceFmt& d, int32_t w) {
     return vec;
 }
 
-// Floats per lane of tiles of 2 to 8 rows for w columns of any alignment
-// (the shapes of vcsr_tile_tall.hip); the reduce of their partial rows takes
-// the same.
-static int tile_tall_vec(int32_t R, int32_t w) { return w > 32 || (w > 16 && R < 4) ? 4 : 1; }
+// Floats per lane of tiles of 1 to 8 rows for w columns of any alignment (the
+// shapes of vcsr_tile_row.hip and vcsr_tile_tall.hip); the reduce of their
+// partial rows takes the same.
+static int tile_valu_vec(int32_t R, int32_t w) { return w > 32 || (w > 16 && R < 4) ? 4 : 1; }
 
-// Floats per lane and B slice of single-row tiles: 4 when O allows 8 lanes of
-// 16-byte vectors and B and C are 16-byte aligned, else 2 or 1.  At O = 32,
-// 4 floats per lane measured 3% / 8% faster than 2 on the banded /
-// power-law matrices.
-static int tile_vec(int32_t O, bool a16, bool a8) {
-    if (O % 4 == 0 && a16 && O >= 32) return 4;
-    if (O % 2 == 0 && a8 && O >= 32) return 2;
-    return 1;
+static int tile_vec(const DeviceFmt& d, int32_t w) {
+    return d.tv_R == kTileMmaRows ? tile_mma_vec(d, w) : tile_valu_vec(d.tv_R, w);
 }
 
-// Floats per lane (tile_vec) and column-slice width of a launch over B and
-// C of width O.  Tiles of 1 to 8 rows with 16-byte vectors: one launch per
-// column slice of at most 256 columns (one column tile of a wave), or 128
-// when B is over 512 MB, so that the B bytes live at a time stay small.
+// Column-slice width of a launch over B and C of width O.  Tiles of 1 to 8
+// rows: one launch per column slice of at most 256 columns (one column tile
+// of a wave), or 128 when B is over 512 MB, so that the B bytes live at a
+// time stay small.
 // Measured against one launch over all columns: banded 62K matrix, slices of
 // 256, O = 512 / 1024 / 2048: same / 16% / 30% faster; slices of 128,
 // uniform-random 1M matrix O = 256 (1 GB): 11% faster, power-law 322K
 // matrix O = 512 (659 MB): 3% faster, O = 256 (330 MB): 3% slower.
-struct TileSlicing {
-    int vec;
-    int32_t width;
-};
-static TileSlicing tile_slicing(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t O,
-                                const float* C) {
-    const bool a16 = (((uintptr_t)B | (uintptr_t)C) & 15u) == 0;
-    const bool a8 = (((uintptr_t)B | (uintptr_t)C) & 7u) == 0;
-    // Narrow B: narrower per-lane vectors give streams of at least 8-16
-    // lanes, so fewer streams share a tile's entries (measured at O = 8:
-    // 4-byte loads with 8 streams 1.3x faster than 16-byte loads with 32).
-    TileSlicing ts{tile_vec(O, a16, a8), O};
-    if (d.tv_R == kTileMmaRows) {
-        ts.vec = tile_mma_vec(d, d.tv_partial_rows > 0 ? std::min(O, kTileWideCols) : O);
-    } else if (ts.vec == 4 || d.tv_R > 1) {
-        if (d.tv_R > 1) ts.vec = tile_tall_vec(d.tv_R, O);
-        if ((uint64_t)v.N * (uint64_t)O * 4u > kTileSliceBytes) ts.width = std::min(O, kTileSliceCols);
-        else ts.width = std::min(O, kTileWideCols);
-    }
+static int32_t tile_slice_width(const Vcsr& v, const DeviceFmt& d, int32_t O) {
+    int32_t width = O;
+    if (d.tv_R != kTileMmaRows)
+        width = std::min(O, (uint64_t)v.N * (uint64_t)O * 4u > kTileSliceBytes ? kTileSliceCols
+                                                                               : kTileWideCols);
     // Split tiles write partial rows one slice wide: whatever the tile
-    // height and vector width, a launch then covers at most the 256 columns
-    // the upload sizes the partial rows for, so no O needs more scratch.
-    if (d.tv_partial_rows > 0) ts.width = std::min(ts.width, kTileWideCols);
-    return ts;
+    // height, a launch then covers at most the 256 columns the upload sizes
+    // the partial rows for, so no O needs more scratch.
+    if (d.tv_partial_rows > 0) width = std::min(width, kTileWideCols);
+    return width;
 }
 
-int64_t tile_partials_floats(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t O,
-                             const float* C) {
+int64_t tile_partials_floats(const Vcsr& v, const DeviceFmt& d, int32_t O) {
     if (O <= 0 || v.M == 0 || d.tv_partial_rows == 0) return 0;
-    return (int64_t)d.tv_partial_rows * tile_slicing(v, d, B, O, C).width;
+    return (int64_t)d.tv_partial_rows * tile_slice_width(v, d, O);
 }
 
 int64_t tile_partials_upload_floats(const DeviceFmt& d) {
     return (int64_t)d.tv_partial_rows * kTileWideCols;
 }
 
-TilePlan tile_launch_plan(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t O,
-                          const float* C) {
+TilePlan tile_launch_plan(const Vcsr& v, const DeviceFmt& d, int32_t O) {
     TilePlan p;
     if (O <= 0 || v.M == 0) return p;
-    const TileSlicing ts = tile_slicing(v, d, B, O, C);
-    p.vec = ts.vec;
-    p.slice_cols = ts.width;
-    p.slices = (O + ts.width - 1) / ts.width;
+    p.slice_cols = tile_slice_width(v, d, O);
+    p.vec = tile_vec(d, p.slice_cols);
+    p.slices = (O + p.slice_cols - 1) / p.slice_cols;
     p.matrix_cores = d.tv_R == kTileMmaRows && d.tv_n_chunks > 0;
     p.reduce_launches = d.tv_n_split > 0 ? p.slices : 0;
-    p.partial_floats = tile_partials_floats(v, d, B, O, C);
+    p.partial_floats = tile_partials_floats(v, d, O);
     return p;
 }
 
 hipError_t launch_vcsr_tile(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t O,
                             float* C, int32_t accumulate, float* partials, hipStream_t st) {
     if (O <= 0 || v.M == 0) return hipSuccess;
-    const TileSlicing ts = tile_slicing(v, d, B, O, C);
-    for (int32_t c0 = 0; c0 < O; c0 += ts.width) {
-        const int32_t w = std::min(ts.width, O - c0);
+    const int32_t width = tile_slice_width(v, d, O);
+    for (int32_t c0 = 0; c0 < O; c0 += width) {
+        const int32_t w = std::min(width, O - c0);
         hipError_t e;
-        switch (d.tv_R == kTileMmaRows ? tile_mma_vec(d, w) : d.tv_R > 1 ? tile_tall_vec(d.tv_R, w) : ts.vec) {
+        switch (tile_vec(d, w)) {
             case 4: e = launch_vec<4>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;
             case 2: e = launch_vec<2>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;
             default: e = launch_vec<1>(v, d, B + c0, w, O, C + c0, accumulate, partials, st); break;

@@ -63,11 +63,11 @@ struct TallLds {
     uint32_t off[Sh::REC ? 1 : Sh::G][Sh::REC ? 1 : Sh::SEG + (Sh::G > 1 ? S : 0)];
 };
 
-template <int VEC, int LPE, int S, int R, int U, bool BUF>
+template <int VEC, int LPE, int S, int R, int U, bool BUF, bool ACC>
 __global__ __launch_bounds__(64 * kWaves)
 __attribute__((amdgpu_waves_per_eu(R <= 3 ? 5 : 1, 8)))
 void vcsr_tall_kernel(
-    int32_t n_pieces, int32_t O, int32_t ld, int32_t accumulate, uint32_t b_bytes,
+    int32_t n_pieces, int32_t O, int32_t ld, uint32_t b_bytes,
     const int4* __restrict__ pieces, const int32_t* __restrict__ ent_brow,
     const uint16_t* __restrict__ ent_mask, const float* __restrict__ ent_val,
     const float* __restrict__ B, float* __restrict__ C, float* __restrict__ partials) {
@@ -121,6 +121,19 @@ void vcsr_tall_kernel(
         if constexpr (BUF) return load_b_buf<VEC>(rsrc, off + koff);
         else return load_mem(B + (int64_t)off * ld + koff / 4, V());
     };
+
+    // C += A*B: this stream's rows of C are read ahead of everything else.
+    constexpr int CR = (R + S - 1) / S;
+    V c[ACC ? CR : 1];
+    if constexpr (ACC) {
+#pragma unroll
+        for (int i = 0; i < CR; ++i) {
+            const int r = i * S + sub;
+            c[i] = r < pc.y && pc.w < 0
+                       ? load_mem(C + (int64_t)(pc.x + r) * ld + vec_col<VEC>(k, O), V())
+                       : zero_vec(V());
+        }
+    }
 
     V acc[R];
 #pragma unroll
@@ -246,15 +259,16 @@ void vcsr_tall_kernel(
     }
     if (!kok) return;
 #pragma unroll
-    for (int i = 0; i < (R + S - 1) / S; ++i) {
+    for (int i = 0; i < CR; ++i) {
         const int r = i * S + sub;
         if (r < R && r < pc.y) {
             V x = acc[0];
 #pragma unroll
             for (int q = 1; q < R; ++q)
                 if (q == r) x = acc[q];
+            if constexpr (ACC) x = add_vec(c[i], x);
             if (pc.w < 0)
-                store_cols<VEC, true>(C + (int64_t)(pc.x + r) * ld, k, O, x, accumulate);
+                store_cols<VEC, true>(C + (int64_t)(pc.x + r) * ld, k, O, x, false);
             else
                 store_cols<VEC, false>(partials + (int64_t)(pc.w + r) * O, k, O, x, false);
         }
@@ -266,10 +280,14 @@ hipError_t launch_shape(const DeviceFmt& d, const float* B, int32_t O, int32_t l
                         int32_t accumulate, uint32_t b_bytes, float* partials, hipStream_t st) {
     constexpr int per = TallShape<LPE, S, R, U>::G * kWaves;
     const dim3 grid((unsigned)(((int64_t)d.tv_n_pieces + per - 1) / per)), block(64 * kWaves);
-    hipLaunchKernelGGL((vcsr_tall_kernel<VEC, LPE, S, R, U, BUF>), grid, block, 0, st, d.tv_n_pieces, O,
-                       ld, accumulate, b_bytes, reinterpret_cast<const int4*>(d.tv_pieces),
-                       d.tv_brow, d.tv_mask, d.tv_val, B, C, partials);
-    return hipGetLastError();
+    auto go = [&](auto acc) {
+        hipLaunchKernelGGL((vcsr_tall_kernel<VEC, LPE, S, R, U, BUF, decltype(acc)::value>), grid,
+                           block, 0, st, d.tv_n_pieces, O, ld, b_bytes,
+                           reinterpret_cast<const int4*>(d.tv_pieces), d.tv_brow, d.tv_mask,
+                           d.tv_val, B, C, partials);
+        return hipGetLastError();
+    };
+    return accumulate ? go(std::true_type()) : go(std::false_type());
 }
 
 template <int X>

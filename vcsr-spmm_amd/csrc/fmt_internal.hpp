@@ -44,11 +44,18 @@ struct DeviceFmt {
     int32_t* tv_pieces = nullptr;       // 4 per piece: row, rows, first entry, partial row;
                                         // then one whose first entry is the entry count
     int32_t tv_n_pieces = 0;
+    // Single-row tiles: instead of the work items and pieces above, 2 ints
+    // per work item (first entry, first piece; and one past the last), and
+    // per piece its row, or ~partial row.
+    int32_t* tv_items = nullptr;
+    int32_t* tv_dest = nullptr;
     int32_t* tv_brow = nullptr;         // per entry: B row, kTileNoEntry for placeholders
                                         // (not uploaded for 1- and 3-row tiles)
     float* tv_val = nullptr;            // tile_dev_stride per entry: values (0 where absent),
-                                        // then the B row's bits for 1- and 3-row tiles
-    uint16_t* tv_mask = nullptr;        // per entry: presence bit per tile row
+                                        // then the B row's bits for 1- and 3-row tiles (for 1:
+                                        // 31 bits, and whether the entry ends its piece)
+    uint16_t* tv_mask = nullptr;        // per entry: presence bit per tile row (not uploaded
+                                        // for single-row tiles)
     int64_t tv_n_entries = 0;
     int32_t* tv_split = nullptr;        // 4*tv_n_split: row, partial row, stride, pieces
     int32_t tv_n_split = 0;

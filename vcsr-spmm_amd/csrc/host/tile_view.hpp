@@ -66,6 +66,9 @@ constexpr int32_t kTileChunkPieces = 32;
 // B row of a placeholder entry (no tile row present) in the device copy of
 // the view's B-row array; the host view keeps 0 there.
 constexpr int32_t kTileNoEntry = -1;
+// The device records of single-row tiles keep the B row in 31 bits (the top
+// bit marks the last entry of a piece); this one is a placeholder's.
+constexpr int32_t kTileNoRow = 0x7fffffff;
 // The device copy of the values of 1- and 3-row tiles also holds each
 // entry's B row (kTileNoEntry for placeholders), as the bits of one more
 // float after its values — for 3 rows in the padding slot of the stride —
