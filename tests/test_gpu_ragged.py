@@ -172,3 +172,36 @@ def test_row_tiles_nonfinite_b(gpu, orc, st, O):
     assert np.array_equal(np.isinf(got), np.isinf(ref))
     fin = np.isfinite(ref)
     assert np.allclose(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("O", [1, 8, 9, 16, 17, 31, 33, 50, 64, 65, 100, 128, 130, 257, 300])
+def test_csr_wave_long_rows_are_bit_exact(gpu, orc, st, O, off):
+    """The plain-CSR kernel on rows around its long-row limit (128 entries)
+    and around whole turns of it, empty rows and columns outside [0, N)
+    (which contribute nothing): bit for bit the oracle's FP32 loop."""
+    vs = gpu
+    rng = np.random.default_rng(O)
+    N = 2000
+    lens = [0, 1, 127, 128, 129, 136, 0, 159, 160, 161, 1700, 3] + [5] * 40 + [257, 300, 1] * 9
+    rows = np.repeat(np.arange(len(lens)), lens)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    col = rng.integers(0, N, rows.size).astype(np.int32)
+    val = rng.standard_normal(rows.size).astype(np.float32)
+    B = vs.gen_dense(O, 0, N, O)
+    ref = orc.spmm_f32(len(lens), rp, col, val, B)
+
+    def run(rp, col, val):
+        d = [vs.DeviceArray.from_numpy(x, st) for x in (rp, col, val)]
+        dB = _Shifted(vs, B, off, st)
+        dC = _Shifted(vs, np.full((len(lens), O), 5.0, np.float32), off, st)
+        vs.run_csr_wave_spmm_gpu(len(lens), N, *d, dB, O, dC, st, timed=True)
+        return dC.numpy()
+
+    assert np.array_equal(run(rp, col, val).view(np.uint32), ref.view(np.uint32))
+    bad = rng.random(rows.size) < 0.1
+    outside = np.where(bad, np.where(rng.random(rows.size) < 0.5, -1, N), col).astype(np.int32)
+    keep = ~bad
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=len(lens)))])
+    ref = orc.spmm_f32(len(lens), rp2.astype(np.int32), col[keep], val[keep], B)
+    assert np.array_equal(run(rp, outside, val).view(np.uint32), ref.view(np.uint32))

@@ -5,13 +5,29 @@
 // C in registers, and C is written once (C = A*B).  No format build.
 //
 // gfx950 form: a row is a stream of LPE lanes holding VEC consecutive
-// columns each (16-byte B loads when O allows), so a wave computes
-// S = 64/LPE rows at once; the reference's warp computes one row per
-// 64-column chunk with 4-byte loads and needs O % 64 == 0, this kernel takes
-// any O.  A stream stages LPE of its row's entries at a time (B-row byte
-// offset and value) in the wave's LDS and applies them in blocks of U loads
-// issued back to back; B is read with raw buffer loads whose range check
-// returns zeros for lanes past the row's end or past O.
+// columns each, so a wave computes S = 64/LPE rows at once; the reference's
+// warp computes one row per 64-column chunk with 4-byte loads and needs
+// O % 64 == 0, this kernel takes any O and any alignment.  Every column of C
+// is one chain of fused multiply-adds in the row's entry order (the CPU
+// loop's bits), so a row's entries cannot be split between lanes.
+//  - Rows of up to kLongRow entries: a stream stages CH of its row's entries
+//    at a time (B-row byte offset and value) in the wave's LDS, the next
+//    ones' loads in flight meanwhile, and applies them in blocks of U loads
+//    issued back to back; B is read with raw buffer loads whose range check
+//    returns zeros for lanes past the row's end or past O.
+//  - Longer rows bound the kernel by their own latency (8 loads in flight a
+//    stream), so the block's four waves take them together afterwards: the
+//    waves take turns of LU entries each, all of a turn's B rows loaded ahead
+//    while the other waves have their turns, and hand the running sums on
+//    through LDS.
+// us per SpMM, three matrices in turn, before the long rows' turns, the
+// entries' prefetch and the 16-byte lanes at any width, and now: power-law
+// 100K rows (longest 1.7K), O = 8 / 47 / 64 138 / 119 / 141 -> 33 / 37 / 37;
+// 322K (5.2K), O = 128 528 -> 206; banded 62K, O = 8 / 47 24.8 / 58.9 -> 14.8 /
+// 38.6; 9 16x16 blocks a row, O = 66 31.9 -> 20.7; uniform 1M x 16, O = 256
+// 2,733 -> 2,722.
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 #include "vecops.hpp"
@@ -19,11 +35,21 @@
 namespace vcsr {
 namespace {
 
+// Waves per block: 4 (with 8, power-law 100K, O = 64 52 against 37 us).
 constexpr int kWaveRowsWaves = 4;
-constexpr uint32_t kNoCol = 0x80000000u;  // buffer offset past any B on the buffer path
+// 64 instead of 128 changes nothing measurable.
+constexpr int32_t kLongRow = 128;
+
+// Long rows: columns per lane (64 lanes a row) and entries per turn: 32
+// loads of 4 bytes a lane in flight (64: the same times, 16: 10% slower).
+template <int VEC, int LPE>
+struct LongShape {
+    static constexpr int LV = VEC * LPE <= 64 ? 1 : VEC * LPE <= 128 ? 2 : 4;
+    static constexpr int LU = 32 / LV;
+};
 
 template <int VEC, int LPE, bool BUF>
-__global__ __launch_bounds__(256) void csr_wave_kernel(int32_t M, int32_t N, int32_t O,
+__global__ __launch_bounds__(64 * kWaveRowsWaves) void csr_wave_kernel(int32_t M, int32_t N, int32_t O,
                                                        uint32_t b_bytes,
                                                        const int32_t* __restrict__ rowptr,
                                                        const int32_t* __restrict__ col,
@@ -31,83 +57,172 @@ __global__ __launch_bounds__(256) void csr_wave_kernel(int32_t M, int32_t N, int
                                                        const float* __restrict__ B,
                                                        float* __restrict__ C) {
     using V = typename VecT<VEC>::T;
-    constexpr int S = 64 / LPE;  // rows per wave
-    constexpr int U = 8;         // loads per block
-    __shared__ uint32_t s_off[kWaveRowsWaves][64];
-    __shared__ float s_val[kWaveRowsWaves][64];
+    constexpr int S = 64 / LPE;                   // rows per wave
+    constexpr int U = 8;                          // loads per block
+    constexpr int NC = LPE >= 32 ? 1 : 32 / LPE;  // entries a lane stages at a time
+    constexpr int CH = LPE * NC;                  // ... and a stream
+    constexpr int PAD = 1;                        // keeps the streams' reads in different banks
+    __shared__ uint2 s_ent[kWaveRowsWaves][S * (CH + PAD)];
+    __shared__ int2 s_row[kWaveRowsWaves * S];    // {first entry, entries} of the block's rows
+    __shared__ __align__(16) float s_sum[64 * 4];
 
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = (int)(threadIdx.x & 63), sub = lane / LPE, kl = lane % LPE;
-    const int64_t w = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * kWaveRowsWaves + wave;
-    const int64_t row = w * S + sub;
-    if (w * S >= M) return;
+    const int64_t row0 = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * (kWaveRowsWaves * S);
+    const int64_t row = row0 + wave * S + sub;
     const bool rowok = row < M;
-    const int32_t p0 = rowok ? rowptr[row] : 0, n = rowok ? rowptr[row + 1] - p0 : 0;
+    const int32_t p0 = rowok ? rowptr[row] : 0, nrow = rowok ? rowptr[row + 1] - p0 : 0;
+    if (kl == 0) s_row[wave * S + sub] = make_int2(p0, nrow);
+    __syncthreads();
+    // The block takes its long rows together only if few rows stand out:
+    // otherwise the rows' streams, side by side, are the faster way (16x16
+    // blocks, 51 a row, O = 100 all together 708 us, side by side 222).
+    constexpr int FEW = S >= 4 ? 4 : 2;
+    int32_t most = lane < kWaveRowsWaves * S ? s_row[lane].y : 0, sum = min(most, 1 << 24);
+#pragma unroll
+    for (int sh = 1; sh < 64; sh <<= 1) {
+        most = max(most, __shfl_xor(most, sh));
+        sum += __shfl_xor(sum, sh);
+    }
+    const bool together = uniform(most) > kLongRow && uniform(sum) / FEW <= uniform(most);
+    const bool islong = together && nrow > kLongRow;
+    const int32_t n = islong ? 0 : nrow;
     int32_t nmax = n;
 #pragma unroll
     for (int sh = LPE; sh < 64; sh <<= 1) nmax = max(nmax, __shfl_xor(nmax, sh));
     nmax = uniform(nmax);
-    uint32_t* lo = s_off[wave];
-    float* lv = s_val[wave];
+    uint2* le = s_ent[wave] + sub * (CH + PAD);
     const uint32_t row_bytes = (uint32_t)O * 4u;
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), (short)0, (int)b_bytes,
                                           kRawBufferFlags);
+    // B-row offset (index off the buffer path) of column cj; a column outside
+    // [0, N) reads nothing.
+    auto b_off = [&](int32_t cj) -> uint32_t {
+        return (uint32_t)cj < (uint32_t)N ? (BUF ? (uint32_t)cj * row_bytes : (uint32_t)cj) : kNoRow;
+    };
 
     for (int32_t k0 = 0; k0 < O; k0 += LPE * VEC) {
         const int32_t k = k0 + kl * VEC;
         const bool kok = k < O;
-        const uint32_t koff = (uint32_t)(kok ? k : 0) * 4u;
+        const uint32_t koff = (uint32_t)vec_col<VEC>(k, O) * 4u;
         V acc = zero_vec(V());
-        for (int32_t c0 = 0; c0 < nmax; c0 += LPE) {
-            // Stage this stream's entries c0 .. c0+LPE-1 (lane kl takes one);
-            // a column outside [0, N) reads nothing.
-            const int32_t i = c0 + kl;
-            const int32_t cj = i < n ? col[p0 + i] : -1;
-            const bool ok = (uint32_t)cj < (uint32_t)N;
-            lo[lane] = ok ? (BUF ? (uint32_t)cj * row_bytes : (uint32_t)cj) : kNoCol;
-            lv[lane] = ok ? val[p0 + i] : 0.f;
+        int32_t cj[NC];
+        float a[NC];
+        auto fetch = [&](int32_t c0) {
+#pragma unroll
+            for (int q = 0; q < NC; ++q) {
+                const int32_t i = c0 + q * LPE + kl;
+                cj[q] = i < n ? col[p0 + i] : -1;
+                a[q] = i < n ? val[p0 + i] : 0.f;
+            }
+        };
+        fetch(0);
+        for (int32_t c0 = 0; c0 < nmax; c0 += CH) {
+#pragma unroll
+            for (int q = 0; q < NC; ++q) {
+                const uint32_t off = b_off(cj[q]);
+                le[q * LPE + kl] =
+                    make_uint2(off, off == kNoRow ? 0u : __builtin_bit_cast(uint32_t, a[q]));
+            }
+            if (c0 + CH < nmax) fetch(c0 + CH);
             wave_sync();
-            const int32_t cnt = min(LPE, nmax - c0);
-            for (int32_t j0 = 0; j0 < cnt; j0 += U) {
+            const int32_t cnt = min(CH, nmax - c0);
+            for (int32_t j0 = 0; j0 < cnt; j0 += U) {  // CH is a multiple of U
+                uint2 e[U];
                 V b[U];
 #pragma unroll
+                for (int u = 0; u < U; ++u) e[u] = le[j0 + u];
+#pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int32_t j = min(j0 + u, LPE - 1);
-                    const uint32_t off = lo[sub * LPE + j];
                     if constexpr (BUF) {
-                        // off + koff < 2^32 (off <= 2^31, koff < 2^31); lanes
-                        // past O or past the chunk read "no column" zeros.
-                        b[u] = load_b_buf<VEC>(
-                            rsrc, (off + koff) | (kok && j0 + u < cnt ? 0u : kNoCol));
+                        b[u] = load_b_buf<VEC>(rsrc, (e[u].x + koff) | (kok ? 0u : kNoRow));
                     } else {
-                        const bool live = off != kNoCol && kok && j0 + u < cnt;
-                        b[u] = live ? *reinterpret_cast<const V*>(B + (int64_t)off * O + k)
+                        const bool live = e[u].x != kNoRow && kok;
+                        b[u] = live ? load_mem(B + (int64_t)e[u].x * O + koff / 4, V())
                                     : zero_vec(V());
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int32_t j = min(j0 + u, LPE - 1);
-                    const float a = j0 + u < cnt ? lv[sub * LPE + j] : 0.f;
-                    fma_vec(acc, a, b[u]);
-                }
+                for (int u = 0; u < U; ++u) fma_vec(acc, __builtin_bit_cast(float, e[u].y), b[u]);
             }
             wave_sync();
         }
-        if (rowok && kok) *reinterpret_cast<V*>(C + row * O + k) = acc;
+        if (rowok && !islong && kok) store_cols<VEC, false>(C + row * O, k, O, acc, false);
+    }
+
+    // Long rows.
+    if (!together) return;
+    constexpr int LV = LongShape<VEC, LPE>::LV, LU = LongShape<VEC, LPE>::LU;
+    using W = typename VecT<LV>::T;
+    for (int slot = 0; slot < kWaveRowsWaves * S; ++slot) {
+        const int32_t nl = uniform(s_row[slot].y);
+        if (nl <= kLongRow) continue;
+        const int32_t pl = uniform(s_row[slot].x), turns = (nl + LU - 1) / LU;
+        for (int32_t k0 = 0; k0 < O; k0 += 64 * LV) {
+            const int32_t k = k0 + lane * LV;
+            const bool kok = k < O;
+            const int32_t kc = vec_col<LV>(k, O);  // O >= LV
+            // This wave's turn (B rows in b, values in lanes' av) and the
+            // entries of the one after it.
+            // (Loads at clamped indices: a branch around them makes the
+            // compiler wait for them before the barrier.)
+            W b[LU];
+            float av, vnext;
+            int32_t cnext;
+            auto fetch_entries = [&](int32_t t) {
+                const int32_t i = pl + min(t * LU + (lane % LU), nl - 1);
+                cnext = col[i];
+                vnext = val[i];
+            };
+            auto fetch_rows = [&](int32_t t) {
+                const uint32_t off = t * LU + (lane % LU) < nl ? b_off(cnext) : kNoRow;
+                av = off == kNoRow ? 0.f : vnext;
+#pragma unroll
+                for (int u = 0; u < LU; ++u) {
+                    const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, u);
+                    if constexpr (BUF) {
+                        b[u] = load_b_buf<LV>(rsrc, o + (uint32_t)kc * 4u);
+                    } else {
+                        b[u] = o != kNoRow ? load_mem(B + (int64_t)o * O + kc, W()) : zero_vec(W());
+                    }
+                }
+                fetch_entries(t + kWaveRowsWaves);
+            };
+            fetch_entries(wave);
+            fetch_rows(wave);
+            // Every wave meets `turns` barriers, one at the end of each turn.
+            int32_t met = 0;
+            for (int32_t t = wave; t < turns; t += kWaveRowsWaves) {
+                for (; met < t; ++met) __syncthreads();
+                W acc = zero_vec(W());
+                if (t > 0) acc = *reinterpret_cast<const W*>(s_sum + lane * LV);
+#pragma unroll
+                for (int u = 0; u < LU; ++u)
+                    fma_vec(acc, __builtin_bit_cast(float, __builtin_amdgcn_readlane(
+                                                               __builtin_bit_cast(int, av), u)),
+                            b[u]);
+                if (t + 1 < turns) {
+                    *reinterpret_cast<W*>(s_sum + lane * LV) = acc;
+                } else if (kok) {
+                    store_cols<LV, false>(C + (row0 + slot) * O, k, O, acc, false);
+                }
+                __syncthreads();
+                ++met;
+                fetch_rows(t + kWaveRowsWaves);
+            }
+            for (; met < turns; ++met) __syncthreads();
+        }
     }
 }
 
 template <int VEC, int LPE>
 hipError_t launch_lpe(int32_t M, const int32_t* rowptr, const int32_t* col, const float* val,
                       const float* B, int32_t N, int32_t O, float* C, hipStream_t st) {
-    constexpr int S = 64 / LPE;
-    const int64_t waves = ((int64_t)M + S - 1) / S;
-    const dim3 grid((unsigned)((waves + kWaveRowsWaves - 1) / kWaveRowsWaves)),
-        block(64 * kWaveRowsWaves);
+    constexpr int rows = 64 / LPE * kWaveRowsWaves;
+    const dim3 grid((unsigned)(((int64_t)M + rows - 1) / rows)), block(64 * kWaveRowsWaves);
     const uint64_t b_bytes = (uint64_t)N * (uint64_t)O * 4u;
-    if (b_bytes + 64u * 4u * VEC >= kBufferLimit)
+    if (b_bytes >= kBufferLimit)
         hipLaunchKernelGGL((csr_wave_kernel<VEC, LPE, false>), grid, block, 0, st, M, N, O, 0u,
                            rowptr, col, val, B, C);
     else
@@ -116,26 +231,17 @@ hipError_t launch_lpe(int32_t M, const int32_t* rowptr, const int32_t* col, cons
     return hipGetLastError();
 }
 
-template <int VEC>
-hipError_t launch_vec(int32_t M, const int32_t* rowptr, const int32_t* col, const float* val,
-                      const float* B, int32_t N, int32_t O, float* C, hipStream_t st) {
-    const int32_t need = (O + VEC - 1) / VEC;
-    if (need <= 8) return launch_lpe<VEC, 8>(M, rowptr, col, val, B, N, O, C, st);
-    if (need <= 16) return launch_lpe<VEC, 16>(M, rowptr, col, val, B, N, O, C, st);
-    if (need <= 32) return launch_lpe<VEC, 32>(M, rowptr, col, val, B, N, O, C, st);
-    return launch_lpe<VEC, 64>(M, rowptr, col, val, B, N, O, C, st);
-}
-
 }  // namespace
 
 hipError_t launch_csr_wave(int32_t M, const int32_t* rowptr, const int32_t* col, const float* val,
                            const float* B, int32_t N, int32_t O, float* C, hipStream_t st) {
     if (M <= 0 || O <= 0) return hipSuccess;
-    const bool a16 = (((uintptr_t)B | (uintptr_t)C) & 15u) == 0;
-    const bool a8 = (((uintptr_t)B | (uintptr_t)C) & 7u) == 0;
-    if (O % 4 == 0 && a16) return launch_vec<4>(M, rowptr, col, val, B, N, O, C, st);
-    if (O % 2 == 0 && a8) return launch_vec<2>(M, rowptr, col, val, B, N, O, C, st);
-    return launch_vec<1>(M, rowptr, col, val, B, N, O, C, st);
+    if (O <= 8) return launch_lpe<1, 8>(M, rowptr, col, val, B, N, O, C, st);
+    if (O <= 16) return launch_lpe<1, 16>(M, rowptr, col, val, B, N, O, C, st);
+    if (O <= 32) return launch_lpe<4, 8>(M, rowptr, col, val, B, N, O, C, st);
+    if (O <= 64) return launch_lpe<4, 16>(M, rowptr, col, val, B, N, O, C, st);
+    if (O <= 128) return launch_lpe<4, 32>(M, rowptr, col, val, B, N, O, C, st);
+    return launch_lpe<4, 64>(M, rowptr, col, val, B, N, O, C, st);
 }
 
 }  // namespace vcsr
