@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -11,6 +12,7 @@
 
 #include "../../../include/vcsr_spmm.h"
 #include "../fmt_internal.hpp"
+#include "../host/parallel.hpp"
 #include "../host/tile_view.hpp"
 #include "entry.hpp"
 #include "launch.hpp"
@@ -49,46 +51,65 @@ struct RowView {
     int32_t n_partials = 0;
 };
 
-RowView make_row_view(const vcsr::Vcsr& v, const std::vector<int32_t>& nact) {
+// `cnt`: entries of every lane (vcsr::lane_counts).  Each task takes a range
+// of rows, so the result does not depend on the number of tasks.
+RowView make_row_view(const vcsr::Vcsr& v, const std::vector<int32_t>& cnt, int nthreads) {
     RowView rv;
-    const int32_t G = v.num_groups(), M = v.M, b = v.bundle;
+    const int32_t M = v.M, b = v.bundle;
     const int32_t E = vcsr::kRowChunkEntries;
-    // Entry count of every active lane (entries are packed from depth 0).
-    std::vector<int64_t> lane_off((size_t)G + 1, 0);
-    for (int32_t g = 0; g < G; ++g) lane_off[(size_t)g + 1] = lane_off[(size_t)g] + nact[(size_t)g];
-    std::vector<int32_t> lane_cnt((size_t)lane_off[(size_t)G]);
+    const vcsr::LaneRanges lr = vcsr::lane_ranges(v, cnt, nthreads);
     std::vector<int64_t> ptr((size_t)M + 1, 0);
-    for (int32_t g = 0; g < G; ++g) {
-        const int32_t depth = v.group_depth[g];
-        for (int32_t l = 0; l < nact[(size_t)g]; ++l) {
-            const int32_t slot0 = v.group_ptr[g] + l;
-            int32_t cnt = 0;
-            while (cnt < depth && v.lcol[(size_t)slot0 + (size_t)cnt * b] >= 0) ++cnt;
-            lane_cnt[(size_t)(lane_off[(size_t)g] + l)] = cnt;
-            ptr[(size_t)v.group_rows[(size_t)g * b + l] + 1] += (cnt + E - 1) / E;
-        }
-    }
+    auto by_rows = [&](auto&& body) {
+        vcsr::parallel_for(lr.ranges, 1, nthreads, [&](int64_t tb, int64_t te) {
+            for (int64_t t = tb; t < te; ++t)
+                lr.each(t, [&](int32_t i) { body(i, v.group_rows[(size_t)i]); });
+        });
+    };
+    by_rows([&](int32_t i, int32_t row) { ptr[(size_t)row + 1] += (cnt[(size_t)i] + E - 1) / E; });
     for (int32_t r = 0; r < M; ++r) ptr[(size_t)r + 1] += ptr[(size_t)r];
     const int64_t nrec = ptr[(size_t)M];
     if (nrec > INT32_MAX) throw vcsr::Error(VCSR_ERANGE, "too many (row, segment) pairs");
     rv.pair_rec.resize((size_t)nrec * 4);
     std::vector<int64_t> cur(ptr.begin(), ptr.end() - 1);
-    for (int32_t g = 0; g < G; ++g) {
-        for (int32_t l = 0; l < nact[(size_t)g]; ++l) {
-            const int32_t row = v.group_rows[(size_t)g * b + l];
-            const int32_t cnt = lane_cnt[(size_t)(lane_off[(size_t)g] + l)];
-            for (int32_t d0 = 0; d0 < cnt; d0 += E) {
-                int32_t* rec = rv.pair_rec.data() + 4 * cur[(size_t)row]++;
-                rec[0] = v.group_ptr[g] + l + d0 * b;
-                rec[1] = v.group_seg_base[g];
-                rec[2] = std::min(E, cnt - d0);
-                rec[3] = row;
-            }
+    by_rows([&](int32_t i, int32_t row) {
+        const int32_t g = i / b, l = i - g * b, c = cnt[(size_t)i];
+        for (int32_t d0 = 0; d0 < c; d0 += E) {
+            int32_t* rec = rv.pair_rec.data() + 4 * cur[(size_t)row]++;
+            rec[0] = v.group_ptr[g] + l + d0 * b;
+            rec[1] = v.group_seg_base[g];
+            rec[2] = std::min(E, c - d0);
+            rec[3] = row;
         }
-    }
-    rv.row_items.reserve((size_t)M * 4);
+    });
+    // Rows that fit one chunk (nearly all) are filled in in parallel; their
+    // positions are final when no row is split.
+    rv.row_items.resize((size_t)M * 4);
+    std::vector<uint8_t> split((size_t)M, 0);
+    std::atomic<bool> any{false};
+    vcsr::parallel_for(M, 8192, nthreads, [&](int64_t rb, int64_t re) {
+        for (int64_t r = rb; r < re; ++r) {
+            const int32_t p0 = (int32_t)ptr[(size_t)r], p1 = (int32_t)ptr[(size_t)r + 1];
+            int64_t entries = 0;
+            for (int32_t p = p0; p < p1; ++p) entries += rv.pair_rec[(size_t)p * 4 + 2];
+            if (p1 - p0 > vcsr::kRowChunkPairs || entries > E) {
+                split[(size_t)r] = 1;
+                any = true;
+            }
+            int32_t* it = &rv.row_items[(size_t)r * 4];
+            it[0] = (int32_t)r, it[1] = p0, it[2] = p1, it[3] = -1;
+        }
+    });
+    if (!any) return rv;
+    std::vector<int32_t> whole;
+    whole.swap(rv.row_items);
+    rv.row_items.reserve(whole.size() + whole.size() / 8);
     std::vector<int32_t> chunk_starts;
     for (int32_t r = 0; r < M; ++r) {
+        if (!split[(size_t)r]) {
+            const int32_t* it = &whole[(size_t)r * 4];
+            rv.row_items.insert(rv.row_items.end(), it, it + 4);
+            continue;
+        }
         const int32_t p0 = (int32_t)ptr[(size_t)r], p1 = (int32_t)ptr[(size_t)r + 1];
         chunk_starts.clear();
         chunk_starts.push_back(p0);
@@ -100,10 +121,6 @@ RowView make_row_view(const vcsr::Vcsr& v, const std::vector<int32_t>& nact) {
                 entries = 0;
             }
             entries += c;
-        }
-        if (chunk_starts.size() == 1) {
-            rv.row_items.insert(rv.row_items.end(), {r, p0, p1, -1});
-            continue;
         }
         const int32_t first = rv.n_partials;
         for (size_t q = 0; q < chunk_starts.size(); ++q) {
@@ -192,58 +209,62 @@ int vcsr_fmt_upload(vcsr_fmt* fmt, void* stream) {
         const vcsr::Vcsr& v = fmt->v;
         hipStream_t st = (hipStream_t)stream;
         // Derived per-group active-lane count: lanes are sorted by entry count,
-        // so the lanes with >= 1 entry are a prefix, and their depth-0 slot is
-        // the first real entry.
+        // so the lanes with >= 1 entry are a prefix.
         const int32_t G = v.num_groups();
+        const int nthreads = vcsr::default_threads();
+        const std::vector<int32_t> cnt = vcsr::lane_counts(v, nthreads);
         std::vector<int32_t> nact((size_t)G);
         int32_t max_depth = 0;
         for (int32_t g = 0; g < G; ++g) {
             int32_t n = 0;
-            for (int32_t l = 0; l < v.bundle; ++l) n += v.lcol[(size_t)v.group_ptr[g] + l] >= 0;
+            for (int32_t l = 0; l < v.bundle; ++l) n += cnt[(size_t)g * v.bundle + l] > 0;
             nact[(size_t)g] = n;
             max_depth = std::max(max_depth, v.group_depth[g]);
         }
         std::vector<int32_t> items = make_items(v, 256);
-        RowView rv = make_row_view(v, nact);
+        const RowView rv = make_row_view(v, cnt, nthreads);
         const vcsr::TileView tv = vcsr::make_tile_view(v, fmt->tile_rows, 0, fmt->tile_fixed);
         // Device copy of the entries' B rows: placeholders (no row present)
         // are marked kTileNoEntry, so the kernels tell them apart without
-        // reading the presence bits.
-        std::vector<int32_t> tv_brow(tv.brow);
-        for (size_t q = 0; q < tv_brow.size(); ++q)
-            if (tv.mask[q] == 0) tv_brow[q] = vcsr::kTileNoEntry;
-        // Device values: for 1- and 3-row tiles each entry's B row follows
-        // its values (vcsr::tile_dev_stride).
+        // reading the presence bits.  For 1- and 3-row tiles each entry's B
+        // row follows its values instead (vcsr::tile_dev_stride).
+        const bool fold = vcsr::tile_dev_folds_brow(tv.R);
+        const size_t E = tv.brow.size();
+        std::vector<int32_t> tv_brow(fold ? 0 : E);
         std::vector<float> tv_val;
-        if (vcsr::tile_dev_folds_brow(tv.R)) {
-            const int32_t rs = vcsr::tile_slot_stride(tv.R), ds = vcsr::tile_dev_stride(tv.R);
-            const size_t E = tv_brow.size();
-            tv_val.assign(E * (size_t)ds, 0.f);
-            for (size_t q = 0; q < E; ++q) {
-                for (int32_t r = 0; r < tv.R; ++r)
-                    tv_val[q * ds + r] = tv.val[q * rs + r];
-                std::memcpy(&tv_val[q * ds + ds - 1], &tv_brow[q], sizeof(float));
+        const int32_t rs = vcsr::tile_slot_stride(tv.R), ds = vcsr::tile_dev_stride(tv.R);
+        if (fold) tv_val.resize(E * (size_t)ds);
+        vcsr::parallel_for((int64_t)E, 1 << 16, nthreads, [&](int64_t qb, int64_t qe) {
+            for (size_t q = (size_t)qb; q < (size_t)qe; ++q) {
+                const int32_t br = tv.mask[q] == 0 ? vcsr::kTileNoEntry : tv.brow[q];
+                if (!fold) {
+                    tv_brow[q] = br;
+                    continue;
+                }
+                float* rec = &tv_val[q * ds];
+                for (int32_t r = 0; r < tv.R; ++r) rec[r] = tv.val[q * rs + r];
+                // Single-row tiles: 31 bits; the pieces' ends are marked below.
+                const int32_t word = tv.R == 1 && br == vcsr::kTileNoEntry ? vcsr::kTileNoRow : br;
+                std::memcpy(&rec[ds - 1], &word, sizeof(float));
             }
-        }
+        });
         const size_t n_pieces = tv.pieces.size() / 4, n_items = tv.chunks.size() / 4;
         std::vector<int32_t> tv_pieces, tv_items, tv_dest;
         if (tv.R == 1) {
-            // Each entry's record {value, B row | end of piece << 31}.
+            // Each entry's record is {value, B row | end of piece << 31}.
             tv_dest.resize(n_pieces);
-            for (size_t q = 0; q < tv_brow.size(); ++q) {
-                const uint32_t br = tv_brow[q] == vcsr::kTileNoEntry ? (uint32_t)vcsr::kTileNoRow
-                                                                     : (uint32_t)tv_brow[q];
-                std::memcpy(&tv_val[2 * q + 1], &br, sizeof(float));
-            }
-            for (size_t p = 0; p < n_pieces; ++p) {
-                const int32_t* pc = &tv.pieces[4 * p];
-                const size_t end = p + 1 < n_pieces ? (size_t)pc[6] : tv_brow.size();
-                uint32_t br;
-                std::memcpy(&br, &tv_val[2 * end - 1], sizeof(float));
-                br |= 0x80000000u;
-                std::memcpy(&tv_val[2 * end - 1], &br, sizeof(float));
-                tv_dest[p] = pc[3] < 0 ? pc[0] : ~pc[3];
-            }
+            vcsr::parallel_for((int64_t)n_pieces, 1 << 15, nthreads, [&](int64_t pb, int64_t pe) {
+                for (size_t p = (size_t)pb; p < (size_t)pe; ++p) {
+                    const int32_t* pc = &tv.pieces[4 * p];
+                    const size_t end = p + 1 < n_pieces ? (size_t)pc[6] : E;
+                    uint32_t br;
+                    std::memcpy(&br, &tv_val[2 * end - 1], sizeof(float));
+                    br |= 0x80000000u;
+                    std::memcpy(&tv_val[2 * end - 1], &br, sizeof(float));
+                    tv_dest[p] = pc[3] < 0 ? pc[0] : ~pc[3];
+                }
+            });
+            tv_items.reserve(2 * n_items + 2);
             for (size_t c = 0; c < n_items; ++c)
                 tv_items.insert(tv_items.end(), {tv.chunks[4 * c], tv.chunks[4 * c + 2]});
             tv_items.insert(tv_items.end(), {(int32_t)tv.n_entries(), (int32_t)n_pieces});

@@ -25,45 +25,36 @@ struct RowLists {
     std::vector<int32_t> col, slot;
 };
 
-int32_t lane_entries(const Vcsr& v, int32_t g, int32_t l) {
-    const int64_t s0 = (int64_t)v.group_ptr[g] + l;
-    int32_t c = 0;
-    while (c < v.group_depth[g] && v.lcol[(size_t)(s0 + (int64_t)c * v.bundle)] >= 0) ++c;
-    return c;
-}
-
 RowLists row_lists(const Vcsr& v, int nthreads) {
-    const int32_t G = v.num_groups(), M = v.M, b = v.bundle;
+    const int32_t M = v.M, b = v.bundle;
+    const std::vector<int32_t> cnt = lane_counts(v, nthreads);
     RowLists rl;
     rl.ptr.assign((size_t)M + 1, 0);
-    for (int32_t g = 0; g < G; ++g) {
-        for (int32_t l = 0; l < b; ++l) {
-            const int32_t c = lane_entries(v, g, l);
-            if (c == 0) continue;
-            const int32_t row = v.group_rows[(size_t)g * b + l];
-            if (row < 0 || row >= M) throw Error(kEinval, "group row out of range");
-            rl.ptr[(size_t)row + 1] += c;
-        }
-    }
+    const LaneRanges lr = lane_ranges(v, cnt, nthreads);
+    parallel_for(lr.ranges, 1, nthreads, [&](int64_t tb, int64_t te) {
+        for (int64_t t = tb; t < te; ++t)
+            lr.each(t, [&](int32_t i) {
+                rl.ptr[(size_t)v.group_rows[(size_t)i] + 1] += cnt[(size_t)i];
+            });
+    });
     for (int32_t r = 0; r < M; ++r) rl.ptr[(size_t)r + 1] += rl.ptr[(size_t)r];
     const int64_t total = rl.ptr[(size_t)M];
     rl.col.resize((size_t)total);
     rl.slot.resize((size_t)total);
     std::vector<int64_t> cur(rl.ptr.begin(), rl.ptr.end() - 1);
-    for (int32_t g = 0; g < G; ++g) {
-        const int32_t base = v.group_seg_base[g];
-        for (int32_t l = 0; l < b; ++l) {
-            const int32_t c = lane_entries(v, g, l);
-            if (c == 0) continue;
-            int64_t& at = cur[(size_t)v.group_rows[(size_t)g * b + l]];
-            for (int32_t d = 0; d < c; ++d) {
-                const int64_t s = (int64_t)v.group_ptr[g] + l + (int64_t)d * b;
-                rl.col[(size_t)at] = base + v.lcol[(size_t)s];
-                rl.slot[(size_t)at] = (int32_t)s;
-                ++at;
-            }
-        }
-    }
+    parallel_for(lr.ranges, 1, nthreads, [&](int64_t tb, int64_t te) {
+        for (int64_t t = tb; t < te; ++t)
+            lr.each(t, [&](int32_t i) {
+                const int32_t g = i / b, l = i - g * b, base = v.group_seg_base[(size_t)g];
+                int64_t& at = cur[(size_t)v.group_rows[(size_t)i]];
+                for (int32_t d = 0; d < cnt[(size_t)i]; ++d) {
+                    const int64_t s = (int64_t)v.group_ptr[(size_t)g] + l + (int64_t)d * b;
+                    rl.col[(size_t)at] = base + v.lcol[(size_t)s];
+                    rl.slot[(size_t)at] = (int32_t)s;
+                    ++at;
+                }
+            });
+    });
     // Groups come in segment order and a lane's slots in local-column order,
     // so rows are already sorted; sort any row that is not (stable, so equal
     // columns keep their slot order).
@@ -119,6 +110,11 @@ void tile_rows(const RowLists& rl, int32_t r0, int32_t r1, int32_t cap, bool fix
                std::vector<Tile>& out) {
     std::vector<int32_t> u, w;
     int32_t i = r0;
+    if (cap == 1) {
+        for (; i < r1; ++i)
+            out.push_back({i, 1, std::max<int64_t>(1, rl.ptr[(size_t)i + 1] - rl.ptr[(size_t)i])});
+        return;
+    }
     while (i < r1) {
         u.assign(rl.col.begin() + rl.ptr[(size_t)i], rl.col.begin() + rl.ptr[(size_t)i + 1]);
         int32_t n = 1;
@@ -135,21 +131,29 @@ void tile_rows(const RowLists& rl, int32_t r0, int32_t r1, int32_t cap, bool fix
     }
 }
 
-std::vector<Tile> make_tiles(const RowLists& rl, int32_t M, int32_t cap, bool fixed,
-                             int nthreads) {
-    const int32_t nblk = (M + kTileRowBlock - 1) / kTileRowBlock;
-    std::vector<std::vector<Tile>> per((size_t)nblk);
-    parallel_for(nblk, 1, nthreads, [&](int64_t bb, int64_t be) {
-        for (int64_t blk = bb; blk < be; ++blk) {
+// Tiles of every height in `caps`; tasks are (height, block of rows).
+std::vector<std::vector<Tile>> make_tiles(const RowLists& rl, int32_t M,
+                                          const std::vector<int32_t>& caps, bool fixed,
+                                          int nthreads) {
+    const int64_t nblk = (M + kTileRowBlock - 1) / kTileRowBlock, nc = (int64_t)caps.size();
+    std::vector<std::vector<Tile>> per((size_t)(nblk * nc));
+    // The tallest tiles first: they take longest.
+    parallel_for(nblk * nc, 1, nthreads, [&](int64_t bb, int64_t be) {
+        for (int64_t q = bb; q < be; ++q) {
+            const int64_t c = nc - 1 - q / nblk, blk = q % nblk;
             const int32_t r0 = (int32_t)blk * kTileRowBlock;
-            tile_rows(rl, r0, std::min(M, r0 + kTileRowBlock), cap, fixed, per[(size_t)blk]);
+            tile_rows(rl, r0, std::min(M, r0 + kTileRowBlock), caps[(size_t)c], fixed,
+                      per[(size_t)(c * nblk + blk)]);
         }
     });
-    std::vector<Tile> tiles;
-    for (auto& p : per) tiles.insert(tiles.end(), p.begin(), p.end());
+    std::vector<std::vector<Tile>> tiles((size_t)nc);
+    for (int64_t c = 0; c < nc; ++c)
+        for (int64_t blk = 0; blk < nblk; ++blk) {
+            const auto& p = per[(size_t)(c * nblk + blk)];
+            tiles[(size_t)c].insert(tiles[(size_t)c].end(), p.begin(), p.end());
+        }
     return tiles;
 }
-
 
 // Single-row views: the kernel hands work items to the XCDs in eight
 // contiguous runs of the item list (one per XCD, device/common.hpp
@@ -166,7 +170,7 @@ std::vector<Tile> make_tiles(const RowLists& rl, int32_t M, int32_t cap, bool fi
 // (more than 64 entries) gave 25.3 / 34.7 / 98.5, from 4 or 16 pieces up
 // 25.1 / 34.3 / 95.3 and 24.9 / 34.1 / 95.4, from 32 pieces up 25.0 / 34.2
 // / 98.2.
-void order_long_pieces_by_column(TileView& tv, int32_t N) {
+void order_long_pieces_by_column(TileView& tv, int32_t N, int nthreads) {
     constexpr int kSeg = 8;
     constexpr int32_t kMinPieces = 8;
     const int32_t nc = (int32_t)(tv.chunks.size() / 4);
@@ -217,30 +221,82 @@ void order_long_pieces_by_column(TileView& tv, int32_t N) {
     out.split = tv.split;
     out.n_partial_rows = tv.n_partial_rows;
     const size_t E = tv.brow.size();
-    out.brow.reserve(E);
-    out.slot.reserve(E);
-    out.val.reserve(E);
-    out.mask.reserve(E);
-    out.pieces.reserve(tv.pieces.size());
-    out.chunks.reserve(tv.chunks.size());
-    for (int32_t c : order) {
-        const int32_t e0 = tv.chunks[4 * (size_t)c], e1 = tv.chunks[4 * (size_t)c + 1];
-        const int32_t p0 = tv.chunks[4 * (size_t)c + 2], p1 = tv.chunks[4 * (size_t)c + 3];
-        const int32_t ne0 = (int32_t)out.brow.size(), np0 = (int32_t)(out.pieces.size() / 4);
-        out.brow.insert(out.brow.end(), tv.brow.begin() + e0, tv.brow.begin() + e1);
-        out.slot.insert(out.slot.end(), tv.slot.begin() + e0, tv.slot.begin() + e1);
-        out.val.insert(out.val.end(), tv.val.begin() + e0, tv.val.begin() + e1);
-        out.mask.insert(out.mask.end(), tv.mask.begin() + e0, tv.mask.begin() + e1);
-        for (int32_t q = p0; q < p1; ++q)
-            out.pieces.insert(out.pieces.end(), {tv.pieces[4 * (size_t)q], tv.pieces[4 * (size_t)q + 1],
-                                                 tv.pieces[4 * (size_t)q + 2] - e0 + ne0,
-                                                 tv.pieces[4 * (size_t)q + 3]});
-        out.chunks.insert(out.chunks.end(), {ne0, ne0 + (e1 - e0), np0, np0 + (p1 - p0)});
+    out.brow.resize(E);
+    out.slot.resize(E);
+    out.val.resize(E);
+    out.mask.resize(E);
+    out.pieces.resize(tv.pieces.size());
+    out.chunks.resize(tv.chunks.size());
+    int32_t ne0 = 0, np0 = 0;
+    for (size_t i = 0; i < order.size(); ++i) {
+        const int32_t* c = &tv.chunks[4 * (size_t)order[i]];
+        int32_t* o = &out.chunks[4 * i];
+        o[0] = ne0;
+        o[1] = ne0 += c[1] - c[0];
+        o[2] = np0;
+        o[3] = np0 += c[3] - c[2];
     }
+    parallel_for((int64_t)order.size(), 4096, nthreads, [&](int64_t ib, int64_t ie) {
+        for (int64_t i = ib; i < ie; ++i) {
+            const int32_t* c = &tv.chunks[4 * (size_t)order[(size_t)i]];
+            const int32_t* o = &out.chunks[4 * (size_t)i];
+            std::copy(tv.brow.begin() + c[0], tv.brow.begin() + c[1], out.brow.begin() + o[0]);
+            std::copy(tv.slot.begin() + c[0], tv.slot.begin() + c[1], out.slot.begin() + o[0]);
+            std::copy(tv.val.begin() + c[0], tv.val.begin() + c[1], out.val.begin() + o[0]);
+            std::copy(tv.mask.begin() + c[0], tv.mask.begin() + c[1], out.mask.begin() + o[0]);
+            for (int32_t q = c[2], w = o[2]; q < c[3]; ++q, ++w) {
+                const int32_t* p = &tv.pieces[4 * (size_t)q];
+                int32_t* x = &out.pieces[4 * (size_t)w];
+                x[0] = p[0];
+                x[1] = p[1];
+                x[2] = p[2] - c[0] + o[0];
+                x[3] = p[3];
+            }
+        }
+    });
     tv = std::move(out);
 }
 
 }  // namespace
+
+std::vector<int32_t> lane_counts(const Vcsr& v, int nthreads) {
+    const int32_t G = v.num_groups(), b = v.bundle;
+    std::vector<int32_t> cnt((size_t)G * b);
+    parallel_for(G, 1024, nthreads, [&](int64_t gb, int64_t ge) {
+        for (int64_t g = gb; g < ge; ++g) {
+            const int32_t* p = v.lcol.data() + v.group_ptr[(size_t)g];
+            int32_t* c = cnt.data() + g * b;
+            for (int32_t l = 0; l < b; ++l) c[l] = 0;
+            // Entries are packed from depth 0: a lane ends at its first -1.
+            for (int32_t d = 0; d < v.group_depth[(size_t)g]; ++d, p += b)
+                for (int32_t l = 0; l < b; ++l) c[l] += c[l] == d && p[l] >= 0;
+        }
+    });
+    return cnt;
+}
+
+LaneRanges lane_ranges(const Vcsr& v, const std::vector<int32_t>& cnt, int nthreads) {
+    const int64_t lanes = (int64_t)v.num_groups() * v.bundle;
+    LaneRanges lr;
+    lr.ranges = lr.blocks = std::min<int64_t>(std::max(1, nthreads), 1 + lanes / 32768);
+    lr.lanes.resize((size_t)(lr.ranges * lr.blocks));
+    // Multiplication instead of a division per lane: the ranges differ by
+    // less than one 2^-32th, and any split into ranges is a valid one.
+    const uint64_t scale = v.M > 0 ? ((uint64_t)lr.ranges << 32) / (uint64_t)v.M : 0;
+    parallel_for(lr.blocks, 1, nthreads, [&](int64_t bb, int64_t be) {
+        for (int64_t blk = bb; blk < be; ++blk) {
+            std::vector<int32_t>* out = &lr.lanes[(size_t)(blk * lr.ranges)];
+            const int64_t i1 = (blk + 1) * lanes / lr.blocks;
+            for (int64_t i = blk * lanes / lr.blocks; i < i1; ++i) {
+                if (cnt[(size_t)i] == 0) continue;
+                const int32_t row = v.group_rows[(size_t)i];
+                if (row < 0 || row >= v.M) throw Error(kEinval, "group row out of range");
+                out[((uint64_t)row * scale) >> 32].push_back((int32_t)i);
+            }
+        }
+    });
+    return lr;
+}
 
 TileView make_tile_view(const Vcsr& v, int32_t R, int nthreads, bool fixed) {
     if (R != 0 && R != 1 && R != 2 && R != 3 && R != 4 && R != 8 && R != kTileMmaRows)
@@ -262,22 +318,28 @@ TileView make_tile_view(const Vcsr& v, int32_t R, int nthreads, bool fixed) {
     };
     if (R == 0) {
         double best = 0;
-        for (int32_t cap : {1, 2, 3, 4, 8, kTileMmaRows}) {
-            std::vector<Tile> t = make_tiles(rl, M, cap, false, nthreads);
-            int64_t ent = 0;
-            for (const Tile& x : t) ent += pad(cap, x.nent);
-            if (cap == kTileMmaRows && (int64_t)t.size() * 12 > (int64_t)M) continue;
-            const double cost = (double)ent * (16.0 + (cap == kTileMmaRows ? 4 : cap));
-            if (R == 0 || cost < best) {
-                best = cost;
-                R = cap;
-                tiles.swap(t);
+        // Heights 1 and 2 first: where rows share no columns (2 costs more
+        // than 1) the taller ones only cost.
+        for (const std::vector<int32_t>& caps :
+             {std::vector<int32_t>{1, 2}, std::vector<int32_t>{3, 4, 8, kTileMmaRows}}) {
+            auto all = make_tiles(rl, M, caps, false, nthreads);
+            for (size_t c = 0; c < caps.size(); ++c) {
+                const int32_t cap = caps[c];
+                std::vector<Tile>& t = all[c];
+                int64_t ent = 0;
+                for (const Tile& x : t) ent += pad(cap, x.nent);
+                if (cap == kTileMmaRows && (int64_t)t.size() * 12 > (int64_t)M) continue;
+                const double cost = (double)ent * (16.0 + (cap == kTileMmaRows ? 4 : cap));
+                if (R == 0 || cost < best) {
+                    best = cost;
+                    R = cap;
+                    tiles.swap(t);
+                }
             }
-            // No sharing between neighbouring rows: taller tiles only cost.
-            if (cap == 2 && R == 1) break;
+            if (R == 1) break;
         }
     } else {
-        tiles = make_tiles(rl, M, R, fixed, nthreads);
+        tiles = std::move(make_tiles(rl, M, {R}, fixed, nthreads)[0]);
     }
     if (R == kTileMmaRows)
         for (Tile& x : tiles) x.nent = pad(R, x.nent);
@@ -295,7 +357,9 @@ TileView make_tile_view(const Vcsr& v, int32_t R, int nthreads, bool fixed) {
     tv.mask.assign((size_t)E, 0);
     const size_t nval = R == kTileMmaRows ? (size_t)E * kTileMmaRows : (size_t)E * stride;
     tv.val.assign(nval, 0.f);
-    parallel_for((int64_t)tiles.size(), 1024, nthreads, [&](int64_t tb, int64_t te) {
+    const int64_t tile_grain =
+        std::min<int64_t>(1024, std::max<int64_t>(64, (int64_t)tiles.size() / (4 * nthreads)));
+    parallel_for((int64_t)tiles.size(), tile_grain, nthreads, [&](int64_t tb, int64_t te) {
         std::vector<int32_t> u, w;
         for (int64_t t = tb; t < te; ++t) {
             const Tile& x = tiles[(size_t)t];
@@ -333,6 +397,8 @@ TileView make_tile_view(const Vcsr& v, int32_t R, int nthreads, bool fixed) {
     // tile_piece_entries that write partial sums when it needs more than
     // one); shorter tiles are packed in row order.
     const int32_t cap_e = tile_chunk_entries(R), cap_p = tile_piece_entries(R);
+    tv.pieces.reserve(4 * tiles.size() + 4 * (size_t)(E / cap_p));
+    tv.chunks.reserve(4 * (size_t)(2 * E / cap_e) + 64);
     int64_t ce0 = 0, cent = 0;
     int32_t cp0 = 0;
     auto close_chunk = [&](int64_t next_e) {
@@ -403,7 +469,7 @@ TileView make_tile_view(const Vcsr& v, int32_t R, int nthreads, bool fixed) {
         tv.split.swap(sorted);
     }
     tv.n_partial_rows = (int32_t)n_partial;
-    if (R == 1 && !fixed) order_long_pieces_by_column(tv, v.N);
+    if (R == 1 && !fixed) order_long_pieces_by_column(tv, v.N, nthreads);
     return tv;
 }
 

@@ -105,6 +105,23 @@ struct TileView {
     int64_t n_entries() const { return (int64_t)brow.size(); }
 };
 
+// Entries of every lane of every group (group_rows' layout).
+std::vector<int32_t> lane_counts(const Vcsr& v, int nthreads);
+
+// The lanes that hold entries (indices into group_rows), by range of rows: a
+// task per range can walk its rows' lanes in group order, whatever the number
+// of ranges.  A lane whose row is outside [0, M) is an error.
+struct LaneRanges {
+    int64_t ranges = 1, blocks = 1;
+    std::vector<std::vector<int32_t>> lanes;  // blocks x ranges
+    template <class F>
+    void each(int64_t range, F&& f) const {
+        for (int64_t b = 0; b < blocks; ++b)
+            for (int32_t i : lanes[(size_t)(b * ranges + range)]) f(i);
+    }
+};
+LaneRanges lane_ranges(const Vcsr& v, const std::vector<int32_t>& cnt, int nthreads);
+
 // Builds the view.  R = 0 picks the tile height that minimises the modelled
 // cost (B-row loads plus accumulator updates); R = 1, 2, 3, 4, 8 or 16 forces
 // it.  fixed = true cuts the rows into fixed windows of R consecutive rows

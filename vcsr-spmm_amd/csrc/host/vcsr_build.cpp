@@ -64,21 +64,55 @@ struct BlockOut {
 };
 
 // Buckets all nnz by segment, keeping (row ascending, p ascending) order
-// inside a segment, the order in which the reference pushes them.
-void bucket_by_segment(const Csr& csr, int segw, int S, std::vector<int64_t>& seg_off,
-                       std::vector<SegEntry>& ent) {
+// inside a segment, the order in which the reference pushes them.  Blocks of
+// rows of about equal nnz count their entries per segment and then write them
+// at the offsets that follow from the blocks before them, so the result does
+// not depend on the number of blocks.
+void bucket_by_segment(const Csr& csr, int segw, int S, int nthreads,
+                       std::vector<int64_t>& seg_off, std::vector<SegEntry>& ent) {
     seg_off.assign((size_t)S + 1, 0);
-    for (int32_t p = 0; p < csr.nnz; ++p) seg_off[(size_t)(csr.col[p] / segw) + 1]++;
-    for (int s = 0; s < S; ++s) seg_off[s + 1] += seg_off[s];
     ent.resize((size_t)csr.nnz);
-    std::vector<int64_t> cur(seg_off.begin(), seg_off.end() - 1);
-    for (int32_t r = 0; r < csr.M; ++r) {
-        for (int32_t p = csr.row_ptr[r]; p < csr.row_ptr[r + 1]; ++p) {
-            const int32_t c = csr.col[p];
-            const int32_t sid = c / segw;
-            ent[(size_t)cur[sid]++] = SegEntry{r, c % segw, csr.val[p]};
+    int64_t nb = std::min<int64_t>(nthreads, 1 + csr.nnz / 65536);
+    while (nb > 1 && nb * (int64_t)S > (int64_t)csr.nnz * 2) nb /= 2;
+    std::vector<int32_t> row_of((size_t)nb + 1, csr.M);
+    for (int64_t b = 0; b < nb; ++b) {
+        const int32_t p = (int32_t)((int64_t)csr.nnz * b / nb);
+        row_of[(size_t)b] = (int32_t)(std::lower_bound(csr.row_ptr.begin(), csr.row_ptr.end(), p) -
+                                      csr.row_ptr.begin());
+    }
+    row_of[0] = 0;
+    std::vector<std::vector<int64_t>> at((size_t)nb);
+    parallel_for(nb, 1, nthreads, [&](int64_t bb, int64_t be) {
+        for (int64_t b = bb; b < be; ++b) {
+            auto& c = at[(size_t)b];
+            c.assign((size_t)S, 0);
+            const int32_t p1 = csr.row_ptr[row_of[(size_t)b + 1]];
+            for (int32_t p = csr.row_ptr[row_of[(size_t)b]]; p < p1; ++p)
+                c[(size_t)(csr.col[p] / segw)]++;
+        }
+    });
+    int64_t off = 0;
+    for (int s = 0; s < S; ++s) {
+        seg_off[(size_t)s] = off;
+        for (auto& c : at) {
+            const int64_t n = c[(size_t)s];
+            c[(size_t)s] = off;
+            off += n;
         }
     }
+    seg_off[(size_t)S] = off;
+    parallel_for(nb, 1, nthreads, [&](int64_t bb, int64_t be) {
+        for (int64_t b = bb; b < be; ++b) {
+            auto& cur = at[(size_t)b];
+            for (int32_t r = row_of[(size_t)b]; r < row_of[(size_t)b + 1]; ++r) {
+                for (int32_t p = csr.row_ptr[r]; p < csr.row_ptr[r + 1]; ++p) {
+                    const int32_t c = csr.col[p];
+                    const int32_t sid = c / segw;
+                    ent[(size_t)cur[(size_t)sid]++] = SegEntry{r, c - sid * segw, csr.val[p]};
+                }
+            }
+        }
+    });
 }
 
 // Splits a segment's entries into per-row runs and orders each run by local
@@ -226,10 +260,15 @@ Vcsr build_vcsr(const Csr& csr, int segw, int bundle, int layout, int nthreads) 
 
     std::vector<int64_t> seg_off;
     std::vector<SegEntry> ent;
-    bucket_by_segment(csr, segw, S, seg_off, ent);
+    bucket_by_segment(csr, segw, S, nthreads, seg_off, ent);
 
     // Segments per task: layout H does O(M log M) work per segment.
-    const int64_t grain = (layout == kLayoutH) ? 8 : 2048;
+    // Others: several tasks per thread (2,048 segments a task left a matrix of
+    // 20,000 columns to 3 of 16 threads).
+    const int64_t grain =
+        layout == kLayoutH
+            ? 8
+            : std::min<int64_t>(2048, std::max<int64_t>(16, S / (8 * (int64_t)nthreads)));
     const int64_t nblocks = (S + grain - 1) / grain;
     std::vector<BlockOut> blocks((size_t)nblocks);
     parallel_for(nblocks, 1, nthreads, [&](int64_t bb, int64_t be) {
@@ -263,34 +302,41 @@ Vcsr build_vcsr(const Csr& csr, int segw, int bundle, int layout, int nthreads) 
     }
     if (P > INT32_MAX) throw Error(5, "packed slot count exceeds int32");
     if (G * (int64_t)bundle > INT32_MAX) throw Error(5, "groups*bundle exceeds int32");
-    V.group_ptr.reserve((size_t)G + 1);
-    V.group_depth.reserve((size_t)G);
-    V.group_seg_base.reserve((size_t)G);
-    V.group_rows.reserve((size_t)(G * bundle));
-    V.lcol.reserve((size_t)P);
-    V.val.reserve((size_t)P);
-    V.segment_group_start.reserve((size_t)S + 1);
-    V.segment_group_start.push_back(0);
-    int64_t slot = 0;
+    V.group_ptr.resize((size_t)G + 1);
+    V.group_depth.resize((size_t)G);
+    V.group_seg_base.resize((size_t)G);
+    V.group_rows.resize((size_t)(G * bundle));
+    V.lcol.resize((size_t)P);
+    V.val.resize((size_t)P);
+    V.segment_group_start.resize((size_t)S + 1);
+    V.segment_group_start[0] = 0;
+    std::vector<int64_t> g0((size_t)nblocks + 1, 0), p0((size_t)nblocks + 1, 0);
     for (int64_t b = 0; b < nblocks; ++b) {
-        const BlockOut& out = blocks[(size_t)b];
-        size_t gi = 0;
-        for (size_t k = 0; k < out.groups_per_seg.size(); ++k) {
-            const int32_t sid = (int32_t)(b * grain + (int64_t)k);
-            for (int32_t q = 0; q < out.groups_per_seg[k]; ++q, ++gi) {
-                V.group_ptr.push_back((int32_t)slot);
-                V.group_depth.push_back(out.depth[gi]);
-                V.group_seg_base.push_back(sid * segw);
-                slot += (int64_t)out.depth[gi] * bundle;
-            }
-            V.segment_group_start.push_back((int32_t)V.group_depth.size());
-        }
-        V.group_rows.insert(V.group_rows.end(), out.rows.begin(), out.rows.end());
-        V.lcol.insert(V.lcol.end(), out.lcol.begin(), out.lcol.end());
-        V.val.insert(V.val.end(), out.val.begin(), out.val.end());
-        blocks[(size_t)b] = BlockOut();  // release as we go
+        g0[(size_t)b + 1] = g0[(size_t)b] + (int64_t)blocks[(size_t)b].depth.size();
+        p0[(size_t)b + 1] = p0[(size_t)b] + (int64_t)blocks[(size_t)b].lcol.size();
     }
-    V.group_ptr.push_back((int32_t)slot);
+    V.group_ptr[(size_t)G] = (int32_t)P;
+    parallel_for(nblocks, 1, nthreads, [&](int64_t bb, int64_t be) {
+        for (int64_t b = bb; b < be; ++b) {
+            const BlockOut& out = blocks[(size_t)b];
+            int64_t gi = 0, slot = p0[(size_t)b];
+            const int64_t gb = g0[(size_t)b];
+            for (size_t k = 0; k < out.groups_per_seg.size(); ++k) {
+                const int32_t sid = (int32_t)(b * grain + (int64_t)k);
+                for (int32_t q = 0; q < out.groups_per_seg[k]; ++q, ++gi) {
+                    V.group_ptr[(size_t)(gb + gi)] = (int32_t)slot;
+                    V.group_depth[(size_t)(gb + gi)] = out.depth[(size_t)gi];
+                    V.group_seg_base[(size_t)(gb + gi)] = sid * segw;
+                    slot += (int64_t)out.depth[(size_t)gi] * bundle;
+                }
+                V.segment_group_start[(size_t)sid + 1] = (int32_t)(gb + gi);
+            }
+            std::copy(out.rows.begin(), out.rows.end(), V.group_rows.begin() + gb * bundle);
+            std::copy(out.lcol.begin(), out.lcol.end(), V.lcol.begin() + p0[(size_t)b]);
+            std::copy(out.val.begin(), out.val.end(), V.val.begin() + p0[(size_t)b]);
+            blocks[(size_t)b] = BlockOut();  // release as we go
+        }
+    });
     return V;
 }
 
