@@ -196,11 +196,22 @@ __device__ __forceinline__ float vec_part(const typename VecT<VEC>::T& b, int c)
     return reinterpret_cast<const float*>(&b)[c];
 }
 
-// GU entry groups (of 16) per block of loads.  SB: a scheduling barrier
-// keeps the block's loads ahead of its MFMAs (more loads in flight per wave,
-// more registers); without it the compiler interleaves them and the kernel
-// fits 8 waves per SIMD.
-template <int VEC, bool BUF, int GU, bool SB>
+// Operands of NG entry groups of one wave.
+template <int VEC, int NUM>
+struct MmaGroups {
+    static constexpr int NG = NUM;
+    float4 a[NG];
+    typename VecT<VEC>::T b[NG][4];
+};
+
+// How a wave's loads and MFMAs follow each other, GU entry groups (of 16) per
+// block of loads.
+enum MmaOrder {
+    kMmaMixed,  // as the compiler interleaves them: the fewest registers
+    kMmaAhead,  // a block's loads ahead of its MFMAs (a scheduling barrier)
+    kMmaTwo     // two sets of operands, one multiplied while the other loads
+};
+template <int VEC, bool BUF, int GU, MmaOrder ORD>
 __global__ __launch_bounds__(256) void vcsr_tile_mma_kernel(
     int32_t n_items, int32_t n_ctiles, int32_t O, int32_t ld, int32_t accumulate, uint32_t b_bytes,
     const int4* __restrict__ chunks, const int4* __restrict__ pieces,
@@ -253,31 +264,54 @@ __global__ __launch_bounds__(256) void vcsr_tile_mma_kernel(
     mma_acc4 d[VEC];
 #pragma unroll
     for (int c = 0; c < VEC; ++c) d[c] = mma_acc4{0.f, 0.f, 0.f, 0.f};
-    auto block = [&](auto n_c, int32_t g0) {
-        constexpr int NG = decltype(n_c)::value;
-        float4 a[NG];
-        V b[NG][4];
+    auto load = [&](auto& x, int32_t g0) {
 #pragma unroll
-        for (int gu = 0; gu < NG; ++gu) {
-            a[gu] = *reinterpret_cast<const float4*>(vp + (int64_t)(g0 + gu) * 256);
+        for (int gu = 0; gu < x.NG; ++gu) {
+            x.a[gu] = *reinterpret_cast<const float4*>(vp + (int64_t)(g0 + gu) * 256);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) b[gu][s] = load_b(16 * (g0 + gu) + 4 * s + kq);
+            for (int s = 0; s < 4; ++s) x.b[gu][s] = load_b(16 * (g0 + gu) + 4 * s + kq);
         }
-        if constexpr (SB) __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](const auto& x) {
 #pragma unroll
-        for (int gu = 0; gu < NG; ++gu)
+        for (int gu = 0; gu < x.NG; ++gu)
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int c = 0; c < VEC; ++c)
                     d[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        reinterpret_cast<const float*>(&a[gu])[s], vec_part<VEC>(b[gu][s], c), d[c],
-                        0, 0, 0);
+                        reinterpret_cast<const float*>(&x.a[gu])[s], vec_part<VEC>(x.b[gu][s], c),
+                        d[c], 0, 0, 0);
+    };
+    auto block = [&](auto n_c, int32_t g0) {
+        MmaGroups<VEC, decltype(n_c)::value> x;
+        load(x, g0);
+        if constexpr (ORD == kMmaAhead) __builtin_amdgcn_sched_barrier(0);
+        multiply(x);
     };
     const int32_t ng = ne / kTileMmaGroup;
     int32_t g0 = 0;
-    if constexpr (SB) {
+    if constexpr (ORD == kMmaAhead) {
         for (; g0 + GU <= ng; g0 += GU) block(std::integral_constant<int, GU>(), g0);
+    } else if constexpr (ORD == kMmaTwo) {
+        const int32_t nb = ng / GU;
+        if (nb > 0) {
+            MmaGroups<VEC, GU> x, y;
+            load(x, 0);
+            int32_t i = 0;
+            for (; i + 2 <= nb; i += 2) {
+                load(y, (i + 1) * GU);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(x);
+                __builtin_amdgcn_sched_barrier(0);
+                load(x, min(i + 2, nb - 1) * GU);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(y);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (i < nb) multiply(x);
+            g0 = nb * GU;
+        }
     } else {
         // Many waves per SIMD, all resident from the start: the SIMD issues
         // oldest first, so with equal work the first waves of a SIMD finish
@@ -346,11 +380,11 @@ __global__ __launch_bounds__(256) void vcsr_tile_mma_kernel(
     }
 }
 
-template <int VEC, bool BUF, int GU, bool SB>
+template <int VEC, bool BUF, int GU, MmaOrder ORD>
 void launch_mma_as(const DeviceFmt& d, dim3 grid, int32_t n_ct, int32_t O, int32_t ld,
                    int32_t accumulate, uint32_t b_bytes, const float* B, float* C, float* partials,
                    hipStream_t st) {
-    hipLaunchKernelGGL((vcsr_tile_mma_kernel<VEC, BUF, GU, SB>), grid, dim3(64 * kMmaWaves), 0, st,
+    hipLaunchKernelGGL((vcsr_tile_mma_kernel<VEC, BUF, GU, ORD>), grid, dim3(64 * kMmaWaves), 0, st,
                        d.tv_n_chunks, n_ct, O, ld, accumulate, b_bytes,
                        reinterpret_cast<const int4*>(d.tv_chunks),
                        reinterpret_cast<const int4*>(d.tv_pieces), d.tv_brow, d.tv_mask, d.tv_val,
@@ -361,25 +395,27 @@ template <int VEC, bool BUF>
 void launch_mma_buf(const DeviceFmt& d, dim3 grid, int64_t waves, int32_t n_ct, int32_t O,
                     int32_t ld, int32_t accumulate, uint32_t b_bytes, const float* B, float* C,
                     float* partials, hipStream_t st) {
-    // Few waves per SIMD (cfg5-like matrices at O <= 192): each wave's loads
-    // in flight bound the time, so its loads go ahead of its MFMAs; with
-    // many, 8 waves per SIMD with interleaved loads hide the latency better.
-    // Measured on the 16K block-sparse matrix (1,024 tiles): O = 32 / 64,
-    // one wave per SIMD, 4 groups with the barrier 27% / 36% faster; O = 128
-    // / 192, two or three, 2 groups with the barrier 20% / 4% faster; O >= 256
-    // slower with the barrier (O = 512: 236 / 186 against 152 us).  Without
-    // it the compiler interleaves loads and MFMAs whatever the block size (42
-    // VGPRs); 8 groups measured 1-4% faster than 4 at O = 256 / 512.
+    // Few waves per SIMD: each wave's loads in flight bound the time, so they
+    // go ahead of the MFMAs; with many, 8 waves per SIMD with interleaved
+    // loads hide the latency better.  us per SpMM on the 16K block-sparse
+    // matrix (1,024 tiles; 100 MB read per launch at O = 64), by waves per
+    // SIMD:
+    //  1 (O = 32 / 64): two sets of 2 groups 17.0 / 22.5, of 1 19.6 / 23.3, of
+    //    4 18.8 / 26.2; 4 groups ahead 18.5 / 24.4.
+    //  2 / 3 (O = 128 / 192): 2 groups ahead 39.1 / 56.7; two sets of 2 42.4 /
+    //    63.0, of 1 40.0 / 59.1.
+    //  4 / 8 (O = 256 / 512): 8 groups mixed 68.4 / 122 (4 groups 1-4% slower);
+    //    two sets of 1 77 / 156.
     const int64_t simds = 4 * (int64_t)device_cus(d.device);
     if (waves <= simds)
-        launch_mma_as<VEC, BUF, 4, true>(d, grid, n_ct, O, ld, accumulate, b_bytes, B, C, partials,
-                                         st);
+        launch_mma_as<VEC, BUF, 2, kMmaTwo>(d, grid, n_ct, O, ld, accumulate, b_bytes, B, C,
+                                            partials, st);
     else if (waves <= 3 * simds)
-        launch_mma_as<VEC, BUF, 2, true>(d, grid, n_ct, O, ld, accumulate, b_bytes, B, C, partials,
-                                         st);
+        launch_mma_as<VEC, BUF, 2, kMmaAhead>(d, grid, n_ct, O, ld, accumulate, b_bytes, B, C,
+                                              partials, st);
     else
-        launch_mma_as<VEC, BUF, 8, false>(d, grid, n_ct, O, ld, accumulate, b_bytes, B, C,
-                                          partials, st);
+        launch_mma_as<VEC, BUF, 8, kMmaMixed>(d, grid, n_ct, O, ld, accumulate, b_bytes, B, C,
+                                              partials, st);
 }
 
 // Columns [0, O) of B and C, whose rows are ld floats apart.
