@@ -205,3 +205,33 @@ def test_csr_wave_long_rows_are_bit_exact(gpu, orc, st, O, off):
     rp2 = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=len(lens)))])
     ref = orc.spmm_f32(len(lens), rp2.astype(np.int32), col[keep], val[keep], B)
     assert np.array_equal(run(rp, outside, val).view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("copies,O", [(2, 8), (2, 16), (2, 31), (2, 50), (2, 128), (2, 257),
+                                      (900, 8), (900, 12), (900, 32), (900, 64), (1800, 8)])
+def test_row_tiles_of_up_to_128_entries_stay_whole(gpu, orc, st, copies, O):
+    """Where rows of 65 to 128 entries hold much of the matrix they are one
+    piece each (only the 129- and 300-entry rows are split), also with 2 and
+    4 work items per wave."""
+    vs = gpu
+    rng = np.random.default_rng(O)
+    lens = [64, 65, 128, 1, 127, 0, 100, 129, 66, 30, 300, 97]
+    N = 1200
+    rp1 = np.concatenate([[0], np.cumsum(lens)])
+    col = np.concatenate([np.sort(rng.choice(N, size=n, replace=False)) for n in lens])
+    val = rng.standard_normal(col.size).astype(np.float32)
+    rp = np.concatenate([[0]] + [rp1[1:] + i * col.size for i in range(copies)]).astype(np.int32)
+    csr = vs.Csr.from_arrays(len(lens) * copies, N, rp, np.tile(col, copies).astype(np.int32),
+                             np.tile(val, copies))
+    fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
+    fmt.set_tile_rows(1)
+    fmt.upload(st)
+    assert fmt.launch_info(O)["split_rows"] == 2 * copies
+    B = vs.gen_dense(O, 0, N, O)
+    ref = np.tile(orc.spmm_f64(len(lens), rp1.astype(np.int32), col.astype(np.int32), val, B),
+                  (copies, 1))
+    C0 = np.ones((csr.M, O), np.float32)
+    for accumulate in (False, True):
+        got = _spmm(vs, fmt, B, C0, 0, st, accumulate)
+        assert_within_tolerance(got - C0 if accumulate else got, ref, csr.row_ptr, csr.val, B,
+                                f"O{O}")

@@ -294,6 +294,7 @@ int vcsr_fmt_upload(vcsr_fmt* fmt, void* stream) {
             d.n_split = (int32_t)(rv.split_rows.size() / 3);
             d.n_partials = rv.n_partials;
             d.tv_R = tv.R;
+            d.tv_piece = tv.piece;
             if (tv.R != 1) d.tv_chunks = upload_array(tv.chunks, st, "upload tile chunks");
             d.tv_items = upload_array(tv_items, st, "upload tile items");
             d.tv_dest = upload_array(tv_dest, st, "upload piece rows");

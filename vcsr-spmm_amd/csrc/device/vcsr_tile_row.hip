@@ -1,8 +1,8 @@
 // vcsr_tile_row.hip - the tile-stationary SpMM on single-row tiles (gfx950).
 // See vcsr_tile.hip for the view and the other tile heights.
 //
-// A wave takes MERGE consecutive work items of the view, at most 64*MERGE
-// entries and 32*MERGE pieces (a piece is a row, or a part of a very long
+// A wave takes MERGE consecutive work items of the view, at most PE*MERGE
+// entries (PE the view's largest piece, 64 or 128) and 32*MERGE pieces (a piece is a row, or a part of a very long
 // one).  The wave is S = 64/LPE streams of LPE lanes; each stream takes an
 // equal run of the wave's entries, and one load instruction fetches one
 // entry's B slice (LPE*VEC columns) for every stream.
@@ -44,10 +44,10 @@ namespace {
 
 constexpr int kWaves = 2;
 
-template <int VEC, int LPE, int MERGE>
+template <int VEC, int LPE, int MERGE, int PE>
 struct RowShape {
     static constexpr int S = 64 / LPE;                          // streams
-    static constexpr int EMAX = tile_piece_entries(1) * MERGE;  // entries per wave
+    static constexpr int EMAX = PE * MERGE;                     // entries per wave
     static constexpr int PMAX = kTileChunkPieces * MERGE;       // pieces per wave
     static constexpr int UT = 2;                                // runs are multiples of this
     static constexpr int IE = EMAX / 64, IP = (PMAX + 63) / 64;
@@ -58,9 +58,9 @@ struct RowShape {
     static constexpr int WORDS = EMAX / 32 + 2;
 };
 
-template <int VEC, int LPE, int MERGE>
+template <int VEC, int LPE, int MERGE, int PE>
 struct RowLds {
-    using Sh = RowShape<VEC, LPE, MERGE>;
+    using Sh = RowShape<VEC, LPE, MERGE, PE>;
     __align__(16) uint2 ent[Sh::LIST];        // (B-row byte offset, value bits)
     typename VecT<VEC>::T xs[Sh::S > 1 ? 64 : 1];  // partial sums of pieces begun earlier
     int32_t dest[Sh::PMAX];                   // row, or ~partial row
@@ -69,7 +69,7 @@ struct RowLds {
     int32_t carry[Sh::S];                     // ... and whether it began in an earlier run
 };
 
-template <int VEC, int LPE, int MERGE, bool BUF, bool ACC>
+template <int VEC, int LPE, int MERGE, int PE, bool BUF, bool ACC>
 __global__ __launch_bounds__(64 * kWaves)
 void vcsr_row_kernel(
     int32_t n_items, int32_t O, int32_t ld, uint32_t b_bytes,
@@ -77,13 +77,13 @@ void vcsr_row_kernel(
     const float2* __restrict__ ent, const float* __restrict__ B, float* __restrict__ C,
     float* __restrict__ partials) {
     using V = typename VecT<VEC>::T;
-    using Sh = RowShape<VEC, LPE, MERGE>;
+    using Sh = RowShape<VEC, LPE, MERGE, PE>;
     constexpr int S = Sh::S, UT = Sh::UT, IE = Sh::IE, IP = Sh::IP;
     // Loads per block: 8; 4 where the rows of C are loaded with them (8 cost
     // two waves per SIMD: uniform 395K x 5, O = 32 65.8 / 74.1 us, power-law
     // 322K, O = 128 167.5 / 178.0; without C's rows 4 are 0-3% slower).
     constexpr int U = ACC && VEC == 4 ? 4 : 8;
-    __shared__ RowLds<VEC, LPE, MERGE> s_lds[kWaves];
+    __shared__ RowLds<VEC, LPE, MERGE, PE> s_lds[kWaves];
 
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = (int)(threadIdx.x & 63);
@@ -91,7 +91,7 @@ void vcsr_row_kernel(
     const int32_t c0 = w * MERGE;
     if (c0 >= n_items) return;
     const int32_t c1 = min(n_items, c0 + MERGE);
-    RowLds<VEC, LPE, MERGE>& L = s_lds[wave];
+    RowLds<VEC, LPE, MERGE, PE>& L = s_lds[wave];
     // Items are {first entry, first piece}.
     const int32_t e0 = uniform(items[c0].x), ne = uniform(items[c1].x) - e0;
     const int32_t p0 = uniform(items[c0].y), np = uniform(items[c1].y) - p0;
@@ -244,13 +244,13 @@ void vcsr_row_kernel(
     }
 }
 
-template <int VEC, int LPE, int MERGE, bool BUF>
+template <int VEC, int LPE, int MERGE, int PE, bool BUF>
 hipError_t launch_shape(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
                         int32_t accumulate, uint32_t b_bytes, float* partials, hipStream_t st) {
     constexpr int per = MERGE * kWaves;
     const dim3 grid((unsigned)(((int64_t)d.tv_n_chunks + per - 1) / per)), block(64 * kWaves);
     auto go = [&](auto acc) {
-        hipLaunchKernelGGL((vcsr_row_kernel<VEC, LPE, MERGE, BUF, decltype(acc)::value>), grid,
+        hipLaunchKernelGGL((vcsr_row_kernel<VEC, LPE, MERGE, PE, BUF, decltype(acc)::value>), grid,
                            block, 0, st, d.tv_n_chunks, O, ld, b_bytes,
                            reinterpret_cast<const int2*>(d.tv_items), d.tv_dest,
                            reinterpret_cast<const float2*>(d.tv_val), B, C, partials);
@@ -269,12 +269,19 @@ hipError_t launch_vcsr_row_tiles(const DeviceFmt& d, const float* B, int32_t O, 
                                  hipStream_t st) {
     if (d.tv_n_chunks <= 0) return hipSuccess;
     if (b_bytes >= kBufferLimit) {
-        if (O < 4) return launch_shape<1, 64, 1, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
-        return launch_shape<4, 64, 1, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
+        constexpr int PE = tile_piece_entries(1);
+        if (O < 4)
+            return launch_shape<1, 64, 1, PE, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
+        return launch_shape<4, 64, 1, PE, false>(d, B, O, ld, C, accumulate, 0u, partials, st);
     }
+    auto go_pe = [&](auto vec, auto lpe, auto merge, auto pe) {
+        return launch_shape<decltype(vec)::value, decltype(lpe)::value, decltype(merge)::value,
+                            decltype(pe)::value, true>(d, B, O, ld, C, accumulate,
+                                                       (uint32_t)b_bytes, partials, st);
+    };
     auto go = [&](auto vec, auto lpe, auto merge) {
-        return launch_shape<decltype(vec)::value, decltype(lpe)::value, decltype(merge)::value, true>(
-            d, B, O, ld, C, accumulate, (uint32_t)b_bytes, partials, st);
+        return d.tv_piece > kTileRowPiece ? go_pe(vec, lpe, merge, I<tile_piece_entries(1)>())
+                                          : go_pe(vec, lpe, merge, I<kTileRowPiece>());
     };
     // Work items per wave.  us per SpMM, three formats in turn (the view comes
     // from beyond L2), 1 / 2 / 4 items:

@@ -164,7 +164,7 @@ std::vector<std::vector<Tile>> make_tiles(const RowLists& rl, int32_t M,
 // it is moved into the run whose eighth of B holds its middle column,
 // sorted by that column among the run's other items, so that the XCD's L2
 // holds its B rows.  Run sizes stay those of the original order.
-// Rows cut into 8 or more pieces (more than 448 entries) are moved;
+// Rows cut into 8 or more pieces of 64 (more than 448 entries) are moved;
 // power-law 322K matrix: O = 8 / 32 / 128 25.6 / 35.9 / 107.8 ->
 // 24.9 / 33.9 / 94.8 us per SpMM.  Moving the pieces of every split row
 // (more than 64 entries) gave 25.3 / 34.7 / 98.5, from 4 or 16 pieces up
@@ -172,7 +172,7 @@ std::vector<std::vector<Tile>> make_tiles(const RowLists& rl, int32_t M,
 // / 98.2.
 void order_long_pieces_by_column(TileView& tv, int32_t N, int nthreads) {
     constexpr int kSeg = 8;
-    constexpr int32_t kMinPieces = 8;
+    const int32_t kMinPieces = 512 / tv.piece;
     const int32_t nc = (int32_t)(tv.chunks.size() / 4);
     if (tv.R != 1 || nc < 4 * kSeg || N <= 0 || tv.split.empty()) return;
     std::unordered_map<int32_t, int32_t> npc;
@@ -217,6 +217,7 @@ void order_long_pieces_by_column(TileView& tv, int32_t N, int nthreads) {
     while (f < fixed.size()) order.push_back(fixed[f++]);
     TileView out;
     out.R = tv.R;
+    out.piece = tv.piece;
     out.n_tiles = tv.n_tiles;
     out.split = tv.split;
     out.n_partial_rows = tv.n_partial_rows;
@@ -396,7 +397,15 @@ TileView make_tile_view(const Vcsr& v, int32_t R, int nthreads, bool fixed) {
     // work items of its own (cut into equal pieces of at most
     // tile_piece_entries that write partial sums when it needs more than
     // one); shorter tiles are packed in row order.
-    const int32_t cap_e = tile_chunk_entries(R), cap_p = tile_piece_entries(R);
+    int32_t cap_p = tile_piece_entries(R);
+    if (R == 1) {
+        int64_t mid = 0;
+        for (const Tile& x : tiles)
+            if (x.nent > kTileRowPiece && x.nent <= cap_p) mid += x.nent;
+        if (8 * mid < E) cap_p = kTileRowPiece;
+    }
+    tv.piece = cap_p;
+    const int32_t cap_e = tile_chunk_entries(R);
     tv.pieces.reserve(4 * tiles.size() + 4 * (size_t)(E / cap_p));
     tv.chunks.reserve(4 * (size_t)(2 * E / cap_e) + 64);
     int64_t ce0 = 0, cent = 0;

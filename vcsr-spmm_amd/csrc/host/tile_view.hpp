@@ -36,16 +36,20 @@ constexpr int32_t tile_chunk_entries(int32_t R) { return 32 * R; }
 // work item of its own.
 constexpr int32_t kTileMmaRows = 16;
 constexpr int32_t kTileMmaGroup = 16;
-// Entries of one piece of a tile longer than half a work item (it gets work
-// items of its own): at least 64, so a long row is cut into fewer pieces
-// (and partial rows for the reduce kernel); larger pieces for single-row
-// tiles measured slower where several work items share a wave (power-law
-// 322K matrix, O = 8: 128 / 256 entries 35.1 / 48.9 against 29.2 us: the
-// wave's LDS list grows with them and fewer waves fit).  The kernel's LDS
-// list holds this many entries per merged work item.
+// Most entries of one piece of a tile longer than half a work item (it gets
+// work items of its own).  A tile cut into pieces pays for partial rows and
+// the reduce kernel, so tiles of up to 128 entries stay whole: banded 60K
+// matrix with 78 entries a row, O = 128, blocks of 2 / 3 rows 86 / 42.5 us
+// with pieces of 64 / 96, 48.3 / 35.4 with 128.
+// Single-row tiles: 128 only where rows of 65 to 128 entries hold an eighth of
+// all entries (TileView::piece), else kTileRowPiece = 64, since the wave's LDS
+// list grows with it and fewer waves fit: banded 60K matrix with 70 entries a
+// row, O = 8 / 50 / 128 27.8 / 60.6 / 115 us with 64, 19.9 / 45.9 / 74.9 with
+// 128; power-law 322K matrix, O = 8 22.2 / 23.6.
 constexpr int32_t tile_piece_entries(int32_t R) {
-    return R == kTileMmaRows ? 1024 : (32 * R > 64 ? 32 * R : 64);
+    return R == kTileMmaRows ? 1024 : (32 * R > 128 ? 32 * R : 128);
 }
+constexpr int32_t kTileRowPiece = 64;
 // Slot indices stored per entry for tile height R (a power of two, so that
 // an entry's slots and staged values are one aligned vector).
 constexpr int32_t tile_slot_stride(int32_t R) {
@@ -83,6 +87,7 @@ constexpr int32_t kTileRowBlock = 4096;
 
 struct TileView {
     int32_t R = 1;                // accumulator rows per tile: 1, 2, 3, 4, 8 or 16
+    int32_t piece = 0;            // most entries of a piece
     int32_t n_tiles = 0;
     // Work items, 4 ints each: first entry, end entry, first piece, end piece.
     std::vector<int32_t> chunks;
