@@ -63,6 +63,8 @@ CONFIGS = {
 # Sources whose code decides the traffic of the dominant (tile) kernel; the
 # counter sets in profiles/traffic.json record their hash.
 TRAFFIC_SOURCES = ("vcsr-spmm_amd/csrc/device/vcsr_tile.hip",
+                   "vcsr-spmm_amd/csrc/device/vcsr_tile_row.hip",
+                   "vcsr-spmm_amd/csrc/device/vcsr_tile_tall.hip",
                    "vcsr-spmm_amd/csrc/device/vecops.hpp",
                    "vcsr-spmm_amd/csrc/device/common.hpp",
                    "vcsr-spmm_amd/csrc/host/tile_view.cpp",

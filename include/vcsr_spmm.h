@@ -283,8 +283,8 @@ int vcsr_tile_mfma_work(const vcsr_fmt* fmt, int32_t O, int64_t* ops, int32_t* f
  * B-row slice loads per column tile), whether its tiles run on the FP32
  * matrix cores, floats per lane, column slices (one launch each) and their
  * width, reduce-kernel launches and split rows, and the partial-row floats
- * of scratch; other kernels report only `kernel`.  As launched on 16-byte
- * aligned B and C.  No reference counterpart. */
+ * of scratch; other kernels report only `kernel`.  The same for any
+ * alignment of B and C.  No reference counterpart. */
 typedef struct {
     int32_t kernel;
     int32_t tile_rows;

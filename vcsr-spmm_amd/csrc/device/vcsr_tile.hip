@@ -11,36 +11,13 @@
 // the B-row traffic through the vector memory pipe, the limiting resource of
 // a row-stationary SpMM, by the block height.
 //
-// This file holds the single-row kernel, the matrix-core kernel of 16-row
-// tiles, the reduce of split tiles and the launcher; tiles of 2 to 8 rows are
-// in vcsr_tile_tall.hip.
+// This file holds the matrix-core kernel of 16-row tiles, the reduce of split
+// tiles and the launcher; single-row tiles are in vcsr_tile_row.hip, tiles of
+// 2 to 8 rows in vcsr_tile_tall.hip.
 //
-// Single-row work item (one wave): MERGE consecutive work items of the view,
-// each a run of tile pieces with at most tile_piece_entries(1) entries
-// (host/tile_view.hpp).
-// Phase 1 (lane per entry): read the entry's record (value and B row, stored
-// together, so these are coalesced loads, not gathers from the VCSR value
-// array) and stage (B-row byte offset, value) in the wave's LDS list.
-// Phase 2, per column tile of LPE*VEC columns: the wave is S = 64/LPE
-// streams of LPE lanes; one load instruction serves one entry of every
-// stream.
-//  - Several pieces: each stream takes a contiguous run of whole pieces
-//    (balanced by entry count), accumulates the piece's row and stores it
-//    when its last entry has been applied.  No cross-lane reduction.  With
-//    several work items per wave every stream gets an equal run of entries
-//    instead; a piece cut between runs is finished by the stream that began
-//    it, from the later streams' partial sums in LDS.
-//  - One piece (a long row): the streams interleave over its entries, whose
-//    list is padded to whole blocks, and their sums are added with
-//    cross-lane shuffles before the store.
-// Loads are issued in blocks of U back to back before the block's FMAs; B is
-// read with raw buffer loads whose range check turns out-of-range offsets
-// into zeros, so inactive lanes and placeholder entries need no branch.
-//
-// The host launcher runs one launch per column slice of at most 256
-// columns (128 when B is over 512 MB) for taller tiles and for single-row
-// tiles with 16-byte vectors, and for any vector width when tiles are split
-// (their partial rows are one slice wide).
+// The host launcher runs one launch per column slice of at most 256 columns
+// (128 when B is over 512 MB) for tiles of up to 8 rows, and for 16-row tiles
+// when some are split (their partial rows are one slice wide).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>

@@ -52,18 +52,6 @@ __device__ __forceinline__ float4 shfl_xor_vec(float4 x, int m) {
                        __shfl_xor(x.w, m));
 }
 
-// Non-temporal stores (written once, not read again by this kernel): they do
-// not displace B rows from L2.
-typedef float nt_float2 __attribute__((ext_vector_type(2)));
-typedef float nt_float4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void store_nt(float* p, float x) { __builtin_nontemporal_store(x, p); }
-__device__ __forceinline__ void store_nt(float2* p, float2 x) {
-    __builtin_nontemporal_store(__builtin_bit_cast(nt_float2, x), reinterpret_cast<nt_float2*>(p));
-}
-__device__ __forceinline__ void store_nt(float4* p, float4 x) {
-    __builtin_nontemporal_store(__builtin_bit_cast(nt_float4, x), reinterpret_cast<nt_float4*>(p));
-}
-
 // The same vectors in memory at any 4-byte boundary (rows of B and C whose
 // length is not a multiple of the vector): gfx950's wide loads and stores
 // need dword alignment only.
@@ -76,6 +64,8 @@ __device__ __forceinline__ float2 load_mem(const float* p, float2) {
 __device__ __forceinline__ float4 load_mem(const float* p, float4) {
     return __builtin_bit_cast(float4, *reinterpret_cast<const mem_float4*>(p));
 }
+// NT: non-temporal (written once, not read again by the kernel), so that the
+// stores do not displace B rows from L2.
 template <bool NT>
 __device__ __forceinline__ void store_mem(float* p, float x) {
     if constexpr (NT) __builtin_nontemporal_store(x, p);
