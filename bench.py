@@ -409,7 +409,7 @@ def extra_point(vs, orc, st, w, algo, steps, warmup, nthreads):
     if fmt is not None and algo in ("vcsr", "tile"):
         li = fmt.launch_info(w.O, vs.KERNEL_AUTO)
         out["timed_kernel"] = ("vcsr_tile_mma_kernel (16-row tiles on FP32 MFMA)"
-                               if li["matrix_cores"] else "vcsr_tile_kernel (row-tile view)")
+                               if li["matrix_cores"] else "vcsr_row_kernel / vcsr_tall_kernel (row-tile view)")
         out["reduce_launches"] = li["reduce_launches"]
     m = mfma_report(vs, fmt, algo, w, cfg_tileK, kernel_ms)
     if m is not None:
@@ -524,7 +524,7 @@ def main():
         li = fmt.launch_info(O, vs.KERNEL_TILE)
         config.update({
             "timed_kernel": ("vcsr_tile_mma_kernel (16-row tiles on FP32 MFMA)"
-                             if li["matrix_cores"] else "vcsr_tile_kernel (row-tile view)"),
+                             if li["matrix_cores"] else "vcsr_row_kernel / vcsr_tall_kernel (row-tile view)"),
             "tile_rows": li["tile_rows"], "tiles": li["tiles"], "entries": li["entries"],
             "column_slices": li["column_slices"], "slice_cols": li["slice_cols"],
             "reduce_launches": li["reduce_launches"],
