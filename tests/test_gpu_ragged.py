@@ -207,6 +207,37 @@ def test_csr_wave_long_rows_are_bit_exact(gpu, orc, st, O, off):
     assert np.array_equal(run(rp, outside, val).view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("O", [1, 3, 7, 8, 9, 13, 16, 17, 20, 32, 33, 47, 64, 65, 127, 128, 129, 200,
+                               256, 257, 516])
+def test_csr_wave_short_rows_are_bit_exact(gpu, orc, st, O, off):
+    """The plain-CSR kernel where no row is long (no barrier in a block):
+    lengths around the blocks of 8 loads and the 32 and 64 entries staged at
+    a time, matrices that end inside a wave and a block, a single row, and
+    inf and NaN in the columns next to those that idle lanes read again."""
+    vs = gpu
+    rng = np.random.default_rng(7 * O)
+    N = 300
+    base = [0, 1, 7, 8, 9, 0, 15, 16, 17, 31, 32, 33, 5, 63, 64, 65, 100, 127, 128, 2]
+    for M in (1, 3, 17, 33, 61, 100):
+        lens = [base[(3 * i + M) % len(base)] for i in range(M)]
+        rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        col = rng.integers(0, N, rp[-1]).astype(np.int32)
+        val = rng.standard_normal(rp[-1]).astype(np.float32)
+        B = vs.gen_dense(O, 0, N, O)
+        if M == 61:
+            B[3, O - 1], B[100, 0], B[299, O // 2] = np.inf, np.nan, -np.inf
+        d = [vs.DeviceArray.from_numpy(x if x.size else np.zeros(1, x.dtype), st)
+             for x in (rp, col, val)]
+        dB = _Shifted(vs, B, off, st)
+        dC = _Shifted(vs, np.full((M, O), 5.0, np.float32), off, st)
+        vs.run_csr_wave_spmm_gpu(M, N, *d, dB, O, dC, st, timed=True)
+        got, ref = dC.numpy(), orc.spmm_f32(M, rp, col, val, B)
+        nan = np.isnan(ref)
+        assert np.array_equal(np.isnan(got), nan), M
+        assert np.array_equal(got.view(np.uint32)[~nan], ref.view(np.uint32)[~nan]), M
+
+
 @pytest.mark.parametrize("copies,O", [(2, 8), (2, 16), (2, 31), (2, 50), (2, 128), (2, 257),
                                       (900, 8), (900, 12), (900, 32), (900, 64), (1800, 8)])
 def test_row_tiles_of_up_to_128_entries_stay_whole(gpu, orc, st, copies, O):

@@ -11,10 +11,14 @@
 // is one chain of fused multiply-adds in the row's entry order (the CPU
 // loop's bits), so a row's entries cannot be split between lanes.
 //  - Rows of up to kLongRow entries: a stream stages CH of its row's entries
-//    at a time (B-row byte offset and value) in the wave's LDS, the next
-//    ones' loads in flight meanwhile, and applies them in blocks of U loads
-//    issued back to back; B is read with raw buffer loads whose range check
-//    returns zeros for lanes past the row's end or past O.
+//    at a time (B-row byte offset and value) in the wave's LDS (one row a
+//    wave: in its lanes' registers), the next ones' loads in flight meanwhile,
+//    and applies them in blocks of U loads issued back to back; B is read with
+//    raw buffer loads whose range check returns zeros past the row's end.
+//    Bound by the waves' chain of loads (row, entries, B rows) where rows are
+//    short, by the L2-to-CU path where they are not: as little as possible
+//    stands before the first load, and the registers leave 7 or 8 waves per
+//    SIMD.
 //  - Longer rows bound the kernel by their own latency (8 loads in flight a
 //    stream), so the block's four waves take them together afterwards: the
 //    waves take turns of LU entries each, all of a turn's B rows loaded ahead
@@ -58,40 +62,56 @@ __global__ __launch_bounds__(64 * kWaveRowsWaves) void csr_wave_kernel(int32_t M
                                                        float* __restrict__ C) {
     using V = typename VecT<VEC>::T;
     constexpr int S = 64 / LPE;                   // rows per wave
+    constexpr int NR = kWaveRowsWaves * S;        // ... and block
     constexpr int U = 8;                          // loads per block
     constexpr int NC = LPE >= 32 ? 1 : 32 / LPE;  // entries a lane stages at a time
     constexpr int CH = LPE * NC;                  // ... and a stream
-    constexpr int PAD = 1;                        // keeps the streams' reads in different banks
-    __shared__ uint2 s_ent[kWaveRowsWaves][S * (CH + PAD)];
-    __shared__ int2 s_row[kWaveRowsWaves * S];    // {first entry, entries} of the block's rows
+    constexpr int LS = CH + 4;                    // keeps the streams' reads in different banks
+    __shared__ __align__(16) uint32_t s_off[kWaveRowsWaves][S * LS];
+    __shared__ __align__(16) float s_val[kWaveRowsWaves][S * LS];
     __shared__ __align__(16) float s_sum[64 * 4];
 
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = (int)(threadIdx.x & 63), sub = lane / LPE, kl = lane % LPE;
-    const int64_t row0 = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * (kWaveRowsWaves * S);
-    const int64_t row = row0 + wave * S + sub;
-    const bool rowok = row < M;
-    const int32_t p0 = rowok ? rowptr[row] : 0, nrow = rowok ? rowptr[row + 1] - p0 : 0;
-    if (kl == 0) s_row[wave * S + sub] = make_int2(p0, nrow);
-    __syncthreads();
+    const int64_t row0 = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * NR;
+    // The block's rows, one a lane, read by every wave for itself beside its
+    // own: a block without long rows has no barrier.  Rows past M repeat the
+    // last one.
+    const int32_t rows = (int32_t)min((int64_t)NR, M - row0), slot = wave * S + sub;
+    const bool rowok = slot < rows;
+    const int32_t* ra = rowptr + row0 + min(slot, rows - 1);
+    const int32_t* rb = rowptr + row0 + min(lane & (NR - 1), rows - 1);
+    const int32_t p0 = ra[0], p1 = ra[1], bp = rb[0], bn = rb[1] - bp;
+    const uint64_t longs = __ballot(bn > kLongRow) & ((2ull << (rows - 1)) - 1ull);
     // The block takes its long rows together only if few rows stand out:
     // otherwise the rows' streams, side by side, are the faster way (16x16
     // blocks, 51 a row, O = 100 all together 708 us, side by side 222).
-    constexpr int FEW = S >= 4 ? 4 : 2;
-    int32_t most = lane < kWaveRowsWaves * S ? s_row[lane].y : 0, sum = min(most, 1 << 24);
+    bool together = false;
+    if (longs != 0) {
+        constexpr int FEW = S >= 4 ? 4 : 2;
+        int32_t most = lane < rows ? bn : 0, sum = min(most, 1 << 24);
 #pragma unroll
-    for (int sh = 1; sh < 64; sh <<= 1) {
-        most = max(most, __shfl_xor(most, sh));
-        sum += __shfl_xor(sum, sh);
+        for (int sh = 1; sh < 64; sh <<= 1) {
+            most = max(most, __shfl_xor(most, sh));
+            sum += __shfl_xor(sum, sh);
+        }
+        together = uniform(sum) / FEW <= uniform(most);
     }
-    const bool together = uniform(most) > kLongRow && uniform(sum) / FEW <= uniform(most);
-    const bool islong = together && nrow > kLongRow;
-    const int32_t n = islong ? 0 : nrow;
-    int32_t nmax = n;
+    // One row a wave: the block's waves start their rows together, so that
+    // neighbouring rows find each other's B rows in the L1 (banded 120K
+    // matrix with 24 entries a row, O = 256 153.4 -> 149.3 us).
+    if constexpr (LPE == 64) __syncthreads();
+    const int32_t limit = together ? kLongRow : INT32_MAX;
+    const bool mine = rowok && p1 - p0 <= limit;  // this stream's row, unless the block takes it
+    const int32_t n = mine ? p1 - p0 : 0;
+    int32_t nmax = 0;
 #pragma unroll
-    for (int sh = LPE; sh < 64; sh <<= 1) nmax = max(nmax, __shfl_xor(nmax, sh));
-    nmax = uniform(nmax);
-    uint2* le = s_ent[wave] + sub * (CH + PAD);
+    for (int i = 0; i < S; ++i) {
+        const int32_t x = __builtin_amdgcn_readlane(bn, wave * S + i);
+        nmax = max(nmax, x <= limit ? x : 0);
+    }
+    uint32_t* lo = s_off[wave] + sub * LS;
+    float* lv = s_val[wave] + sub * LS;
     const uint32_t row_bytes = (uint32_t)O * 4u;
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), (short)0, (int)b_bytes,
@@ -102,63 +122,100 @@ __global__ __launch_bounds__(64 * kWaveRowsWaves) void csr_wave_kernel(int32_t M
         return (uint32_t)cj < (uint32_t)N ? (BUF ? (uint32_t)cj * row_bytes : (uint32_t)cj) : kNoRow;
     };
 
-    for (int32_t k0 = 0; k0 < O; k0 += LPE * VEC) {
+    // Narrower shapes hold all columns at once: no loop, whose invariants
+    // (addresses) would be kept in registers.
+    const int32_t kend = LPE == 64 ? O : LPE * VEC;
+    for (int32_t k0 = 0; k0 < kend; k0 += LPE * VEC) {
         const int32_t k = k0 + kl * VEC;
         const bool kok = k < O;
-        const uint32_t koff = (uint32_t)vec_col<VEC>(k, O) * 4u;
+        const int32_t kc = vec_col<VEC>(k, O);
+        // Lanes past O read their row's last vector once more.  Masking them
+        // with offsets past the end of B costs twice the time of the loads
+        // (banded 62K matrix, O = 1 / 7 / 9: 19.8 / 22.2 / 34.0 us so masked,
+        // 10.8 / 13.0 / 15.1 now).
+        auto load_b = [&](uint32_t off, int32_t c) -> V {
+            if constexpr (BUF) return load_b_buf<VEC>(rsrc, off + (uint32_t)c * 4u);
+            else return off != kNoRow ? load_mem(B + (int64_t)off * O + c, V()) : zero_vec(V());
+        };
         V acc = zero_vec(V());
         int32_t cj[NC];
         float a[NC];
         auto fetch = [&](int32_t c0) {
 #pragma unroll
             for (int q = 0; q < NC; ++q) {
+                if (q > 0 && c0 + q * LPE >= nmax) break;
                 const int32_t i = c0 + q * LPE + kl;
                 cj[q] = i < n ? col[p0 + i] : -1;
                 a[q] = i < n ? val[p0 + i] : 0.f;
             }
         };
         fetch(0);
-        for (int32_t c0 = 0; c0 < nmax; c0 += CH) {
+        if constexpr (LPE == 64) {
+            // One row a wave: the entries stay in its lanes' registers.
+            for (int32_t c0 = 0; c0 < nmax; c0 += CH) {
+                const uint32_t off = b_off(cj[0]);
+                const float av = off == kNoRow ? 0.f : a[0];
+                if (c0 + CH < nmax) fetch(c0 + CH);
+                const int32_t cnt = min(CH, nmax - c0);
+                for (int32_t j0 = 0; j0 < cnt; j0 += U) {
+                    uint32_t o[U];
+                    float x[U];
+                    V b[U];
 #pragma unroll
-            for (int q = 0; q < NC; ++q) {
-                const uint32_t off = b_off(cj[q]);
-                le[q * LPE + kl] =
-                    make_uint2(off, off == kNoRow ? 0u : __builtin_bit_cast(uint32_t, a[q]));
-            }
-            if (c0 + CH < nmax) fetch(c0 + CH);
-            wave_sync();
-            const int32_t cnt = min(CH, nmax - c0);
-            for (int32_t j0 = 0; j0 < cnt; j0 += U) {  // CH is a multiple of U
-                uint2 e[U];
-                V b[U];
+                    for (int u = 0; u < U; ++u)
+                        o[u] = (uint32_t)__builtin_amdgcn_readlane((int)off, j0 + u);
 #pragma unroll
-                for (int u = 0; u < U; ++u) e[u] = le[j0 + u];
+                    for (int u = 0; u < U; ++u) b[u] = load_b(o[u], kc);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    if constexpr (BUF) {
-                        b[u] = load_b_buf<VEC>(rsrc, (e[u].x + koff) | (kok ? 0u : kNoRow));
-                    } else {
-                        const bool live = e[u].x != kNoRow && kok;
-                        b[u] = live ? load_mem(B + (int64_t)e[u].x * O + koff / 4, V())
-                                    : zero_vec(V());
-                    }
+                    for (int u = 0; u < U; ++u)
+                        x[u] = __builtin_bit_cast(
+                            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, av), j0 + u));
+#pragma unroll
+                    for (int u = 0; u < U; ++u) fma_vec(acc, x[u], b[u]);
                 }
-#pragma unroll
-                for (int u = 0; u < U; ++u) fma_vec(acc, __builtin_bit_cast(float, e[u].y), b[u]);
             }
-            wave_sync();
+        } else {
+            for (int32_t c0 = 0; c0 < nmax; c0 += CH) {
+#pragma unroll
+                for (int q = 0; q < NC; ++q) {
+                    if (q > 0 && c0 + q * LPE >= nmax) break;
+                    const uint32_t off = b_off(cj[q]);
+                    lo[q * LPE + kl] = off;
+                    lv[q * LPE + kl] = off == kNoRow ? 0.f : a[q];
+                }
+                if (c0 + CH < nmax) fetch(c0 + CH);
+                wave_sync();
+                const int32_t cnt = min(CH, nmax - c0);
+                for (int32_t j0 = 0; j0 < cnt; j0 += U) {  // CH is a multiple of U
+                    uint32_t o[U];
+                    float x[U];
+                    V b[U];
+#pragma unroll
+                    for (int u = 0; u < U; u += 4)
+                        *reinterpret_cast<uint4*>(o + u) = *reinterpret_cast<const uint4*>(lo + j0 + u);
+#pragma unroll
+                    for (int u = 0; u < U; ++u) b[u] = load_b(o[u], kc);
+#pragma unroll
+                    for (int u = 0; u < U; u += 4)
+                        *reinterpret_cast<float4*>(x + u) = *reinterpret_cast<const float4*>(lv + j0 + u);
+#pragma unroll
+                    for (int u = 0; u < U; ++u) fma_vec(acc, x[u], b[u]);
+                }
+                wave_sync();
+            }
         }
-        if (rowok && !islong && kok) store_cols<VEC, false>(C + row * O, k, O, acc, false);
+        if (mine && kok)
+            store_cols<VEC, false>(C + (row0 + wave * S) * O + sub * O, k, O, acc, false);
     }
 
     // Long rows.
     if (!together) return;
     constexpr int LV = LongShape<VEC, LPE>::LV, LU = LongShape<VEC, LPE>::LU;
     using W = typename VecT<LV>::T;
-    for (int slot = 0; slot < kWaveRowsWaves * S; ++slot) {
-        const int32_t nl = uniform(s_row[slot].y);
-        if (nl <= kLongRow) continue;
-        const int32_t pl = uniform(s_row[slot].x), turns = (nl + LU - 1) / LU;
+    for (uint64_t left = longs; left != 0; left &= left - 1) {
+        const int slot = __builtin_ctzll(left);  // of the block's rows
+        const int32_t nl = __builtin_amdgcn_readlane(bn, slot);
+        const int32_t pl = __builtin_amdgcn_readlane(bp, slot), turns = (nl + LU - 1) / LU;
         for (int32_t k0 = 0; k0 < O; k0 += 64 * LV) {
             const int32_t k = k0 + lane * LV;
             const bool kok = k < O;
