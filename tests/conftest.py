@@ -94,6 +94,49 @@ def assert_within_tolerance(C, ref64, row_ptr, val, B, what=""):
     return rel, worst
 
 
+def tile_csr(vs, one, copies):
+    """`copies` of a matrix below each other."""
+    rp = np.concatenate([[0]] + [one.row_ptr[1:].astype(np.int64) + i * one.nnz
+                                 for i in range(copies)]).astype(np.int32)
+    return vs.Csr.from_arrays(one.M * copies, one.N, rp, np.tile(one.col, copies),
+                              np.tile(one.val, copies))
+
+
+def work_items(csr):
+    """(work items, pieces, entries, largest piece) of the single-row view: rows
+    of more than 16 entries take items of their own, cut into pieces of at most
+    64 entries (128 where rows of 65 to 128 hold an eighth of all entries);
+    shorter ones (one placeholder for an empty row) are packed in row order
+    into items of at most 32 entries and 32 rows."""
+    n = np.maximum(np.diff(csr.row_ptr), 1)
+    piece = 128 if 8 * n[(n > 64) & (n <= 128)].sum() >= n.sum() else 64
+    items = pieces = entries = rows = 0
+    for x in n.tolist():
+        if x > 16:
+            items += (rows > 0) + -(-x // piece)
+            pieces += -(-x // piece)
+            entries = rows = 0
+            continue
+        if entries + x > 32 or rows == 32:
+            items += rows > 0
+            entries = rows = 0
+        entries, rows, pieces = entries + x, rows + 1, pieces + 1
+    return items + (rows > 0), pieces, int(n.sum()), piece
+
+
+def items_per_wave(items, pieces, O):
+    """Work items a wave of the single-row kernel takes at width O on 256
+    compute units (vcsr_tile_row.hip), its 16-lane shape aside."""
+    simds, single = 1024, pieces < 2 * items
+    if O <= 8:
+        return 4 if items >= (16 if single else 24) * simds else \
+            2 if not single and items >= 5 * simds else 1
+    if O <= 32:
+        return 4 if single and items >= 16 * simds else 2 if items >= 5 * simds else 1
+    least = 16 if O <= 64 else 48 if O <= 128 else 64
+    return 2 if single and items >= least * simds else 1
+
+
 def random_csr(rng, M, N, density=0.05, dup_rate=0.0, empty_rows=0.0, max_row=None):
     """Random COO arrays (rows, cols, vals), rows ascending and each row's
     columns shuffled, duplicates allowed: the unsorted input the reference's

@@ -16,8 +16,8 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from conftest import (assert_within_tolerance, block_csr, host_threads, random_csr,
-                      row_abs_sums)
+from conftest import (assert_within_tolerance, block_csr, host_threads, items_per_wave, random_csr,
+                      row_abs_sums, tile_csr, work_items)
 
 pytestmark = pytest.mark.gpu
 
@@ -416,17 +416,22 @@ _EQ_PATTERN = [0, 1, 3, 17, 2, 150, 5, 64, 65, 9, 400, 1, 1, 30, 0, 12, 2, 2, 90
 @pytest.mark.parametrize("O", [1, 4, 8, 32])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_equal_runs_of_single_row_tiles(gpu, orc, st, O, accumulate):
-    """Single-row tiles at O <= 8 and O = 32 run four work items per wave,
-    each of 8 streams taking an equal run of the wave's entries; a piece cut
-    between runs is finished by the stream that began it from the later
+    """Single-row tiles at O <= 8 and O = 32 run one to four work items per
+    wave, each of 8 streams taking an equal run of the wave's entries; a piece
+    cut between runs is finished by the stream that began it from the later
     streams' partial sums.  Rows of every length, pieces spanning up to
-    seven runs, and a matrix with fewer entries than streams (empty runs):
-    all of C within the north-star bounds, in both C modes, the same bits
-    on a second call."""
+    seven runs, a matrix with fewer entries than streams (empty runs), and one
+    large enough (over 16 work items per SIMD) for four items per wave, whose
+    rows of 65 and 90 entries are cut (such rows hold less than an eighth of
+    its entries): all of C within the north-star bounds, in both C modes, the
+    same bits on a second call."""
     vs = gpu
     rng = np.random.default_rng(500 + O)
+    one = _row_lengths_csr(vs, rng, _EQ_PATTERN + [450], 1000)
     cases = [_row_lengths_csr(vs, rng, _EQ_PATTERN * 12, 1000),
-             _row_lengths_csr(vs, rng, [1, 0, 2, 0, 1], 9)]
+             _row_lengths_csr(vs, rng, [1, 0, 2, 0, 1], 9), tile_csr(vs, one, 640)]
+    items, pieces, _, piece = work_items(cases[2])
+    assert piece == 64 and items_per_wave(items, pieces, O) == 4
     for csr in cases:
         print(f"equal runs M={csr.M} nnz={csr.nnz} O={O} accumulate={accumulate}", flush=True)
         fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
@@ -434,6 +439,8 @@ def test_equal_runs_of_single_row_tiles(gpu, orc, st, O, accumulate):
         fmt.upload(st)
         li = fmt.launch_info(O, vs.KERNEL_TILE)
         assert li["tile_rows"] == 1 and (li["vec"] == 4 if O == 32 else li["vec"] == 1)
+        if csr.M == one.M * 640:
+            assert li["split_rows"] == 5 * 640  # 150, 65, 400, 90 and 450 entries
         B = vs.gen_dense(O + 3, 0, csr.N, O)
         C0 = rng.uniform(-2, 2, size=(csr.M, O)).astype(np.float32)
         ref64 = orc.spmm_f64(csr.M, csr.row_ptr, csr.col, csr.val, B)
@@ -448,9 +455,8 @@ def test_equal_runs_of_single_row_tiles(gpu, orc, st, O, accumulate):
 def test_equal_runs_nonfinite_b(gpu, orc, st, O):
     """Inf and NaN in B rows read by long rows (pieces cut between streams'
     runs, and split rows) and by short ones reach exactly the C entries the
-    reference's loop reaches: the stream that finishes a piece from other
-    streams' partial sums recomputes it with the presence bits when the sum
-    is not finite."""
+    reference's loop reaches: a row holds only entries it has, and entries
+    that pad a stream's run read zeros."""
     vs = gpu
     rng = np.random.default_rng(900 + O)
     csr = _row_lengths_csr(vs, rng, _EQ_PATTERN * 6, 600)

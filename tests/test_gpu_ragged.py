@@ -4,6 +4,7 @@ boundary, the last vector of a row moved back to end with it."""
 import numpy as np
 import pytest
 
+from conftest import items_per_wave, tile_csr, work_items
 from test_gpu_parity import _block_csr, _Shifted, assert_within_tolerance
 
 pytestmark = pytest.mark.gpu
@@ -126,18 +127,19 @@ _ROW_WIDTHS = [1, 3, 7, 8, 9, 16, 17, 30, 32, 33, 50, 64, 65, 127, 129, 255, 257
 
 @pytest.mark.parametrize("copies,O,off", [(c, O, off) for c in (1, 40) for O in _ROW_WIDTHS
                                           for off in (0, 4)] +
+                         [(120, O, 0) for O in _ROW_WIDTHS if O < 33] +
                          [(600, O, 0) for O in _ROW_WIDTHS if O < 130])
 def test_row_tiles_any_width(gpu, orc, st, copies, O, off):
-    """Single-row tiles at every width class and its edges; 40 and 600
-    copies of the matrix below each other take 1, 2 and 4 work items per
-    wave.  C = A*B and C += A*B against the oracle, twice the same bits."""
+    """Single-row tiles at every width class and its edges; 40, 120 and 600
+    copies of the matrix below each other: waves of 1, 2 and 4 work items.
+    C = A*B and C += A*B against the oracle, twice the same bits."""
     vs = gpu
     rng = np.random.default_rng(O)
     one = _mixed_rows(vs, rng)
-    rp = np.concatenate([[0]] + [one.row_ptr[1:].astype(np.int64) + i * one.nnz
-                                 for i in range(copies)]).astype(np.int32)
-    csr = vs.Csr.from_arrays(one.M * copies, one.N, rp, np.tile(one.col, copies),
-                             np.tile(one.val, copies))
+    csr = tile_csr(vs, one, copies)
+    items, pieces, _, piece = work_items(csr)
+    assert piece == 64
+    assert items_per_wave(items, pieces, O) == {1: 1, 40: 1, 120: 2, 600: 4 if O <= 8 else 2}[copies] or O > 32
     fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
     fmt.set_tile_rows(1)
     fmt.upload(st)
@@ -152,6 +154,50 @@ def test_row_tiles_any_width(gpu, orc, st, copies, O, off):
     l1 = np.add.reduceat(np.append(np.abs(csr.val), 0), csr.row_ptr[:-1])
     l1[np.diff(csr.row_ptr) == 0] = 0
     assert (err <= 1e-4 * l1[:, None] * np.abs(B).max()).all()
+
+
+# Rows of one piece each: 17 to 64 entries (mean 35 or 20), or 65 to 128.
+_ONE_PIECE = {"mid": [17, 20, 33, 64, 40, 31, 25, 48], "short": [17, 19, 20, 24, 22, 18],
+              "long": [65, 128, 100, 77]}
+
+
+@pytest.mark.parametrize("kind,copies,O,merge", [
+    ("mid", 1, 1, 1), ("mid", 1, 12, 1), ("mid", 1, 31, 1), ("mid", 1, 50, 1), ("mid", 1, 101, 1),
+    ("mid", 1, 257, 1), ("long", 1, 8, 1), ("long", 1, 13, 1), ("long", 1, 64, 1),
+    ("long", 1, 128, 1), ("short", 1000, 20, 2), ("mid", 2100, 8, 4), ("mid", 2100, 12, 0),
+    ("mid", 2100, 30, 4), ("mid", 2100, 50, 2), ("long", 4200, 7, 4), ("long", 4200, 15, 0),
+    ("long", 4200, 33, 2), ("short", 5500, 12, 4), ("short", 5500, 15, 4), ("short", 8300, 100, 2),
+    ("short", 11000, 130, 2)])
+def test_row_tiles_of_one_piece(gpu, orc, st, kind, copies, O, merge):
+    """Single-row tiles where every work item is one row: a wave of one item
+    (its streams' sums meet in a butterfly), and waves of several (pieces cut
+    between streams), C = A*B and C += A*B.  merge 0: the 16-lane shape, one
+    item a wave at any size."""
+    vs = gpu
+    rng = np.random.default_rng(copies + O)
+    lens = _ONE_PIECE[kind]
+    N = 700
+    rows = np.repeat(np.arange(len(lens)), lens).astype(np.int32)
+    cols = np.concatenate([np.sort(rng.choice(N, size=n, replace=False)) for n in lens])
+    one = vs.coo_to_csr(vs.Coo.from_arrays(len(lens), N, rows, cols.astype(np.int32),
+                                           rng.standard_normal(rows.size).astype(np.float32)))
+    csr = tile_csr(vs, one, copies)
+    fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
+    fmt.set_tile_rows(1)
+    fmt.upload(st)
+    info = fmt.launch_info(O)
+    assert info["split_rows"] == 0
+    if merge:
+        assert items_per_wave(csr.M, csr.M, O) == merge
+    else:
+        assert info["vec"] == 1
+    B = vs.gen_dense(O, 0, N, O)
+    ref = np.tile(orc.spmm_f64(one.M, one.row_ptr, one.col, one.val, B), (copies, 1))
+    C0 = np.ones((csr.M, O), np.float32)
+    for accumulate in (False, True):
+        got = _spmm(vs, fmt, B, C0, 4 * accumulate, st, accumulate)
+        assert_within_tolerance(got - C0 if accumulate else got, ref, csr.row_ptr, csr.val, B,
+                                f"{kind} O{O}")
 
 
 @pytest.mark.parametrize("O", [5, 8, 12, 30, 47, 100])

@@ -67,6 +67,7 @@ int64_t tile_partials_floats(const Vcsr& v, const DeviceFmt& d, int32_t O);
 hipError_t launch_vcsr_row_tiles(const DeviceFmt& d, const float* B, int32_t O, int32_t ld,
                                  float* C, int32_t accumulate, uint64_t b_bytes, float* partials,
                                  hipStream_t st);
+int row_tiles_vec(const DeviceFmt& d, int32_t O);  // floats per lane of that launch
 hipError_t launch_vcsr_tall(const DeviceFmt& d, const float* B, int32_t O, int32_t ld, float* C,
                             int32_t accumulate, uint64_t b_bytes, float* partials, hipStream_t st);
 // Partial-row floats that cover tile_partials_floats for every O:

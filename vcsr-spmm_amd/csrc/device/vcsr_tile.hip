@@ -479,15 +479,13 @@ static int tile_mma_vec(const DeviceFmt& d, int32_t w) {
     return vec;
 }
 
-// Floats per lane of tiles of 1 to 8 rows for w columns of any alignment (the
-// shapes of vcsr_tile_row.hip and vcsr_tile_tall.hip); the reduce of their
-// partial rows takes the same.
-static int tile_valu_vec(int32_t R, int32_t w) {
-    return w > 32 || (w > 16 && R < 4) ? 4 : w > 8 && R == 1 ? 2 : 1;
-}
-
+// Floats per lane of any tiles for w columns of any alignment (the shapes of
+// vcsr_tile_row.hip and vcsr_tile_tall.hip); the reduce of their partial rows
+// takes the same.
 static int tile_vec(const DeviceFmt& d, int32_t w) {
-    return d.tv_R == kTileMmaRows ? tile_mma_vec(d, w) : tile_valu_vec(d.tv_R, w);
+    if (d.tv_R == kTileMmaRows) return tile_mma_vec(d, w);
+    if (d.tv_R == 1) return row_tiles_vec(d, w);
+    return w > 32 || (w > 16 && d.tv_R < 4) ? 4 : 1;
 }
 
 // Column-slice width of a launch over B and C of width O.  Tiles of 1 to 8

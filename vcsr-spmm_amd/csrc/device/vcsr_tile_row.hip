@@ -2,10 +2,10 @@
 // See vcsr_tile.hip for the view and the other tile heights.
 //
 // A wave takes MERGE consecutive work items of the view, at most PE*MERGE
-// entries (PE the view's largest piece, 64 or 128) and 32*MERGE pieces (a piece is a row, or a part of a very long
-// one).  The wave is S = 64/LPE streams of LPE lanes; each stream takes an
-// equal run of the wave's entries, and one load instruction fetches one
-// entry's B slice (LPE*VEC columns) for every stream.
+// entries (PE the view's largest piece, 64 or 128) and 32*MERGE pieces (a piece
+// is a row, or a part of a very long one).  The wave is S = 64/LPE streams of
+// LPE lanes; each stream takes an equal run of the wave's entries, and one load
+// instruction fetches one entry's B slice (LPE*VEC columns) for every stream.
 //  1. Staging, lane per entry: the entry records (value, B row, and whether
 //     the entry ends its piece) and the pieces' destinations are read with
 //     all loads in flight at once.  The records go to LDS as (B-row byte
@@ -16,22 +16,26 @@
 //  2. Blocks of U loads back to back, then their FMAs; where an entry ends
 //     its piece the sum is stored and cleared.
 //  3. A piece cut between runs is finished by the stream that began it, from
-//     the later streams' partial sums in LDS, added in stream order.
+//     the later streams' partial sums in LDS, added in stream order; their
+//     number comes from one ballot.  A wave of one piece adds its streams'
+//     sums in a butterfly instead and has no step for ends.
 // B is read with raw buffer loads whose range check turns "no row" offsets
 // into zeros; a B of 2 GB or more is read at 64-bit addresses and "no row"
 // entries select zero.  A row holds only entries it has, so a non-finite B
 // needs no second pass.
 // Bound by L2 misses (one 128-byte line per random B slice at narrow B, the
 // slices themselves at wide B) and by the waves' chain of loads on smaller
-// matrices.  Against one kernel with a path for several pieces and one for a
-// long piece, and a piece table of 16 bytes per piece read after the entries:
-// 39 instead of 55 registers at O = 8, 21 instead of 29 bytes of view per
-// two-entry row, one round of loads, no bounds test per entry, and 16-byte
-// lanes at any width.  Three formats in turn, us per SpMM: power-law 322K, O
-// = 8 24.0 -> 22.2; 100K, O = 20 / 47 / 257 18.3 / 23.4 / 121 -> 15.5 / 20.9 /
-// 85; uniform 27K x 14, O = 12 10.0 -> 6.1; banded 60K x 30, O = 50 32.8 ->
-// 25.1; uniform 102K x 6, O = 200 107 -> 88; C += A*B, power-law 100K, O = 47
-// 34.2 -> 29.2.
+// matrices: the runs' sums read one after the other, each behind two reads
+// that said whether to go on, cost more than the loop there (banded 8K x 20, O
+// = 8 / 32 5.2 / 5.7 us, 3.6 / 3.7 with the ballot and the butterfly).
+// Against one kernel with a path for several pieces and one for a long piece,
+// and a piece table of 16 bytes per piece read after the entries: 37 instead of
+// 55 registers at O = 8, 21 instead of 29 bytes of view per two-entry row, one
+// round of loads, no bounds test per entry, and 16-byte lanes at any width.
+// Three formats in turn, us per SpMM: power-law 322K, O = 8 24.0 -> 21.7; 100K,
+// O = 20 / 47 / 257 18.3 / 23.4 / 121 -> 14.7 / 20.8 / 85; banded 60K x 30, O =
+// 50 32.8 -> 25.1; uniform 102K x 6, O = 200 107 -> 88; C += A*B, power-law
+// 100K, O = 47 34.2 -> 29.2.
 #include <type_traits>
 
 #include "../host/tile_view.hpp"
@@ -69,7 +73,14 @@ struct RowLds {
     int32_t carry[Sh::S];                     // ... and whether it began in an earlier run
 };
 
-template <int VEC, int LPE, int MERGE, int PE, bool BUF, bool ACC>
+// What becomes of C: written (C = A*B), or added to (C += A*B), whose rows are
+// then read ahead of their pieces' ends, so that an end does not wait for
+// memory: a block's rows together with its B slices where pieces are short,
+// each piece's row where the piece begins where they are long (one row in
+// registers instead of one per entry of a block).
+enum RowOut { kRowWrite, kRowAddShort, kRowAddLong };
+
+template <int VEC, int LPE, int MERGE, int PE, bool BUF, RowOut OUT>
 __global__ __launch_bounds__(64 * kWaves)
 void vcsr_row_kernel(
     int32_t n_items, int32_t O, int32_t ld, uint32_t b_bytes,
@@ -81,8 +92,9 @@ void vcsr_row_kernel(
     constexpr int S = Sh::S, UT = Sh::UT, IE = Sh::IE, IP = Sh::IP;
     // Loads per block: 8; 4 where the rows of C are loaded with them (8 cost
     // two waves per SIMD: uniform 395K x 5, O = 32 65.8 / 74.1 us, power-law
-    // 322K, O = 128 167.5 / 178.0; without C's rows 4 are 0-3% slower).
-    constexpr int U = ACC && VEC == 4 ? 4 : 8;
+    // 322K, O = 128 167.5 / 178.0; without C's rows 4 are 0-3% slower), and
+    // where a row of C is held for short runs (banded 120K x 20, O = 64 38.9 / 37.6).
+    constexpr int U = VEC == 4 && (OUT == kRowAddShort || (OUT == kRowAddLong && LPE <= 16)) ? 4 : 8;
     __shared__ RowLds<VEC, LPE, MERGE, PE> s_lds[kWaves];
 
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -163,8 +175,7 @@ void vcsr_row_kernel(
         }
     };
     const int32_t kc = vec_col<VEC>(k, O);
-    auto load_c = [&](int32_t p) -> V {
-        const int32_t d = L.dest[p];
+    auto load_c = [&](int32_t d) -> V {
         return d >= 0 ? load_mem(C + (int64_t)d * ld + kc, V()) : zero_vec(V());
     };
     // Stores the sum x of piece p; c are the row's values in C.
@@ -172,7 +183,7 @@ void vcsr_row_kernel(
         const int32_t d = L.dest[p];
         if (!kok) return;
         if (d >= 0) {
-            if constexpr (ACC) x = add_vec(c, x);
+            if constexpr (OUT != kRowWrite) x = add_vec(c, x);
             store_cols<VEC, true>(C + (int64_t)d * ld, k, O, x, false);
         } else {
             store_cols<VEC, false>(partials + (int64_t)~d * O, k, O, x, false);
@@ -182,8 +193,12 @@ void vcsr_row_kernel(
     int32_t p = L.first[sub];
     bool carry = S > 1 && L.carry[sub] != 0;
     V acc = zero_vec(V());
-    auto block = [&](auto n_c, int32_t i0) {
+    V c_next = zero_vec(V());  // a row of C read ahead of its piece's end
+    // Entries i0 .. i0 + NU - 1 of every stream's run; `ends`: pieces may end
+    // among them.
+    auto block = [&](auto n_c, auto ends, int32_t i0) {
         constexpr int NU = decltype(n_c)::value;
+        constexpr bool ENDS = decltype(ends)::value;
         uint2 r[NU];
         V b[NU];
 #pragma unroll
@@ -196,50 +211,95 @@ void vcsr_row_kernel(
         for (int u = 0; u < NU; ++u) b[u] = load_b(r[u].x);
         // End bits of entries tb + i0 .. + NU - 1.
         const int32_t t = tb + i0;
-        const uint32_t bits = __builtin_amdgcn_alignbit(L.ends[(t >> 5) + 1], L.ends[t >> 5], t & 31);
-        // C += A*B: the rows that end in this block are read with its B
-        // slices, so that a row's end does not wait for memory.
-        V c[ACC ? NU : 1];
-        if constexpr (ACC) {
+        const uint32_t bits =
+            ENDS ? __builtin_amdgcn_alignbit(L.ends[(t >> 5) + 1], L.ends[t >> 5], t & 31) : 0u;
+        V c[OUT == kRowAddShort ? NU : 1];
+        if constexpr (ENDS && OUT == kRowAddShort) {
+            int32_t d[NU];
 #pragma unroll
             for (int u = 0; u < NU; ++u)
-                if (bits & (1u << u)) c[u] = load_c(p + __popc(bits & ((1u << u) - 1u)));
+                d[u] = L.dest[min(p + (int32_t)__popc(bits & ((1u << u) - 1u)), np - 1)];
+#pragma unroll
+            for (int u = 0; u < NU; ++u)
+                if (bits & (1u << u)) c[u] = load_c(d[u]);
         }
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
             fma_vec(acc, __builtin_bit_cast(float, r[u].y), b[u]);
-            if (bits & (1u << u)) {
+            if (ENDS && (bits & (1u << u))) {
                 if (S > 1 && carry) {
                     // The end of a piece begun in an earlier run.
                     L.xs[lane] = acc;
                     carry = false;
                 } else {
-                    store_piece(p, acc, c[ACC ? u : 0]);
+                    store_piece(p, acc, OUT == kRowAddShort ? c[u] : c_next);
                 }
                 acc = zero_vec(V());
                 ++p;
+                if constexpr (OUT == kRowAddLong) {
+                    if (p < np) c_next = load_c(L.dest[p]);
+                }
             }
         }
     };
-    int32_t i0 = 0;
-    for (; i0 + U <= run; i0 += U) block(std::integral_constant<int, U>(), i0);
-    if (i0 + U / 2 <= run) {
-        block(std::integral_constant<int, U / 2>(), i0);
-        i0 += U / 2;
+    auto walk = [&](auto ends) {
+        int32_t i0 = 0;
+        for (; i0 + U <= run; i0 += U) block(std::integral_constant<int, U>(), ends, i0);
+        if (i0 + U / 2 <= run) {
+            block(std::integral_constant<int, U / 2>(), ends, i0);
+            i0 += U / 2;
+        }
+        if constexpr (U / 4 >= UT)
+            if (i0 + U / 4 <= run) block(std::integral_constant<int, U / 4>(), ends, i0);
+    };
+
+    if constexpr (MERGE == 1 && S > 1) {
+        // One piece in the wave: nothing ends before the last entry, and the
+        // streams' sums meet in a butterfly.
+        if (np == 1) {
+            if (OUT != kRowWrite && sub == 0) c_next = load_c(L.dest[0]);
+            walk(std::false_type());
+#pragma unroll
+            for (int sh = LPE; sh < 64; sh <<= 1) acc = add_vec(acc, shfl_xor_vec(acc, sh));
+            if (sub == 0) store_piece(0, acc, c_next);
+            return;
+        }
     }
-    if constexpr (U / 4 >= UT)
-        if (i0 + U / 4 <= run) block(std::integral_constant<int, U / 4>(), i0);
+
+    // The row of C of the piece that this stream begins and the next run opens
+    // with (the stream finishes it below), or of its first piece.
+    const int32_t p_first = p;
+    const int nsub = sub + 1 < S ? sub + 1 : sub;
+    if constexpr (OUT == kRowAddShort && S > 1) {
+        const int32_t p_open = L.first[nsub];
+        if (nsub > sub && L.carry[nsub] != 0 && !(carry && p_open == p_first))
+            c_next = load_c(L.dest[p_open]);
+    }
+    if constexpr (OUT == kRowAddLong) {
+        if (!carry && p < np) c_next = load_c(L.dest[p]);
+    }
+    walk(std::true_type());
 
     if constexpr (S > 1) {
-        // A run that ends inside a piece: its owner adds the following runs'
-        // partial sums; a run that lies wholly inside one leaves its own.
+        // A piece cut between runs: its owner adds the following runs' partial
+        // sums, in stream order, up to the run in which it ends (a run that
+        // lies wholly inside one leaves its own sum).  Their number comes from
+        // one ballot, so that the sums are read without waiting in between.
         if (carry) L.xs[lane] = acc;
+        const uint64_t ended = __ballot(p != p_first);
         wave_sync();
-        const bool open = sub + 1 < S && L.carry[sub + 1 < S ? sub + 1 : sub] != 0;
-        if (open && !carry) {
-            for (int s2 = sub + 1; s2 < S && L.carry[s2] != 0 && L.first[s2] == p; ++s2)
-                acc = add_vec(acc, L.xs[s2 * LPE + kl]);
-            store_piece(p, acc, ACC ? load_c(p) : zero_vec(V()));
+        if (nsub > sub && L.carry[nsub] != 0 && !carry) {
+            const int more = __builtin_ctzll(ended >> (nsub * LPE)) / LPE;  // runs after the next one
+            acc = add_vec(acc, L.xs[nsub * LPE + kl]);
+            if (more > 0) {
+                V x[S];
+#pragma unroll
+                for (int j = 1; j < S - 1; ++j) x[j] = L.xs[min(nsub + j, S - 1) * LPE + kl];
+#pragma unroll
+                for (int j = 1; j < S - 1; ++j)
+                    if (j <= more) acc = add_vec(acc, x[j]);
+            }
+            store_piece(p, acc, c_next);
         }
     }
 }
@@ -249,20 +309,47 @@ hipError_t launch_shape(const DeviceFmt& d, const float* B, int32_t O, int32_t l
                         int32_t accumulate, uint32_t b_bytes, float* partials, hipStream_t st) {
     constexpr int per = MERGE * kWaves;
     const dim3 grid((unsigned)(((int64_t)d.tv_n_chunks + per - 1) / per)), block(64 * kWaves);
-    auto go = [&](auto acc) {
-        hipLaunchKernelGGL((vcsr_row_kernel<VEC, LPE, MERGE, PE, BUF, decltype(acc)::value>), grid,
+    auto go = [&](auto out) {
+        hipLaunchKernelGGL((vcsr_row_kernel<VEC, LPE, MERGE, PE, BUF, decltype(out)::value>), grid,
                            block, 0, st, d.tv_n_chunks, O, ld, b_bytes,
                            reinterpret_cast<const int2*>(d.tv_items), d.tv_dest,
                            reinterpret_cast<const float2*>(d.tv_val), B, C, partials);
         return hipGetLastError();
     };
-    return accumulate ? go(std::true_type()) : go(std::false_type());
+    // C += A*B: a row of C ahead of each piece where pieces average more than
+    // 16 entries (banded 30K x 40, O = 8 / 256 8.8 / 51.3 -> 7.8 / 47.9 us; 60K x
+    // 70, O = 64 47.0 -> 45.3), else a block's rows with its B slices (power-law
+    // 322K, O = 47 91.2 us with neither, 75.5).
+    if (!accumulate) return go(std::integral_constant<RowOut, kRowWrite>());
+    return d.tv_n_entries > 16 * (int64_t)d.tv_n_pieces
+               ? go(std::integral_constant<RowOut, kRowAddLong>())
+               : go(std::integral_constant<RowOut, kRowAddShort>());
 }
 
 template <int X>
 using I = std::integral_constant<int, X>;
 
 }  // namespace
+
+// Whether the work items mostly hold one piece (rows of more than 16 entries).
+static bool single_pieces(const DeviceFmt& d) {
+    return (int64_t)d.tv_n_pieces < 2 * (int64_t)d.tv_n_chunks;
+}
+
+// 9 to 16 columns: 8 lanes of 2 floats, half the load instructions an entry, or
+// 16 lanes of 1, half the streams a piece is cut between and so one piece a
+// wave at little cost.  The second where items are single pieces, unless there
+// are many and short ones, which then share waves.  us per SpMM, 16 lanes / 8
+// lanes, O = 16: banded 4K x 30 2.9 / 3.5, 30K x 40 8.6 / 9.2, 45K x 50 18.2 /
+// 18.5, 60K x 70 23.3 / 24.7, 60K x 30 17.4 / 13.4, 120K x 20 30.3 / 18.6; items
+// of several pieces: uniform 50K x 10 9.0 / 7.9, power-law 322K 26.4 / 24.1.
+
+int row_tiles_vec(const DeviceFmt& d, int32_t O) {
+    if (O > 16) return 4;
+    if (O <= 8) return 1;
+    const bool few = d.tv_n_chunks < 32 * (4 * (int64_t)device_cus(d.device));
+    return single_pieces(d) && (few || d.tv_n_entries > 32 * (int64_t)d.tv_n_pieces) ? 1 : 2;
+}
 
 hipError_t launch_vcsr_row_tiles(const DeviceFmt& d, const float* B, int32_t O, int32_t ld,
                                  float* C, int32_t accumulate, uint64_t b_bytes, float* partials,
@@ -283,35 +370,45 @@ hipError_t launch_vcsr_row_tiles(const DeviceFmt& d, const float* B, int32_t O, 
         return d.tv_piece > kTileRowPiece ? go_pe(vec, lpe, merge, I<tile_piece_entries(1)>())
                                           : go_pe(vec, lpe, merge, I<kTileRowPiece>());
     };
-    // Work items per wave.  us per SpMM, three formats in turn (the view comes
-    // from beyond L2), 1 / 2 / 4 items:
-    //  - O <= 32: as many as leave 4 waves per SIMD.  Power-law 322K rows (57K
-    //    items), O = 8 29.6 / 24.6 / 22.8; 100K rows (17K), O = 8 14.1 / 13.4 /
-    //    12.9; uniform 27K x 14 (13K), O = 12 7.7 / 6.2 / 6.8; uniform 20K x 10
-    //    (7K), O = 16 5.1 / 5.3 / 6.3; 8 items 27.4 on the first.
-    //  - wider: 2 where the items mostly hold one piece (rows of more than 16
-    //    entries), else 1.  Banded 60K x 30, O = 50 / 64 30.7 / 24.9 / 24.9 and
-    //    29.2 / 22.6 / 22.5; uniform 137K x 11, O = 64 54.9 / 57.4 / 56.9;
-    //    power-law 100K, O = 47 22.0 / 24.7 / 25.3, 322K, O = 128 109.7 / 113.6
-    //    / 126.4 (longer waves leave the XCD's range of B later).
+    // Work items per wave: as many as still leave every SIMD its waves, fewer
+    // where long waves leave the XCD's range of B late.  us per SpMM, two
+    // formats in turn, 1 / 2 / 4 items:
+    //  - several pieces an item: uniform 20K x 10 (7K items), O = 1 / 32 4.0 / 3.5
+    //    / 4.2 and 5.1 / 4.7 / 5.7; power-law 100K (17K), O = 1 10.9 / 10.4 / 10.6;
+    //    322K (57K), O = 1 / 8 / 32 23.6 / 19.3 / 18.1, 25.5 / 21.8 / 21.2 and
+    //    31.2 / 28.6 / 30.1; wider always 1: power-law 100K, O = 47 21.0 / 22.8 /
+    //    23.7, 322K, O = 128 107 / 111 / 125.
+    //  - one piece an item: banded 8K x 60, O = 8 / 64 4.1 / 4.6 / 5.5 and 7.0 /
+    //    7.4 / 8.1; 20K x 25, O = 8 5.9 / 5.8 / 5.1; 30K x 40, O = 32 / 64 11.4 /
+    //    10.5 / 10.0 and 16.4 / 15.8 / 16.2; 120K x 20, O = 8 / 64 27.8 / 20.4 /
+    //    15.9 and 39.3 / 32.3 / 42.6; O = 128: 45K x 50 47.5 / 48.3, 120K x 20 56.6
+    //    / 53.4; O = 256: 120K x 20 137 / 133.
     const int64_t items = d.tv_n_chunks, simds = 4 * (int64_t)device_cus(d.device);
-    const bool single = (int64_t)d.tv_n_pieces < 2 * items;
-    auto narrow = [&](auto vec, auto lpe) {
-        return items >= 16 * simds  ? go(vec, lpe, I<4>())
-               : items >= 8 * simds ? go(vec, lpe, I<2>())
-                                    : go(vec, lpe, I<1>());
-    };
-    auto wide = [&](auto lpe) {
-        return single && items >= 8 * simds ? go(I<4>(), lpe, I<2>()) : go(I<4>(), lpe, I<1>());
-    };
-    if (O <= 8) return narrow(I<1>(), I<8>());
-    // 8 lanes of 2 floats: power-law 100K / 322K, O = 16 13.3 / 26.4 us against
-    // 14.6 / 28.4 with 16 lanes of 1 (half the load instructions).
-    if (O <= 16) return narrow(I<2>(), I<8>());
-    if (O <= 32) return narrow(I<4>(), I<8>());
-    if (O <= 64) return wide(I<16>());
-    if (O <= 128) return wide(I<32>());
-    return wide(I<64>());
+    const bool single = single_pieces(d);
+    if (O <= 8) {
+        const int64_t four = single ? 16 : 24;
+        return items >= four * simds          ? go(I<1>(), I<8>(), I<4>())
+               : !single && items >= 5 * simds ? go(I<1>(), I<8>(), I<2>())
+                                               : go(I<1>(), I<8>(), I<1>());
+    }
+    if (O <= 16) {
+        if (row_tiles_vec(d, O) == 1) return go(I<1>(), I<16>(), I<1>());
+        return single                ? go(I<2>(), I<8>(), I<4>())
+               : items >= 5 * simds ? go(I<2>(), I<8>(), I<2>())
+                                    : go(I<2>(), I<8>(), I<1>());
+    }
+    if (O <= 32)
+        return single && items >= 16 * simds ? go(I<4>(), I<8>(), I<4>())
+               : items >= 5 * simds          ? go(I<4>(), I<8>(), I<2>())
+                                             : go(I<4>(), I<8>(), I<1>());
+    if (O <= 64)
+        return single && items >= 16 * simds ? go(I<4>(), I<16>(), I<2>())
+                                             : go(I<4>(), I<16>(), I<1>());
+    if (O <= 128)
+        return single && items >= 48 * simds ? go(I<4>(), I<32>(), I<2>())
+                                             : go(I<4>(), I<32>(), I<1>());
+    return single && items >= 64 * simds ? go(I<4>(), I<64>(), I<2>())
+                                         : go(I<4>(), I<64>(), I<1>());
 }
 
 }  // namespace vcsr
