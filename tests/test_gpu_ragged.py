@@ -44,6 +44,54 @@ def test_mfma_tiles_any_width_are_bit_exact(gpu, orc, st, O, off):
     assert np.array_equal(got, C0 + ref)
 
 
+def _sixteen_rows(vs, rng, copies):
+    """Seven 16-row tiles of 1 to 7 whole groups of 16 entries, one entry in ten
+    absent, `copies` times below each other; and the seven alone."""
+    rows, cols = [], []
+    for t in range(7):
+        c = np.sort(rng.choice(200, size=16 * (t + 1), replace=False))
+        for i in range(16):
+            keep = c[(rng.random(c.size) < 0.9) | (np.arange(c.size) % 16 == i)]
+            rows.append(np.full(keep.size, 16 * t + i))
+            cols.append(keep)
+    rows, cols = np.concatenate(rows).astype(np.int32), np.concatenate(cols).astype(np.int32)
+    one = vs.coo_to_csr(vs.Coo.from_arrays(112, 200, rows, cols,
+                                           rng.standard_normal(rows.size).astype(np.float32)))
+    return one, tile_csr(vs, one, copies)
+
+
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("tiles,O", [
+    (91, 8), (602, 16), (399, 18), (602, 31), (1099, 24), (1099, 31), (91, 47), (98, 257), (602, 33),
+    (602, 50), (602, 64), (1022, 61), (602, 65), (1099, 33), (1099, 64), (1099, 127), (700, 131),
+    (1099, 259), (1099, 256)])
+def test_mfma_tiles_of_every_wave_count(gpu, orc, st, tiles, O, off):
+    """16-row MFMA tiles at lanes of 1, 2 and 4 floats, whole rows and odd ones,
+    at up to 1,024 waves (two operand sets), up to 3,072 (loads ahead) and more
+    (mixed), with pieces of an odd and an even number of blocks: bit for bit the
+    oracle's FP32 loop, C += A*B and inf and NaN next to a row's moved-back end
+    among them."""
+    vs = gpu
+    one, csr = _sixteen_rows(vs, np.random.default_rng(O), tiles // 7)
+    fmt = vs.build_vcsr(csr, 16, 16, vs.LAYOUT_TC)
+    fmt.set_tile_rows(16)
+    fmt.upload(st)
+    info = fmt.launch_info(O)
+    assert info["tiles"] == tiles and info["split_rows"] == 0
+    B = vs.gen_dense(O, 1, csr.N, O)
+    C0 = np.full((csr.M, O), 2.0, np.float32)
+    ref = np.tile(orc.spmm_f32(one.M, one.row_ptr, one.col, one.val, B), (tiles // 7, 1))
+    got = _spmm(vs, fmt, B, C0, off, st, False)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    assert np.array_equal(_spmm(vs, fmt, B, C0, off, st, True), C0 + ref)
+    B[3, O - 1], B[50, O - 2], B[199, 0] = np.inf, np.nan, -np.inf
+    ref = np.tile(orc.spmm_f32(one.M, one.row_ptr, one.col, one.val, B), (tiles // 7, 1))
+    got = _spmm(vs, fmt, B, C0, off, st, False)
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got.view(np.uint32)[~nan], ref.view(np.uint32)[~nan])
+
+
 def _mixed_blocks(vs, rng, h):
     """Block rows of h equal-pattern rows: short and long ones, one cut into
     several pieces (600 columns), empty rows, a last block row cut short."""

@@ -276,17 +276,26 @@ __global__ __launch_bounds__(256) void vcsr_tile_mma_kernel(
             MmaGroups<VEC, GU> x, y;
             load(x, 0);
             int32_t i = 0;
-            for (; i + 2 <= nb; i += 2) {
+            for (; i + 3 <= nb; i += 2) {
                 load(y, (i + 1) * GU);
                 __builtin_amdgcn_sched_barrier(0);
                 multiply(x);
                 __builtin_amdgcn_sched_barrier(0);
-                load(x, min(i + 2, nb - 1) * GU);
+                load(x, (i + 2) * GU);
                 __builtin_amdgcn_sched_barrier(0);
                 multiply(y);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (i < nb) multiply(x);
+            // The last two blocks apart: a load past them, though its result
+            // goes unused, is waited for before the wave's stores.
+            if (i + 2 == nb) {
+                load(y, (i + 1) * GU);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(x);
+                multiply(y);
+            } else {
+                multiply(x);
+            }
             g0 = nb * GU;
         }
     } else {
