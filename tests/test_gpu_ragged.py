@@ -61,11 +61,12 @@ def _sixteen_rows(vs, rng, copies):
 
 
 @pytest.mark.parametrize("off", [0, 4])
-@pytest.mark.parametrize("tiles,O", [
-    (91, 8), (602, 16), (399, 18), (602, 31), (1099, 24), (1099, 31), (91, 47), (98, 257), (602, 33),
-    (602, 50), (602, 64), (1022, 61), (602, 65), (1099, 33), (1099, 64), (1099, 127), (700, 131),
-    (1099, 259), (1099, 256)])
-def test_mfma_tiles_of_every_wave_count(gpu, orc, st, tiles, O, off):
+@pytest.mark.parametrize("tiles,O,vec", [
+    (91, 8, 1), (602, 16, 1), (399, 18, 1), (602, 31, 2), (1099, 24, 2), (1099, 31, 2), (91, 47, 1),
+    (91, 48, 2), (98, 257, 1), (98, 259, 1), (602, 33, 4), (602, 50, 4), (602, 64, 4), (1022, 61, 4),
+    (602, 65, 2), (602, 72, 2), (384, 131, 2), (1099, 33, 4), (1099, 64, 4), (1099, 127, 4),
+    (700, 101, 4), (700, 131, 2), (1099, 259, 4), (1099, 256, 4)])
+def test_mfma_tiles_of_every_wave_count(gpu, orc, st, tiles, O, vec, off):
     """16-row MFMA tiles at lanes of 1, 2 and 4 floats, whole rows and odd ones,
     at up to 1,024 waves (two operand sets), up to 3,072 (loads ahead) and more
     (mixed), with pieces of an odd and an even number of blocks: bit for bit the
@@ -77,7 +78,7 @@ def test_mfma_tiles_of_every_wave_count(gpu, orc, st, tiles, O, off):
     fmt.set_tile_rows(16)
     fmt.upload(st)
     info = fmt.launch_info(O)
-    assert info["tiles"] == tiles and info["split_rows"] == 0
+    assert info["tiles"] == tiles // 7 * 7 and info["split_rows"] == 0 and info["vec"] == vec
     B = vs.gen_dense(O, 1, csr.N, O)
     C0 = np.full((csr.M, O), 2.0, np.float32)
     ref = np.tile(orc.spmm_f32(one.M, one.row_ptr, one.col, one.val, B), (tiles // 7, 1))

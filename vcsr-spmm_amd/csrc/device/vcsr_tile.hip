@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) void vcsr_tile_reduce(int32_t O, int32_t ld, i
 //
 // Rows of B and C need not be aligned to VEC floats: a lane whose columns
 // would reach past O takes the last VEC of the row and stores its own ones
-// (vec_col, store_cols), so every O over 32 reads 16 bytes per lane.
+// (vec_col, store_cols), so VEC depends on O and the tiles only (tile_mma_vec).
 // Block-sparse 16K matrix, O = 65 / 127 / 333: 51.8 / 84.1 / 229 us with the
 // 4-byte lanes an odd O used to take, 39.8 / 41.8 / 101 now; O = 64, 100,
 // 512 unchanged.
@@ -481,10 +481,31 @@ hipError_t launch_vec(const Vcsr& v, const DeviceFmt& d, const float* B, int32_t
 // all values again: block-sparse 16K matrix, O = 24 16.7 us as one tile of
 // 2 floats per lane against 24.6 as two of 1, O = 50 22.7 as one of 4
 // against 30.4 as two of 2.
+// Four floats a lane give way to two where the launch then takes less than 3/2
+// of its rounds of waves (a wave with two takes two thirds of the time), and two
+// to one where all waves still fit one round.  A second time, or with three
+// rounds for short pieces of very few tiles, only where a row is no whole number
+// of vectors, whose moved-back ends cost more than the values read again.
+// us per SpMM, 2 / 4 floats: 380 tiles of 320 entries, O = 144 14.5 / 18.2; 768,
+// O = 130 / 200 25.1 / 28.4 and 32.2 / 28.5; 512 of 816, O = 128 30.3 / 22.6;
+// 1 / 2 / 4: 128 of 96, O = 47 4.1 / 4.9 / 6.1, O = 257 5.6 / 6.5 / 6.3; 128 of
+// 400, O = 257 14.8 / 16.6 / 13.1; 256 of 400, O = 47 7.6 / 9.0 / 12.0, O = 64,
+// C += A*B 10.0 / 8.7 / 11.8; 512 of 816, O = 33 24.0 / 17.4 / 22.4.
 static int tile_mma_vec(const DeviceFmt& d, int32_t w) {
-    int vec = w > 32 ? 4 : w > 16 ? 2 : 1;
-    const int64_t n_ct = vec > 1 ? (w + 8 * vec - 1) / (8 * vec) : 0;
-    if (vec > 1 && (int64_t)d.tv_n_chunks * n_ct <= 4 * (int64_t)device_cus(d.device)) vec /= 2;
+    const int widest = w > 32 ? 4 : w > 16 ? 2 : 1;
+    const int64_t simds = 4 * (int64_t)device_cus(d.device), tiles = d.tv_n_chunks;
+    const bool tiny = 8 * tiles <= simds && d.tv_n_entries <= 128 * tiles;
+    auto rounds = [&](int vec) {
+        return (tiles * ((w + 16 * vec - 1) / (16 * vec)) + simds - 1) / simds;
+    };
+    int vec = widest;
+    while (vec > 1) {
+        const bool whole = w % vec == 0;
+        const int64_t half = rounds(vec / 2);
+        const bool better = vec < widest ? !whole && half == 1 : 2 * half < 3 * rounds(vec);
+        if (!better && !(tiny && !whole && half <= 3)) break;
+        vec /= 2;
+    }
     return vec;
 }
 
