@@ -137,6 +137,30 @@ def test_tall_tiles_any_width(gpu, orc, st, R, O, off):
     assert (err <= 1e-4 * l1[:, None] * np.abs(B).max()).all()
 
 
+@pytest.mark.parametrize("copies", [40, 500])
+@pytest.mark.parametrize("O", [128, 129, 200, 256, 259])
+@pytest.mark.parametrize("R", [2, 3, 4])
+def test_tall_tiles_accumulate_many(gpu, orc, st, R, O, copies):
+    """C += A*B on fewer and on more tiles than 8 waves per SIMD: rows of C read
+    ahead, and for 2 and 3 rows at O > 128 late; split tiles among them, one
+    rounding from C0 + A*B, the same bits twice."""
+    vs = gpu
+    one = _mixed_blocks(vs, np.random.default_rng(R + O), R)
+    csr = tile_csr(vs, one, copies)
+    fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
+    fmt.set_tile_rows(R)
+    fmt.upload(st)
+    assert (fmt.launch_info(O)["tiles"] > 8192) == (copies == 500)
+    B = vs.gen_dense(O, 0, csr.N, O)
+    C0 = np.random.default_rng(O).integers(-2, 3, size=(csr.M, O)).astype(np.float32)
+    ref = np.tile(orc.spmm_f64(one.M, one.row_ptr, one.col, one.val, B), (copies, 1))
+    got = _spmm(vs, fmt, B, C0, 4, st, True)
+    err = np.abs(got - (C0 + ref)) - 2.0 ** -23 * (np.abs(C0) + np.abs(ref))
+    l1 = np.array([np.abs(one.val[a:b]).sum() for a, b in zip(one.row_ptr, one.row_ptr[1:])])
+    assert (err <= 1e-4 * np.tile(l1, copies)[:, None] * np.abs(B).max()).all()
+    assert np.array_equal(got, _spmm(vs, fmt, B, C0, 0, st, True))
+
+
 @pytest.mark.parametrize("O", [5, 12, 30, 47, 100])
 @pytest.mark.parametrize("R", [2, 3, 4, 8])
 def test_tall_tiles_nonfinite_b(gpu, orc, st, R, O):

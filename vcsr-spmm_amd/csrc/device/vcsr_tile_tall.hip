@@ -63,7 +63,11 @@ struct TallLds {
     uint32_t off[Sh::REC ? 1 : Sh::G][Sh::REC ? 1 : Sh::SEG + (Sh::G > 1 ? S : 0)];
 };
 
-template <int VEC, int LPE, int S, int R, int U, bool BUF, bool ACC>
+// What becomes of C: written (C = A*B), or added to (C += A*B), whose rows are
+// then read ahead of everything else, or just before they are stored.
+enum TallOut { kTallWrite, kTallAdd, kTallAddLate };
+
+template <int VEC, int LPE, int S, int R, int U, bool BUF, TallOut OUT>
 __global__ __launch_bounds__(64 * kWaves)
 __attribute__((amdgpu_waves_per_eu(R <= 3 ? 5 : 1, 8)))
 void vcsr_tall_kernel(
@@ -122,10 +126,10 @@ void vcsr_tall_kernel(
         else return load_mem(B + (int64_t)off * ld + koff / 4, V());
     };
 
-    // C += A*B: this stream's rows of C are read ahead of everything else.
+    // C += A*B: this stream's rows of C.
     constexpr int CR = (R + S - 1) / S;
-    V c[ACC ? CR : 1];
-    if constexpr (ACC) {
+    V c[OUT == kTallWrite ? 1 : CR];
+    auto load_c = [&] {
 #pragma unroll
         for (int i = 0; i < CR; ++i) {
             const int r = i * S + sub;
@@ -133,7 +137,8 @@ void vcsr_tall_kernel(
                        ? load_mem(C + (int64_t)(pc.x + r) * ld + vec_col<VEC>(k, O), V())
                        : zero_vec(V());
         }
-    }
+    };
+    if constexpr (OUT == kTallAdd) load_c();
 
     V acc[R];
 #pragma unroll
@@ -258,6 +263,7 @@ void vcsr_tall_kernel(
         }
     }
     if (!kok) return;
+    if constexpr (OUT == kTallAddLate) load_c();
 #pragma unroll
     for (int i = 0; i < CR; ++i) {
         const int r = i * S + sub;
@@ -266,7 +272,7 @@ void vcsr_tall_kernel(
 #pragma unroll
             for (int q = 1; q < R; ++q)
                 if (q == r) x = acc[q];
-            if constexpr (ACC) x = add_vec(c[i], x);
+            if constexpr (OUT != kTallWrite) x = add_vec(c[i], x);
             if (pc.w < 0)
                 store_cols<VEC, true>(C + (int64_t)(pc.x + r) * ld, k, O, x, false);
             else
@@ -280,14 +286,27 @@ hipError_t launch_shape(const DeviceFmt& d, const float* B, int32_t O, int32_t l
                         int32_t accumulate, uint32_t b_bytes, float* partials, hipStream_t st) {
     constexpr int per = TallShape<LPE, S, R, U>::G * kWaves;
     const dim3 grid((unsigned)(((int64_t)d.tv_n_pieces + per - 1) / per)), block(64 * kWaves);
-    auto go = [&](auto acc) {
-        hipLaunchKernelGGL((vcsr_tall_kernel<VEC, LPE, S, R, U, BUF, decltype(acc)::value>), grid,
+    auto go = [&](auto out) {
+        hipLaunchKernelGGL((vcsr_tall_kernel<VEC, LPE, S, R, U, BUF, decltype(out)::value>), grid,
                            block, 0, st, d.tv_n_pieces, O, ld, b_bytes,
                            reinterpret_cast<const int4*>(d.tv_pieces), d.tv_brow, d.tv_mask,
                            d.tv_val, B, C, partials);
         return hipGetLastError();
     };
-    return accumulate ? go(std::true_type()) : go(std::false_type());
+    if (!accumulate) return go(std::integral_constant<TallOut, kTallWrite>());
+    // C is read ahead, except where the registers that its rows take cost waves
+    // (2 and 3 rows, O > 128: 6 instead of 8 per SIMD at 3) that more waves than
+    // are resident at once would fill, and where B and C fit into the 256 MB MALL
+    // with room, so that a late read waits for little.  us per SpMM, ahead / late:
+    // blocks of 2 rows, O = 256 62K x 24 58 / 44, 90K x 24 84 / 61; of 3 rows 62K x
+    // 64 70 / 62, 120K x 24, O = 200 69 / 54; few waves: 12K x 64, 3 rows, O = 200
+    // 13.5 / 14.5; B and C of 246 MB: 120K x 64, 3 rows, O = 256 132 / 149.
+    if constexpr (VEC == 4 && LPE == 64 && R <= 3 && BUF) {
+        const uint64_t c_bytes = (uint64_t)d.tv_n_pieces * R * (uint64_t)ld * 4u;
+        if (d.tv_n_pieces > 32 * (int64_t)device_cus(d.device) && b_bytes + c_bytes <= (192ull << 20))
+            return go(std::integral_constant<TallOut, kTallAddLate>());
+    }
+    return go(std::integral_constant<TallOut, kTallAdd>());
 }
 
 template <int X>
