@@ -295,7 +295,8 @@ int vcsr_fmt_upload(vcsr_fmt* fmt, void* stream) {
             d.n_partials = rv.n_partials;
             d.tv_R = tv.R;
             d.tv_piece = tv.piece;
-            if (tv.R != 1) d.tv_chunks = upload_array(tv.chunks, st, "upload tile chunks");
+            if (tv.R == vcsr::kTileMmaRows)
+                d.tv_chunks = upload_array(tv.chunks, st, "upload tile chunks");
             d.tv_items = upload_array(tv_items, st, "upload tile items");
             d.tv_dest = upload_array(tv_dest, st, "upload piece rows");
             d.tv_n_chunks = (int32_t)(tv.chunks.size() / 4);

@@ -40,7 +40,8 @@ struct DeviceFmt {
     // Row-tile view (host/tile_view.hpp) walked by the tile-stationary kernel.
     int32_t tv_R = 1;                   // accumulator rows per tile
     int32_t tv_piece = 0;               // most entries of a piece
-    int32_t* tv_chunks = nullptr;       // 4*tv_n_chunks: entry range, piece range
+    int32_t* tv_chunks = nullptr;       // 4*tv_n_chunks: entry range, piece range (16-row
+                                        // tiles only; tiles of 2 to 8 rows go by piece)
     int32_t tv_n_chunks = 0;
     int32_t* tv_pieces = nullptr;       // 4 per piece: row, rows, first entry, partial row;
                                         // then one whose first entry is the entry count
