@@ -173,7 +173,7 @@ static int check_cst(const Csr& csr, int segw, int bundle, int layout) {
 }
 
 static int check(const Csr& csr, int segw, int bundle, int layout, int R_req, int expect_R,
-                 bool fixed = false) {
+                 bool fixed = false, int expect_piece = 0) {
     const Vcsr v = build_vcsr(csr, segw, bundle, layout, 2);
     const TileView tv = make_tile_view(v, R_req, 2, fixed);
     const int R = tv.R, RS = tile_slot_stride(R), M = csr.M;
@@ -183,7 +183,11 @@ static int check(const Csr& csr, int segw, int bundle, int layout, int R_req, in
     if ((int64_t)tv.val.size() != E * RS) return fail("value array size", M, R);
     if ((int64_t)tv.mask.size() != E) return fail("mask array size", M, R);
     const int nc = (int)tv.chunks.size() / 4, np = (int)tv.pieces.size() / 4;
-    const int cap = tile_piece_entries(R);
+    // The kernels' LDS lists hold TileView::piece entries a work item.
+    const int cap = tv.piece;
+    if (cap != tile_piece_entries(R) && !(R == 1 && cap == kTileRowPiece))
+        return fail("largest piece is not a kernel's", M, R);
+    if (expect_piece > 0 && cap != expect_piece) return fail("largest piece", M, R);
     int64_t prev_e = 0;
     int prev_p = 0;
     for (int c = 0; c < nc; ++c) {
@@ -304,9 +308,11 @@ static Csr block_matrix(uint64_t seed, int nbr, int bh, int N, int blocks, int b
 
 // Single-row views move the pieces of rows cut into 8 or more pieces into
 // the eighth of the work-item list whose eighth of B holds their middle
-// column (one run per XCD).  A banded matrix with a few long random rows:
-// the view stays valid, and nearly every moved piece sits in its run.
-static int check_long_piece_runs() {
+// column (one run per XCD).  A banded matrix of `short_row` entries a row with a
+// few long random rows: the view stays valid, with the largest piece that the
+// short rows ask for (128 where rows of 65 to 128 entries hold an eighth of all
+// entries, else 64), and nearly every moved piece sits in its run.
+static int check_long_piece_runs(int short_row) {
     Coo c;
     c.M = 8192;
     c.N = 8192;
@@ -319,17 +325,18 @@ static int check_long_piece_runs() {
     };
     for (int r = 0; r < c.M; ++r) {
         const bool long_row = r % 200 == 7;
-        const int k = long_row ? 2000 : 6;
+        const int k = long_row ? 2000 : short_row;
         for (int i = 0; i < k; ++i) {
             const int col = long_row ? (int)(next() % (uint64_t)c.N)
-                                     : std::min(c.N - 1, std::max(0, r - 60 + (int)(next() % 121)));
+                                     : std::min(c.N - 1, std::max(0, r - 60 + (short_row > 64 ? i : (int)(next() % 121))));
             c.rows.push_back(r);
             c.cols.push_back(col);
             c.vals.push_back((float)((int)(next() % 201) - 100) / 64.f);
         }
     }
     const Csr csr = coo_to_csr(c);
-    int bad = check(csr, 4, 64, kLayoutS, 1, 1);
+    const int piece = short_row > 64 ? 128 : kTileRowPiece;
+    int bad = check(csr, 4, 64, kLayoutS, 1, 1, false, piece);
     const Vcsr v = build_vcsr(csr, 4, 64, kLayoutS, 2);
     const TileView tv = make_tile_view(v, 1, 2, false);
     std::vector<int> npc((size_t)csr.M, 0);
@@ -339,7 +346,7 @@ static int check_long_piece_runs() {
     for (int ch = 0; ch < nc; ++ch) {
         const int e0 = tv.chunks[4 * ch], e1 = tv.chunks[4 * ch + 1], p0 = tv.chunks[4 * ch + 2];
         if (tv.chunks[4 * ch + 3] - p0 != 1 || tv.pieces[4 * p0 + 3] < 0) continue;
-        if (npc[(size_t)tv.pieces[4 * p0]] < 8) continue;
+        if (npc[(size_t)tv.pieces[4 * p0]] < 512 / piece) continue;
         ++moved;
         const int run = (int)((int64_t)ch * 8 / nc);
         const int want = (int)std::min<int64_t>(7, (int64_t)tv.brow[(size_t)(e0 + (e1 - e0) / 2)] * 8 / csr.N);
@@ -428,7 +435,20 @@ int main() {
             }
         bad |= check_cst(coo_to_csr(g), 4, 64, kLayoutS);
     }
-    bad |= check_long_piece_runs();
+    for (int short_row : {6, 90}) bad |= check_long_piece_runs(short_row);
+    // Rows of 65 to 128 entries: an eighth of all entries and just under it.
+    for (int n65 : {30, 29}) {
+        Coo c;
+        c.M = n65 + 455;
+        c.N = 4096;
+        for (int r = 0; r < c.M; ++r)
+            for (int k = 0; k < (r < n65 ? 65 : 30); ++k) {
+                c.rows.push_back(r);
+                c.cols.push_back((r * 31 + k * 7) % c.N);
+                c.vals.push_back((float)(k - 9) / 8.f);
+            }
+        bad |= check(coo_to_csr(c), 4, 64, kLayoutS, 1, 1, false, n65 == 30 ? 128 : kTileRowPiece);
+    }
     {
         const Csr cfg3 = coo_to_csr(gen_coo(3, 0));
         bad |= check_thread_independence(cfg3, 0, false);
