@@ -26,9 +26,9 @@ def _spmm(vs, fmt, B, C0, off, st, accumulate):
 @pytest.mark.parametrize("off", [0, 4])
 @pytest.mark.parametrize("O", [1, 15, 16, 17, 31, 33, 34, 63, 65, 66, 127, 259])
 def test_mfma_tiles_any_width_are_bit_exact(gpu, orc, st, O, off):
-    """16-row MFMA tiles: lanes of 1, 2 and 4 floats with a moved-back last
-    vector, bit for bit the oracle's FP32 loop; C += A*B on top of C0 = 2
-    stays within one rounding of it."""
+    """Few 16-row MFMA tiles: lanes of 1 and 2 floats (4 take more tiles, below),
+    bit for bit the oracle's FP32 loop; C += A*B on top of C0 = 2 stays within
+    one rounding of it."""
     vs = gpu
     rng = np.random.default_rng(O)
     csr = _block_csr(vs, rng, 9, 16, 400, 6, 16, 0.9)
@@ -93,10 +93,9 @@ def test_mfma_tiles_of_every_wave_count(gpu, orc, st, tiles, O, vec, off):
     assert np.array_equal(got.view(np.uint32)[~nan], ref.view(np.uint32)[~nan])
 
 
-def _mixed_blocks(vs, rng, h):
+def _mixed_blocks(vs, rng, h, N=1500):
     """Block rows of h equal-pattern rows: short and long ones, one cut into
     several pieces (600 columns), empty rows, a last block row cut short."""
-    N = 1500
     rows, cols, r = [], [], 0
     for n in [1, 5, 33, 64, 65, 97, 129, 600, 0, 7, 40, 63, 2, 90, 20, 20, 11]:
         c = np.sort(rng.choice(N, size=n, replace=False))
@@ -385,3 +384,106 @@ def test_row_tiles_of_up_to_128_entries_stay_whole(gpu, orc, st, copies, O):
         got = _spmm(vs, fmt, B, C0, 0, st, accumulate)
         assert_within_tolerance(got - C0 if accumulate else got, ref, csr.row_ptr, csr.val, B,
                                 f"O{O}")
+
+
+# B of 2 GiB and a little more, addressed with 64 bits; rows of any width O.
+_BIG_FLOATS = (1 << 29) + 4096
+
+
+@pytest.fixture(scope="module")
+def big_b(gpu, st):
+    vs = gpu
+    host = vs.gen_dense(77, 0, _BIG_FLOATS // 1024, 1024).reshape(-1)
+    return host, vs.DeviceArray.from_numpy(host, st)
+
+
+class _Rows:
+    """The big buffer as N x O."""
+
+    def __init__(self, big, N, O):
+        self.host = big[0][:N * O].reshape(N, O)
+        self.ptr, self.shape, self.nbytes, self.dtype = big[1].ptr, (N, O), N * O * 4, np.float32
+
+
+def _far(csr_cols, N):
+    """Columns of a 1500-column matrix, the upper half moved to the end of N."""
+    return np.where(csr_cols < 750, csr_cols, csr_cols + (N - 1500)).astype(np.int32)
+
+
+@pytest.mark.parametrize("O", [50, 257, 1024])
+@pytest.mark.parametrize("R", [1, 2, 3, 4, 8, 16])
+def test_tiles_on_b_of_2gb_or_more(gpu, orc, st, big_b, R, O):
+    """Every tile height with B of 2 GiB (64-bit addresses; at O = 257 a last
+    slice of one column): the first and last B rows, split tiles, placeholders
+    and padding, which read B row 0 there; C = A*B and C += A*B, and inf and NaN
+    in B row 0 reach only the rows that hold column 0."""
+    vs = gpu
+    N = (1 << 29) // O + 2
+    rng = np.random.default_rng(R + O)
+    one = _mixed_blocks(vs, rng, R) if R > 1 else _mixed_rows(vs, rng)
+    col = one.col.copy()
+    col[one.row_ptr[7]] = 0  # a row that holds column 0, and one with the last
+    one = vs.Csr.from_arrays(one.M, 1500, one.row_ptr, col, one.val)
+    csr = vs.Csr.from_arrays(one.M, N, one.row_ptr, _far(one.col, N), one.val)
+    fmt = vs.build_vcsr(csr, 64, 64, vs.LAYOUT_S)
+    fmt.set_tile_rows(R)
+    fmt.upload(st)
+    B = _Rows(big_b, N, O)
+    assert B.nbytes >= 1 << 31
+    small = np.concatenate([B.host[:750], B.host[N - 750:]])
+    C0 = rng.integers(-2, 3, size=(csr.M, O)).astype(np.float32)
+
+    def run(accumulate):
+        dC = _Shifted(vs, C0, 4, st)
+        vs.run_vcsr_spmm_gpu_ex(fmt, B, O, 64, dC, st, timed=True, kernel=vs.KERNEL_TILE,
+                                accumulate=accumulate)
+        return dC.numpy()
+
+    ref = orc.spmm_f64(one.M, one.row_ptr, one.col, one.val, small)
+    assert_within_tolerance(run(False), ref, one.row_ptr, one.val, small, f"R{R} O{O}")
+    err = np.abs(run(True) - (C0 + ref)) - 2.0 ** -23 * (np.abs(C0) + np.abs(ref))
+    l1 = np.array([np.abs(one.val[a:b]).sum() for a, b in zip(one.row_ptr, one.row_ptr[1:])])
+    assert (err <= 1e-4 * l1[:, None] * np.abs(small).max()).all()
+
+    row0, odd = B.host[0].copy(), np.full(O, np.inf, np.float32)
+    odd[O // 2], odd[0] = np.nan, -np.inf
+    lib = vs.load_library()
+    try:
+        assert lib.vcsr_memcpy_h2d(B.ptr, odd.ctypes.data, odd.nbytes, st.h) == 0
+        st.sync()
+        small[0] = odd
+        got = run(False)
+    finally:
+        assert lib.vcsr_memcpy_h2d(B.ptr, row0.ctypes.data, row0.nbytes, st.h) == 0
+        st.sync()
+    ref = orc.spmm_f32(one.M, one.row_ptr, one.col, one.val, small)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isinf(got), np.isinf(ref)) and np.isinf(ref).any()
+    fin = np.isfinite(ref)
+    assert np.allclose(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("O", [7, 16, 30, 47, 100, 130, 1024])
+def test_csr_wave_on_b_of_2gb_or_more_is_bit_exact(gpu, orc, st, big_b, O):
+    """The plain-CSR kernel with B of 2 GiB (64-bit addresses) in each of its
+    shapes: long rows taken by turns, short and empty rows, columns outside
+    [0, N), the first and last rows of B: bit for bit the oracle's FP32 loop."""
+    vs = gpu
+    rng = np.random.default_rng(O)
+    N = (1 << 29) // O + 2
+    lens = [0, 1, 127, 128, 129, 0, 160, 1700, 3] + [5] * 40 + [257, 1] * 5
+    rows = np.repeat(np.arange(len(lens)), lens)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    near = rng.integers(0, 1500, rows.size).astype(np.int32)
+    near[1:3] = 0, 1499
+    val = rng.standard_normal(rows.size).astype(np.float32)
+    bad = rng.random(rows.size) < 0.1
+    far = np.where(bad, np.where(rng.random(rows.size) < 0.5, -1, N), _far(near, N)).astype(np.int32)
+    B = _Rows(big_b, N, O)
+    small = np.concatenate([B.host[:750], B.host[N - 750:]])
+    d = [vs.DeviceArray.from_numpy(x, st) for x in (rp, far, val)]
+    dC = _Shifted(vs, np.full((len(lens), O), 5.0, np.float32), 4, st)
+    vs.run_csr_wave_spmm_gpu(len(lens), N, *d, B, O, dC, st, timed=True)
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(rows[~bad], minlength=len(lens)))])
+    ref = orc.spmm_f32(len(lens), rp2.astype(np.int32), near[~bad], val[~bad], small)
+    assert np.array_equal(dC.numpy().view(np.uint32), ref.view(np.uint32))
