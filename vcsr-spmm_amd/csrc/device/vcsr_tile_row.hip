@@ -77,8 +77,9 @@ struct RowLds {
 // then read ahead of their pieces' ends, so that an end does not wait for
 // memory: a block's rows together with its B slices where pieces are short,
 // each piece's row where the piece begins where they are long (one row in
-// registers instead of one per entry of a block).
-enum RowOut { kRowWrite, kRowAddShort, kRowAddLong };
+// registers instead of one per entry of a block); or at the piece's end, where
+// other waves or streams work meanwhile (launch_shape).
+enum RowOut { kRowWrite, kRowAddShort, kRowAddLong, kRowAddLate };
 
 template <int VEC, int LPE, int MERGE, int PE, bool BUF, RowOut OUT>
 __global__ __launch_bounds__(64 * kWaves)
@@ -183,7 +184,8 @@ void vcsr_row_kernel(
         const int32_t d = L.dest[p];
         if (!kok) return;
         if (d >= 0) {
-            if constexpr (OUT != kRowWrite) x = add_vec(c, x);
+            if constexpr (OUT == kRowAddLate) x = add_vec(load_c(d), x);
+            else if constexpr (OUT != kRowWrite) x = add_vec(c, x);
             store_cols<VEC, true>(C + (int64_t)d * ld, k, O, x, false);
         } else {
             store_cols<VEC, false>(partials + (int64_t)~d * O, k, O, x, false);
@@ -257,7 +259,7 @@ void vcsr_row_kernel(
         // One piece in the wave: nothing ends before the last entry, and the
         // streams' sums meet in a butterfly.
         if (np == 1) {
-            if (OUT != kRowWrite && sub == 0) c_next = load_c(L.dest[0]);
+            if (OUT != kRowWrite && OUT != kRowAddLate && sub == 0) c_next = load_c(L.dest[0]);
             walk(std::false_type());
 #pragma unroll
             for (int sh = LPE; sh < 64; sh <<= 1) acc = add_vec(acc, shfl_xor_vec(acc, sh));
@@ -316,14 +318,25 @@ hipError_t launch_shape(const DeviceFmt& d, const float* B, int32_t O, int32_t l
                            reinterpret_cast<const float2*>(d.tv_val), B, C, partials);
         return hipGetLastError();
     };
-    // C += A*B: a row of C ahead of each piece where pieces average more than
-    // 16 entries (banded 30K x 40, O = 8 / 256 8.8 / 51.3 -> 7.8 / 47.9 us; 60K x
-    // 70, O = 64 47.0 -> 45.3), else a block's rows with its B slices (power-law
-    // 322K, O = 47 91.2 us with neither, 75.5).
     if (!accumulate) return go(std::integral_constant<RowOut, kRowWrite>());
-    return d.tv_n_entries > 16 * (int64_t)d.tv_n_pieces
-               ? go(std::integral_constant<RowOut, kRowAddLong>())
-               : go(std::integral_constant<RowOut, kRowAddShort>());
+    // C += A*B, us per SpMM:
+    //  - pieces of more than 16 entries on average: a row of C ahead of each piece
+    //    (banded 30K x 40, O = 256 50.1 with a block's rows, 48.7 so); late where
+    //    narrow waves hold several pieces, some streams of which end while others
+    //    load (ahead / late: 30K x 40, O = 4 / 24 8.6 / 8.1 and 12.2 / 10.9; 60K x
+    //    30, O = 16 / 64 14.8 / 13.5 and 25.4 / 24.7; 120K x 20, O = 24 25.7 / 23.8).
+    //  - shorter ones: a block's rows with its B slices (power-law 322K, O = 47
+    //    91.2 late, 75.5 so); late in narrow waves of one or two items (uniform
+    //    20K x 10, O = 4 4.4 / 4.1; 100K x 5 8.5 / 7.1; with four, power-law 322K
+    //    25.2 / 26.8).
+    const bool long_pieces = d.tv_n_entries > 16 * (int64_t)d.tv_n_pieces;
+    if constexpr (BUF && MERGE > 1 && VEC * LPE <= 64)
+        if (long_pieces) return go(std::integral_constant<RowOut, kRowAddLate>());
+    if (long_pieces) return go(std::integral_constant<RowOut, kRowAddLong>());
+    if constexpr (BUF && MERGE <= 2 && VEC * LPE == 8)
+        return go(std::integral_constant<RowOut, kRowAddLate>());
+    else
+        return go(std::integral_constant<RowOut, kRowAddShort>());
 }
 
 template <int X>
@@ -386,10 +399,14 @@ hipError_t launch_vcsr_row_tiles(const DeviceFmt& d, const float* B, int32_t O, 
     const int64_t items = d.tv_n_chunks, simds = 4 * (int64_t)device_cus(d.device);
     const bool single = single_pieces(d);
     if (O <= 8) {
+        // C += A*B on pieces of at most 8 entries: 100K x 5, O = 4, 1 / 2 items 7.1
+        // / 8.1, uniform 50K x 4 4.1 / 4.3, power-law 100K 11.4 / 11.7; uniform 20K
+        // x 10 4.6 / 4.1.
         const int64_t four = single ? 16 : 24;
-        return items >= four * simds          ? go(I<1>(), I<8>(), I<4>())
-               : !single && items >= 5 * simds ? go(I<1>(), I<8>(), I<2>())
-                                               : go(I<1>(), I<8>(), I<1>());
+        const bool ends = accumulate && d.tv_n_entries <= 8 * (int64_t)d.tv_n_pieces;
+        return items >= four * simds                    ? go(I<1>(), I<8>(), I<4>())
+               : !single && !ends && items >= 5 * simds ? go(I<1>(), I<8>(), I<2>())
+                                                        : go(I<1>(), I<8>(), I<1>());
     }
     if (O <= 16) {
         if (row_tiles_vec(d, O) == 1) return go(I<1>(), I<16>(), I<1>());
