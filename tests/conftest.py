@@ -124,15 +124,23 @@ def work_items(csr):
     return items + (rows > 0), pieces, int(n.sum()), piece
 
 
-def items_per_wave(items, pieces, O):
-    """Work items a wave of the single-row kernel takes at width O on 256
-    compute units (vcsr_tile_row.hip), its 16-lane shape aside."""
-    simds, single = 1024, pieces < 2 * items
+def items_per_wave(items, pieces, entries, O):
+    """Work items a wave of the single-row kernel takes for C = A*B at width O on
+    256 compute units (vcsr_tile_row.hip)."""
+    simds, single, mean32 = 1024, pieces < 2 * items, entries > 32 * pieces
+    few = items < 32 * simds
+    if single and ((8 < O < 32 and (few or mean32)) or
+                   (32 < O < 64 and O % 4 and few and not mean32)):
+        return 1  # one float a lane
     if O <= 8:
         return 4 if items >= (16 if single else 24) * simds else \
             2 if not single and items >= 5 * simds else 1
     if O <= 32:
-        return 4 if single and items >= 16 * simds else 2 if items >= 5 * simds else 1
+        if single:
+            return 4 if O <= 16 or items >= 16 * simds else 1
+        if items < 5 * simds or (entries <= 7 * pieces and items < 32 * simds):
+            return 1
+        return 4 if items >= 24 * simds and entries > 8 * pieces else 2
     least = 16 if O <= 64 else 48 if O <= 128 else 64
     return 2 if single and items >= least * simds else 1
 

@@ -209,9 +209,9 @@ def test_row_tiles_any_width(gpu, orc, st, copies, O, off):
     rng = np.random.default_rng(O)
     one = _mixed_rows(vs, rng)
     csr = tile_csr(vs, one, copies)
-    items, pieces, _, piece = work_items(csr)
+    *counts, piece = work_items(csr)
     assert piece == 64
-    assert items_per_wave(items, pieces, O) == {1: 1, 40: 1, 120: 2, 600: 4 if O <= 8 else 2}[copies] or O > 32
+    assert items_per_wave(*counts, O) == {1: 1, 40: 1, 120: 2, 600: 4}[copies] or O > 32
     fmt = vs.build_vcsr(csr, 4, 64, vs.LAYOUT_S)
     fmt.set_tile_rows(1)
     fmt.upload(st)
@@ -228,23 +228,27 @@ def test_row_tiles_any_width(gpu, orc, st, copies, O, off):
     assert (err <= 1e-4 * l1[:, None] * np.abs(B).max()).all()
 
 
-# Rows of one piece each: 17 to 64 entries (mean 35 or 20), or 65 to 128.
+# Rows of one piece each: 17 to 64 entries (mean 35 or 20), 65 to 128, or short
+# ones and one of 100 that makes the largest piece 128.
 _ONE_PIECE = {"mid": [17, 20, 33, 64, 40, 31, 25, 48], "short": [17, 19, 20, 24, 22, 18],
-              "long": [65, 128, 100, 77]}
+              "long": [65, 128, 100, 77], "some": [17, 18, 100, 19, 17, 20, 18, 17]}
 
 
 @pytest.mark.parametrize("kind,copies,O,merge", [
     ("mid", 1, 1, 1), ("mid", 1, 12, 1), ("mid", 1, 31, 1), ("mid", 1, 50, 1), ("mid", 1, 101, 1),
     ("mid", 1, 257, 1), ("long", 1, 8, 1), ("long", 1, 13, 1), ("long", 1, 64, 1),
-    ("long", 1, 128, 1), ("short", 1000, 20, 2), ("mid", 2100, 8, 4), ("mid", 2100, 12, 0),
-    ("mid", 2100, 30, 4), ("mid", 2100, 50, 2), ("long", 4200, 7, 4), ("long", 4200, 15, 0),
+    ("long", 1, 128, 1), ("short", 1000, 20, 0), ("short", 1000, 32, 1), ("mid", 2100, 8, 4),
+    ("mid", 2100, 12, 0), ("mid", 2100, 17, 0), ("mid", 2100, 31, 0), ("mid", 2100, 32, 4),
+    ("mid", 2100, 50, 2), ("short", 1, 33, 0), ("short", 40, 63, 0), ("short", 40, 60, 1),
+    ("short", 5400, 47, 0), ("some", 1, 47, 0), ("some", 30, 21, 0), ("some", 30, 63, 0),
+    ("long", 3, 31, 0), ("short", 5500, 30, 4), ("short", 5500, 47, 2), ("long", 4200, 7, 4), ("long", 4200, 15, 0),
     ("long", 4200, 33, 2), ("short", 5500, 12, 4), ("short", 5500, 15, 4), ("short", 8300, 100, 2),
     ("short", 11000, 130, 2)])
 def test_row_tiles_of_one_piece(gpu, orc, st, kind, copies, O, merge):
     """Single-row tiles where every work item is one row: a wave of one item
     (its streams' sums meet in a butterfly), and waves of several (pieces cut
-    between streams), C = A*B and C += A*B.  merge 0: the 16-lane shape, one
-    item a wave at any size."""
+    between streams), C = A*B and C += A*B.  merge 0: one float a lane, one item a
+    wave at any size (33 to 63 columns: C = A*B only)."""
     vs = gpu
     rng = np.random.default_rng(copies + O)
     lens = _ONE_PIECE[kind]
@@ -259,9 +263,8 @@ def test_row_tiles_of_one_piece(gpu, orc, st, kind, copies, O, merge):
     fmt.upload(st)
     info = fmt.launch_info(O)
     assert info["split_rows"] == 0
-    if merge:
-        assert items_per_wave(csr.M, csr.M, O) == merge
-    else:
+    assert items_per_wave(csr.M, csr.M, csr.nnz, O) == max(merge, 1)
+    if not merge:
         assert info["vec"] == 1
     B = vs.gen_dense(O, 0, N, O)
     ref = np.tile(orc.spmm_f64(one.M, one.row_ptr, one.col, one.val, B), (copies, 1))

@@ -349,19 +349,27 @@ static bool single_pieces(const DeviceFmt& d) {
     return (int64_t)d.tv_n_pieces < 2 * (int64_t)d.tv_n_chunks;
 }
 
-// 9 to 16 columns: 8 lanes of 2 floats, half the load instructions an entry, or
-// 16 lanes of 1, half the streams a piece is cut between and so one piece a
-// wave at little cost.  The second where items are single pieces, unless there
-// are many and short ones, which then share waves.  us per SpMM, 16 lanes / 8
-// lanes, O = 16: banded 4K x 30 2.9 / 3.5, 30K x 40 8.6 / 9.2, 45K x 50 18.2 /
-// 18.5, 60K x 70 23.3 / 24.7, 60K x 30 17.4 / 13.4, 120K x 20 30.3 / 18.6; items
-// of several pieces: uniform 50K x 10 9.0 / 7.9, power-law 322K 26.4 / 24.1.
-
+// Floats per lane.  Fewer floats on more lanes halve or quarter the streams that
+// a piece is cut between, and so make one piece a wave cheap, but take more load
+// instructions an entry: where items are single pieces, unless there are many
+// and short ones, which then share waves.  us per SpMM, 1 float / several:
+//  - 9 to 16 columns (16 lanes / 8 of 2), O = 16: banded 4K x 30 2.9 / 3.5, 30K x
+//    40 8.6 / 9.2, 45K x 50 18.2 / 18.5, 60K x 70 23.3 / 24.7, 60K x 30 17.4 /
+//    13.4, 120K x 20 30.3 / 18.6; items of several pieces: uniform 50K x 10 9.0 /
+//    7.9, power-law 322K 26.4 / 24.1.
+//  - 17 to 31 (32 / 8 of 4), O = 17 / 31: banded 8K x 25 4.3 / 4.9 and 4.4 / 5.4,
+//    16K x 60 8.5 / 9.5 and 9.8 / 11.1, 24K x 50 13.0 / 14.8 and 14.7 / 16.6, 60K
+//    x 30 16.7 / 14.8 and 18.3 / 17.7.  32 fill the 8 lanes (9K x 40 6.7 / 5.5).
+//  - 33 to 63 that are no whole vectors of 4, short pieces (64 / 16 of 4), O = 47 /
+//    63: 4K x 30 4.3 / 4.6 and 4.4 / 4.7, 15K x 30 8.2 / 8.7 and 8.9 / 9.3, 9K x 40
+//    7.3 / 7.1; not C += A*B (4K x 30, O = 47 4.7 / 4.3).
 int row_tiles_vec(const DeviceFmt& d, int32_t O) {
-    if (O > 16) return 4;
     if (O <= 8) return 1;
     const bool few = d.tv_n_chunks < 32 * (4 * (int64_t)device_cus(d.device));
-    return single_pieces(d) && (few || d.tv_n_entries > 32 * (int64_t)d.tv_n_pieces) ? 1 : 2;
+    const bool mean32 = d.tv_n_entries > 32 * (int64_t)d.tv_n_pieces;
+    const bool narrow = single_pieces(d) && (O < 32 ? few || mean32 : few && !mean32);
+    if (O <= 16) return narrow ? 1 : 2;
+    return narrow && (O < 32 || (O < 64 && O % 4 != 0)) ? 1 : 4;
 }
 
 hipError_t launch_vcsr_row_tiles(const DeviceFmt& d, const float* B, int32_t O, int32_t ld,
@@ -392,32 +400,45 @@ hipError_t launch_vcsr_row_tiles(const DeviceFmt& d, const float* B, int32_t O, 
     //    31.2 / 28.6 / 30.1; wider always 1: power-law 100K, O = 47 21.0 / 22.8 /
     //    23.7, 322K, O = 128 107 / 111 / 125.
     //  - one piece an item: banded 8K x 60, O = 8 / 64 4.1 / 4.6 / 5.5 and 7.0 /
-    //    7.4 / 8.1; 20K x 25, O = 8 5.9 / 5.8 / 5.1; 30K x 40, O = 32 / 64 11.4 /
-    //    10.5 / 10.0 and 16.4 / 15.8 / 16.2; 120K x 20, O = 8 / 64 27.8 / 20.4 /
+    //    7.4 / 8.1; 20K x 25, O = 8 5.9 / 5.8 / 5.1; 9K x 40, O = 32 5.1 / 5.4 / 5.5;
+    //    30K x 40, O = 32 / 64 11.4 / 10.5 / 10.0 and 16.4 / 15.8 / 16.2; 120K x 20, O = 8 / 64 27.8 / 20.4 /
     //    15.9 and 39.3 / 32.3 / 42.6; O = 128: 45K x 50 47.5 / 48.3, 120K x 20 56.6
     //    / 53.4; O = 256: 120K x 20 137 / 133.
     const int64_t items = d.tv_n_chunks, simds = 4 * (int64_t)device_cus(d.device);
     const bool single = single_pieces(d);
+    // Short pieces, up to 7 entries on average (2 to 6 in the matrices measured).
+    const bool ends = d.tv_n_entries <= 7 * (int64_t)d.tv_n_pieces;
+    // 9 to 32 columns, several pieces an item, us per SpMM at 1 / 2 / 4 items:
+    // uniform 50K x 4, O = 16 / 20 / 27 4.0 / 4.4 / 5.1, 4.7 / 5.2 / 6.0 and 7.0 /
+    // 8.1 / 7.8; 100K x 5, O = 20 11.7 / 13.1 / 13.4; 200K x 4, O = 27 30.9 / 34.1 /
+    // 34.2; power-law 100K, O = 27 16.4 / 17.8 / 18.1, 200K, O = 12 20.4 / 19.3 /
+    // 20.4; 40K x 8, O = 32 6.2 / 5.7 / 6.0; 60K x 14, O = 16 12.1 / 9.8 / 9.1; 100K
+    // x 12, C += A*B, O = 12 21.7 / 15.0 / 13.7.
+    const int many = items < (ends ? 32 : 5) * simds                                          ? 1
+                     : items >= 24 * simds && d.tv_n_entries > 8 * (int64_t)d.tv_n_pieces ? 4
+                                                                                               : 2;
     if (O <= 8) {
-        // C += A*B on pieces of at most 8 entries: 100K x 5, O = 4, 1 / 2 items 7.1
-        // / 8.1, uniform 50K x 4 4.1 / 4.3, power-law 100K 11.4 / 11.7; uniform 20K
-        // x 10 4.6 / 4.1.
+        // C += A*B on short pieces, O = 4: uniform 100K x 5, 1 / 2 items 7.0 / 7.9, 50K
+        // x 4 4.1 / 4.4, power-law 60K 9.4 / 10.1; 40K x 8 4.9 / 4.8.
         const int64_t four = single ? 16 : 24;
-        const bool ends = accumulate && d.tv_n_entries <= 8 * (int64_t)d.tv_n_pieces;
-        return items >= four * simds                    ? go(I<1>(), I<8>(), I<4>())
-               : !single && !ends && items >= 5 * simds ? go(I<1>(), I<8>(), I<2>())
-                                                        : go(I<1>(), I<8>(), I<1>());
+        return items >= four * simds ? go(I<1>(), I<8>(), I<4>())
+               : !single && !(accumulate && ends) && items >= 5 * simds
+                   ? go(I<1>(), I<8>(), I<2>())
+                   : go(I<1>(), I<8>(), I<1>());
     }
     if (O <= 16) {
         if (row_tiles_vec(d, O) == 1) return go(I<1>(), I<16>(), I<1>());
-        return single                ? go(I<2>(), I<8>(), I<4>())
-               : items >= 5 * simds ? go(I<2>(), I<8>(), I<2>())
-                                    : go(I<2>(), I<8>(), I<1>());
+        return single || many == 4 ? go(I<2>(), I<8>(), I<4>())
+               : many == 2         ? go(I<2>(), I<8>(), I<2>())
+                                   : go(I<2>(), I<8>(), I<1>());
     }
+    const bool narrow = row_tiles_vec(d, O) == 1;
+    if (O < 32 && narrow) return go(I<1>(), I<32>(), I<1>());
+    if (O < 64 && narrow && !accumulate) return go(I<1>(), I<64>(), I<1>());
     if (O <= 32)
-        return single && items >= 16 * simds ? go(I<4>(), I<8>(), I<4>())
-               : items >= 5 * simds          ? go(I<4>(), I<8>(), I<2>())
-                                             : go(I<4>(), I<8>(), I<1>());
+        return (single ? items >= 16 * simds : many == 4) ? go(I<4>(), I<8>(), I<4>())
+               : !single && many == 2                     ? go(I<4>(), I<8>(), I<2>())
+                                                          : go(I<4>(), I<8>(), I<1>());
     if (O <= 64)
         return single && items >= 16 * simds ? go(I<4>(), I<16>(), I<2>())
                                              : go(I<4>(), I<16>(), I<1>());
