@@ -26,10 +26,10 @@
 //    through LDS.
 // us per SpMM, three matrices in turn, before the long rows' turns, the
 // entries' prefetch and the 16-byte lanes at any width, and now: power-law
-// 100K rows (longest 1.7K), O = 8 / 47 / 64 138 / 119 / 141 -> 33 / 37 / 37;
-// 322K (5.2K), O = 128 528 -> 206; banded 62K, O = 8 / 47 24.8 / 58.9 -> 14.8 /
-// 38.6; 9 16x16 blocks a row, O = 66 31.9 -> 20.7; uniform 1M x 16, O = 256
-// 2,733 -> 2,722.
+// 100K rows (longest 1.7K), O = 8 / 47 / 64 136 / 118 / 138 -> 27 / 34 / 34;
+// 322K (5.2K), O = 128 539 -> 206; banded 62K, O = 8 / 47 24.8 / 58.4 -> 14.4 /
+// 38.5; 16K rows of 9 16x16 blocks, O = 66 67.7 -> 36.0; uniform 1M x 16, O =
+// 256 2,737 -> 2,732.
 #include <type_traits>
 
 #include "common.hpp"

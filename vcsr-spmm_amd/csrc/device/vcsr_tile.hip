@@ -153,9 +153,9 @@ __global__ __launch_bounds__(256) void vcsr_tile_reduce(int32_t O, int32_t ld, i
 // Rows of B and C need not be aligned to VEC floats: a lane whose columns
 // would reach past O takes the last VEC of the row and stores its own ones
 // (vec_col, store_cols), so VEC depends on O and the tiles only (tile_mma_vec).
-// Block-sparse 16K matrix, O = 65 / 127 / 333: 51.8 / 84.1 / 229 us with the
-// 4-byte lanes an odd O used to take, 39.8 / 41.8 / 101 now; O = 64, 100,
-// 512 unchanged.
+// Block-sparse 16K matrix, O = 65 / 127 / 333: 51.8 / 83.9 / 229 us with the
+// 4-byte lanes an odd O used to take, 39.2 / 41.0 / 102 now; O = 100 and 512
+// unchanged.
 //
 // One wave per (piece, column tile of 16*VEC columns).  The grid runs
 // column-tile-major with the XCD-aware block order, so each XCD works on one

@@ -29,13 +29,13 @@
 // that said whether to go on, cost more than the loop there (banded 8K x 20, O
 // = 8 / 32 5.2 / 5.7 us, 3.6 / 3.7 with the ballot and the butterfly).
 // Against one kernel with a path for several pieces and one for a long piece,
-// and a piece table of 16 bytes per piece read after the entries: 37 instead of
+// and a piece table of 16 bytes per piece read after the entries: 38 instead of
 // 55 registers at O = 8, 21 instead of 29 bytes of view per two-entry row, one
 // round of loads, no bounds test per entry, and 16-byte lanes at any width.
 // Three formats in turn, us per SpMM: power-law 322K, O = 8 24.0 -> 21.7; 100K,
-// O = 20 / 47 / 257 18.3 / 23.4 / 121 -> 14.7 / 20.8 / 85; banded 60K x 30, O =
-// 50 32.8 -> 25.1; uniform 102K x 6, O = 200 107 -> 88; C += A*B, power-law
-// 100K, O = 47 34.2 -> 29.2.
+// O = 20 / 47 / 257 18.2 / 23.2 / 121 -> 14.4 / 20.7 / 87; banded 60K x 30, O =
+// 50 32.8 -> 24.7; uniform 102K x 6, O = 200 107 -> 87; C += A*B, power-law
+// 100K, O = 47 34.2 -> 28.6.
 #include <type_traits>
 
 #include "../host/tile_view.hpp"

@@ -17,12 +17,12 @@
 // Bound by the L2-to-CU path (one B slice per entry) at wide B, by the view's
 // arrival and the loads' latency at narrow B.  Against one kernel for all
 // tile heights that packed several tiles per wave in stream mode: only this
-// path's registers are held (66 instead of 94 at 3 rows and O = 128: 7 waves
+// path's registers are held (54 instead of 94 at 3 rows and O = 128: 8 waves
 // per SIMD instead of 5), a wave waits for one record and one round of entry
 // loads instead of up to four loads in sequence, and short tiles share a wave
 // without a per-entry test for the piece's end.  Banded 62K matrix, three
-// formats in turn, O = 8 / 32 / 128 / 512: 17.3 / 23.1 / 33.2 / 151 -> 8.4 /
-// 12.2 / 30.3 / 145 us; 30K rows of 6-row blocks, O = 50: 27.5 -> 12.2.
+// formats in turn, O = 8 / 32 / 128 / 512: 17.3 / 22.9 / 34.5 / 151 -> 8.4 /
+// 12.8 / 31.8 / 146 us; 30K rows of 6-row blocks, O = 50: 27.4 -> 13.2.
 // Rows absent from an entry are updated with a zero value, which is exact for
 // finite B; a piece with a non-finite sum is recomputed with the presence
 // bits before it is stored.
