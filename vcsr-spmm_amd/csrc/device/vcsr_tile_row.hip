@@ -18,7 +18,9 @@
 //  3. A piece cut between runs is finished by the stream that began it, from
 //     the later streams' partial sums in LDS, added in stream order; their
 //     number comes from one ballot.  A wave of one piece adds its streams'
-//     sums in a butterfly instead and has no step for ends.
+//     sums in a butterfly instead and has neither masks nor a step for ends
+//     (banded 8K x 25, O = 16 / 64 4.1 / 5.5 us with the masks, 3.9 / 5.0; 30K x
+//     40, O = 12 9.3 / 8.5).
 // B is read with raw buffer loads whose range check turns "no row" offsets
 // into zeros; a B of 2 GB or more is read at 64-bit addresses and "no row"
 // entries select zero.  A row holds only entries it has, so a non-finite B
@@ -81,6 +83,21 @@ struct RowLds {
 // other waves or streams work meanwhile (launch_shape).
 enum RowOut { kRowWrite, kRowAddShort, kRowAddLong, kRowAddLate };
 
+// Stores a piece's sum x, columns k and on, to row d of C or partial row ~d; c
+// are the row's values in C.
+template <int VEC, RowOut OUT, class V>
+__device__ __forceinline__ void store_row(float* C, float* partials, int32_t ld, int32_t O,
+                                          int32_t k, int32_t d, V x, V c) {
+    if (d >= 0) {
+        float* row = C + (int64_t)d * ld;
+        if constexpr (OUT == kRowAddLate) c = load_mem(row + vec_col<VEC>(k, O), V());
+        if constexpr (OUT != kRowWrite) x = add_vec(c, x);
+        store_cols<VEC, true>(row, k, O, x, false);
+    } else {
+        store_cols<VEC, false>(partials + (int64_t)~d * O, k, O, x, false);
+    }
+}
+
 template <int VEC, int LPE, int MERGE, int PE, bool BUF, RowOut OUT>
 __global__ __launch_bounds__(64 * kWaves)
 void vcsr_row_kernel(
@@ -121,40 +138,50 @@ void vcsr_row_kernel(
     const uint32_t row_bytes = (uint32_t)ld * 4u;
     // i / run for i < 1024 by multiplication (exact: run < 1024).
     const uint32_t inv = (1u << 20) / (uint32_t)run + 1u;
-    int32_t before = 0, last = 1;  // ends before this round; whether the entry before it is one
+    // Writes the staged lists to LDS; `one`: the wave holds one piece, which
+    // needs no masks and no first pieces.
+    auto stage = [&](auto one) {
+        constexpr bool ONE = decltype(one)::value;
+        int32_t before = 0, last = 1;  // ends before this round; whether the entry before it is one
 #pragma unroll
-    for (int it = 0; it < IE; ++it) {
-        const int32_t i = it * 64 + lane;
-        if (it * 64 >= S * run) break;  // S*run <= EMAX
-        const bool in = i < ne;
-        const uint32_t word = in ? __builtin_bit_cast(uint32_t, rec[it].y) : 0u;
-        const uint64_t m = __ballot(word >> 31);
-        if (i < S * run) {
-            const uint32_t br = word & 0x7fffffffu;
-            const bool real = in && br != (uint32_t)kTileNoRow;
-            const int32_t s = (int32_t)(((uint32_t)i * inv) >> 20), j = i - s * run;
-            uint2 x;
-            x.x = real ? (BUF ? br * row_bytes : br) : kNoRow;
-            x.y = in ? __builtin_bit_cast(uint32_t, rec[it].x) : 0u;
-            L.ent[s * (run + 2) + j] = x;
-            if (j == 0) {
-                const uint32_t prev = lane == 0 ? (uint32_t)last : (uint32_t)(m >> ((lane - 1) & 63)) & 1u;
-                L.first[s] = before + (int32_t)__builtin_amdgcn_mbcnt_hi(
-                                          (uint32_t)(m >> 32),
-                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                L.carry[s] = in && prev == 0u;
+        for (int it = 0; it < IE; ++it) {
+            const int32_t i = it * 64 + lane;
+            if (it * 64 >= S * run) break;  // S*run <= EMAX
+            const bool in = i < ne;
+            const uint32_t word = in ? __builtin_bit_cast(uint32_t, rec[it].y) : 0u;
+            const uint64_t m = ONE ? 0u : __ballot(word >> 31);
+            if (i < S * run) {
+                const uint32_t br = word & 0x7fffffffu;
+                const bool real = in && br != (uint32_t)kTileNoRow;
+                const int32_t s = (int32_t)(((uint32_t)i * inv) >> 20), j = i - s * run;
+                uint2 x;
+                x.x = real ? (BUF ? br * row_bytes : br) : kNoRow;
+                x.y = in ? __builtin_bit_cast(uint32_t, rec[it].x) : 0u;
+                L.ent[s * (run + 2) + j] = x;
+                if (!ONE && j == 0) {
+                    const uint32_t prev =
+                        lane == 0 ? (uint32_t)last : (uint32_t)(m >> ((lane - 1) & 63)) & 1u;
+                    L.first[s] = before + (int32_t)__builtin_amdgcn_mbcnt_hi(
+                                              (uint32_t)(m >> 32),
+                                              __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                    L.carry[s] = in && prev == 0u;
+                }
+            }
+            if constexpr (!ONE) {
+                if (lane < 2) L.ends[2 * it + lane] = (uint32_t)(m >> (32 * lane));
+                before += __popcll(m);
+                last = (int32_t)(m >> 63);
             }
         }
-        if (lane < 2) L.ends[2 * it + lane] = (uint32_t)(m >> (32 * lane));
-        before += __popcll(m);
-        last = (int32_t)(m >> 63);
-    }
+        if constexpr (!ONE) {
 #pragma unroll
-    for (int it = 0; it < IP; ++it) {
-        const int32_t i = it * 64 + lane;
-        if (i < np) L.dest[i] = ds[it];
-    }
-    wave_sync();
+            for (int it = 0; it < IP; ++it) {
+                const int32_t i = it * 64 + lane;
+                if (i < np) L.dest[i] = ds[it];
+            }
+        }
+        wave_sync();
+    };
 
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), (short)0, (int)b_bytes,
@@ -179,21 +206,13 @@ void vcsr_row_kernel(
     auto load_c = [&](int32_t d) -> V {
         return d >= 0 ? load_mem(C + (int64_t)d * ld + kc, V()) : zero_vec(V());
     };
-    // Stores the sum x of piece p; c are the row's values in C.
-    auto store_piece = [&](int32_t p, V x, const V& c) {
-        const int32_t d = L.dest[p];
-        if (!kok) return;
-        if (d >= 0) {
-            if constexpr (OUT == kRowAddLate) x = add_vec(load_c(d), x);
-            else if constexpr (OUT != kRowWrite) x = add_vec(c, x);
-            store_cols<VEC, true>(C + (int64_t)d * ld, k, O, x, false);
-        } else {
-            store_cols<VEC, false>(partials + (int64_t)~d * O, k, O, x, false);
-        }
+    auto store_to = [&](int32_t d, V x, V c) {
+        if (kok) store_row<VEC, OUT>(C, partials, ld, O, k, d, x, c);
     };
+    auto store_piece = [&](int32_t p, V x, V c) { store_to(L.dest[p], x, c); };
 
-    int32_t p = L.first[sub];
-    bool carry = S > 1 && L.carry[sub] != 0;
+    int32_t p = 0;       // the stream's piece ...
+    bool carry = false;  // ... and whether it began in an earlier run
     V acc = zero_vec(V());
     V c_next = zero_vec(V());  // a row of C read ahead of its piece's end
     // Entries i0 .. i0 + NU - 1 of every stream's run; `ends`: pieces may end
@@ -201,16 +220,17 @@ void vcsr_row_kernel(
     auto block = [&](auto n_c, auto ends, int32_t i0) {
         constexpr int NU = decltype(n_c)::value;
         constexpr bool ENDS = decltype(ends)::value;
-        uint2 r[NU];
+        uint32_t off[NU];
+        float a[NU];
         V b[NU];
 #pragma unroll
         for (int u = 0; u < NU; u += 2) {
             const uint4 x = *reinterpret_cast<const uint4*>(le + i0 + u);
-            r[u] = make_uint2(x.x, x.y);
-            r[u + 1] = make_uint2(x.z, x.w);
+            off[u] = x.x, a[u] = __builtin_bit_cast(float, x.y);
+            off[u + 1] = x.z, a[u + 1] = __builtin_bit_cast(float, x.w);
         }
 #pragma unroll
-        for (int u = 0; u < NU; ++u) b[u] = load_b(r[u].x);
+        for (int u = 0; u < NU; ++u) b[u] = load_b(off[u]);
         // End bits of entries tb + i0 .. + NU - 1.
         const int32_t t = tb + i0;
         const uint32_t bits =
@@ -227,7 +247,7 @@ void vcsr_row_kernel(
         }
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-            fma_vec(acc, __builtin_bit_cast(float, r[u].y), b[u]);
+            fma_vec(acc, a[u], b[u]);
             if (ENDS && (bits & (1u << u))) {
                 if (S > 1 && carry) {
                     // The end of a piece begun in an earlier run.
@@ -259,14 +279,20 @@ void vcsr_row_kernel(
         // One piece in the wave: nothing ends before the last entry, and the
         // streams' sums meet in a butterfly.
         if (np == 1) {
-            if (OUT != kRowWrite && OUT != kRowAddLate && sub == 0) c_next = load_c(L.dest[0]);
+            stage(std::true_type());
+            const int32_t d = uniform(ds[0]);
+            V c = zero_vec(V());
+            if (OUT != kRowWrite && OUT != kRowAddLate && sub == 0) c = load_c(d);
             walk(std::false_type());
 #pragma unroll
             for (int sh = LPE; sh < 64; sh <<= 1) acc = add_vec(acc, shfl_xor_vec(acc, sh));
-            if (sub == 0) store_piece(0, acc, c_next);
+            if (sub == 0) store_to(d, acc, c);
             return;
         }
     }
+    stage(std::false_type());
+    p = L.first[sub];
+    carry = S > 1 && L.carry[sub] != 0;
 
     // The row of C of the piece that this stream begins and the next run opens
     // with (the stream finishes it below), or of its first piece.
