@@ -356,13 +356,10 @@ hipError_t launch_shape(const DeviceFmt& d, const float* B, int32_t O, int32_t l
     //    20K x 10, O = 4 4.4 / 4.1; 100K x 5 8.5 / 7.1; with four, power-law 322K
     //    25.2 / 26.8).
     const bool long_pieces = d.tv_n_entries > 16 * (int64_t)d.tv_n_pieces;
-    if constexpr (BUF && MERGE > 1 && VEC * LPE <= 64)
-        if (long_pieces) return go(std::integral_constant<RowOut, kRowAddLate>());
-    if (long_pieces) return go(std::integral_constant<RowOut, kRowAddLong>());
-    if constexpr (BUF && MERGE <= 2 && VEC * LPE == 8)
-        return go(std::integral_constant<RowOut, kRowAddLate>());
-    else
-        return go(std::integral_constant<RowOut, kRowAddShort>());
+    constexpr RowOut LONG = BUF && MERGE > 1 && VEC * LPE <= 64 ? kRowAddLate : kRowAddLong;
+    constexpr RowOut SHORT = BUF && MERGE <= 2 && VEC * LPE == 8 ? kRowAddLate : kRowAddShort;
+    return long_pieces ? go(std::integral_constant<RowOut, LONG>())
+                       : go(std::integral_constant<RowOut, SHORT>());
 }
 
 template <int X>
